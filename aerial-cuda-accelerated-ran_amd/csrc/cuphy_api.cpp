@@ -448,6 +448,8 @@ cuphyStatus_t CUPHYWINAPI cuphySetupLDPCEncode(cuphyLDPCEncodeLaunchConfig_t cfg
     d.Z = (int16_t)Z;
     d.num_rows = (int16_t)num_rows;
     d.puncture = puncture ? 1 : 0;
+    const nrldpc::encode_geometry g = nrldpc::encode_bits_geometry(BG, Z, num_rows);
+    d.zi = (int16_t)g.zi;
     if (enable_desc_async_copy &&
         (hipMemcpyAsync(d_workspace, h_workspace, 2u * n_tbs * sizeof(nrldpc::enc_tensor), hipMemcpyHostToDevice,
                         strm) != hipSuccess ||
@@ -457,9 +459,9 @@ cuphyStatus_t CUPHYWINAPI cuphySetupLDPCEncode(cuphyLDPCEncodeLaunchConfig_t cfg
     // the descriptor is the kernel's by-value argument (ldpc_encode.cu:544-546)
     cfg->m_kernelArgs[0] = cpu_desc;
     const int max_cw = cols(*inDesc);
-    set_node(cfg->m_kernelNodeParams, nrldpc::encode_bits_kernel(), dim3((unsigned)std::max(1, max_cw), (unsigned)n_tbs, 1),
-             dim3(256), &cfg->m_kernelArgs[0]);
-    cfg->m_kernelNodeParams.sharedMemBytes = (unsigned)((nsys + std::max(num_rows, 4) + 4) * Z);
+    set_node(cfg->m_kernelNodeParams, g.func, dim3((unsigned)std::max(1, max_cw), (unsigned)n_tbs, 1), dim3(g.block),
+             &cfg->m_kernelArgs[0]);
+    cfg->m_kernelNodeParams.sharedMemBytes = g.lds_bytes;
     return CUPHY_STATUS_SUCCESS;
 }
 

@@ -22,12 +22,18 @@ struct enc_descr {
     const enc_tensor* output;
     int32_t num_TBs;
     int16_t BG, Kb, Z, num_rows;
-    int32_t puncture;
+    int16_t puncture, zi;  // zi: index of Z among the lifting sizes
 };
 
-// The bit-packed encoder kernel (argument: enc_descr by value; grid
-// (code words, TBs), 256 threads, (nsys + num_rows + 4) * Z bytes of LDS).
-void* encode_bits_kernel();
+// The bit-packed encoder kernel (argument: enc_descr by value; grid (code
+// words, TBs)), its workgroup size and its bytes of dynamic LDS; zi: the
+// index of Z among the lifting sizes (enc_descr).
+struct encode_geometry {
+    void* func;
+    unsigned block, lds_bytes;
+    int zi;
+};
+encode_geometry encode_bits_geometry(int bg, int Z, int num_rows);
 
 // Encode ncb code blocks: info bytes (nsys*Z bits, 0/1) -> codeword bytes
 // ((nsys + nrows) * Z bits).

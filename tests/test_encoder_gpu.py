@@ -43,3 +43,27 @@ def test_gpu_encoder_matches_reference_goldens():
     cw = W.encode(1, 52, torch.from_numpy(src).cuda())
     torch.cuda.synchronize()
     assert np.array_equal(cw.cpu().numpy(), enc)
+
+
+@pytest.mark.parametrize("bg", [1, 2])
+def test_every_lifting_size(bg):
+    """All 51 lifting sizes (words of a column partly filled, one to twelve
+    of them): the byte encoder and the bit-packed one against the oracle."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from aerial_amd import workloads as W
+    from aerial_amd.encoder import LdpcEncoder, pack_bits, unpack_bits
+    print("[case] encoder BG%d, every lifting size" % bg, flush=True)
+    ns = 22 if bg == 1 else 10
+    enc = LdpcEncoder(puncturing=False, max_tbs=1)
+    for Z in W.LIFTING_SIZES:
+        info = np.stack([O.random_bits(7 * Z + i, ns * Z) for i in range(2)])
+        ref = np.stack([O.encode(bg, Z, x) for x in info])
+        dev = torch.from_numpy(info).cuda()
+        cw = W.encode(bg, Z, dev).cpu().numpy()
+        assert np.array_equal(cw, ref), "bytes, Z = %d" % Z
+        words = enc.encode_words(bg, Z, [pack_bits(dev.t().contiguous())])[0]
+        n = ref.shape[1]
+        assert np.array_equal(unpack_bits(words, n).t().cpu().numpy(), ref), "words, Z = %d" % Z
+        if n % 32:  # the rest of the last word is 0
+            assert not torch.any((words[:, -1].to(torch.int64) & 0xFFFFFFFF) >> (n % 32)).item()
