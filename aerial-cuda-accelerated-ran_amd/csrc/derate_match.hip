@@ -43,10 +43,7 @@ __global__ __launch_bounds__(256) void derate_match_kernel(const rm_descriptor* 
     const uint32_t w_base = (uint32_t)g.start >> 5;
     if (descr) {
         const uint32_t nw = min(((uint32_t)(g.start + g.E - 1) >> 5) - w_base + 1u, (uint32_t)RM_SEQ_WORDS);
-        const uint32_t nwave = blockDim.x >> 6, wave = threadIdx.x >> 6;
-        const uint32_t per = (nw + nwave - 1) / nwave;
-        const uint32_t a = min(nw, wave * per), b = min(nw, a + per);
-        gold_words_wave(p.cinit, w_base + a, w_base + b, seq + a);
+        if (threadIdx.x < 64) gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w_base, (int)nw, seq);
         __syncthreads();
     }
 

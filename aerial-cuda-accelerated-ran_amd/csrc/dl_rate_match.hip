@@ -54,13 +54,10 @@ __global__ __launch_bounds__(256) void dl_rate_match_kernel(const PerTbParams* _
     if (ok) {
         const uint32_t* src = cw[t] + (size_t)r * words_in;
         for (int w = tid; w < words_in; w += nthr) cb_in[w] = src[w];
-        if (scrambling) {  // the CB's words of c, each wave generating a share
+        if (scrambling) {  // the CB's words of c
             const uint32_t w_base = (uint32_t)g.start >> 5;
             const int nw = (int)(((uint32_t)(g.start + g.E - 1) >> 5) - w_base + 1u);
-            const int nwave = nthr >> 6, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-            const int per = (nw + nwave - 1) / nwave;
-            const int a = min(nw, wave * per), b = min(nw, a + per);
-            gold_words_wave(p.cinit, w_base + (uint32_t)a, w_base + (uint32_t)b, seq + a);
+            if (tid < 64) gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w_base, nw, seq);
             if (tid == 0) seq[nw] = 0u;
         }
     }

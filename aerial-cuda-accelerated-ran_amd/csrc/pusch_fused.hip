@@ -318,13 +318,10 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
         for (int n = nv * 8 + tid; n < nh; n += nthr) hb[n] = harq[n];
     }
     const uint32_t w_base = (uint32_t)g.start >> 5;
-    if (descr) {  // each wave generates its share of the words while the loads land
+    if (descr && tid >= nthr - 64) {  // the last wave generates the words while the loads land
         const int nw = rm_seq_words(g);
-        const int nwave = nthr >> 6, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int per = (nw + nwave - 1) / nwave;
-        const int a = min(nw, wave * per), b = min(nw, a + per);
-        gold_words_wave(p.cinit, w_base + (uint32_t)a, w_base + (uint32_t)b, seq + a);
-        if (tid == 0) seq[nw] = 0u;
+        gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w_base, nw, seq);
+        if (tid == nthr - 64) seq[nw] = 0u;
     }
     __syncthreads();
     if (g.ndi)
