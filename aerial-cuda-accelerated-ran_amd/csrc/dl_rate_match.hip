@@ -5,9 +5,7 @@
 // PDSCH kernel (cuPHY/src/cuphy/dl_rate_matching/dl_rate_matching.cu:1951-2260)
 // does the same with enable_layer_mapping = 0 and enable_modulation = 0 and
 // writes CB r of TB t at bit (t * cmax + r) * emax of the output; so does
-// this kernel.  Here every thread builds whole output words (32 output bits,
-// each gathered from the CB's encoded bits staged in LDS) instead of
-// OR-ing single bits into LDS words with atomics.
+// this kernel.
 //
 // Output bit i of CB r (i < E_r) is bit (i mod Qm) of symbol i / Qm, i.e.
 // selected bit m = (i mod Qm) * E_r / Qm + i / Qm; selected bit m sits at
@@ -15,6 +13,16 @@
 // buffer, buffer position c < Kd ? c : c + F (the same closed form as the
 // uplink de-rate-matcher).  Scrambling XORs c(start_r + i), start_r the
 // CB's first bit in the TB.
+//
+// So the output interleaves Qm contiguous runs of the circular buffer.  A
+// thread takes 32 symbols: 32 bits of each run (one funnel shift of two
+// words read straight from the encoder's output: consecutive lanes read
+// consecutive words, nothing is staged) and Qm output words, each a
+// compile-time pattern of single-bit inserts.  One bit at a time, with a
+// division, a modulo and an LDS read each, 2,800 code blocks of 9,088 bits
+// (R = 0.93, 256QAM, scrambled) took 47 us (81 us with the earlier
+// sequence generator); this takes 13 us, 6.4 MB in and out being 1.3 us: the
+// sequence, the selection and one wave per code block bound it.
 #include <hip/hip_runtime.h>
 
 #include "derate_core.hpp"
@@ -25,12 +33,70 @@ namespace nrldpc {
 
 constexpr int DL_RM_MAX_N = 66 * 384;  // encoded bits of a BG1 Zc = 384 code block
 
+// Where a code block's selected bits come from.
+struct dl_source {
+    const uint32_t* __restrict__ src;  // encoded bits
+    int words, L, Kd, F;
+};
+
+__device__ __forceinline__ uint32_t low_bits(int n) { return n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u; }
+
+// 32 selected bits from circle position c (< L) on, of which the first
+// `want` (1 .. 32) are used.
+__device__ __forceinline__ uint32_t circle_bits(const dl_source& s, int c, int want)
+{
+    uint32_t v = 0;
+    for (int got = 0;;) {
+        const bool head = c < s.Kd;
+        const int p = head ? c : c + s.F, end = head ? min(s.Kd, s.L) : s.L;
+        const int i = p >> 5;
+        const uint32_t hi = (i + 1 < s.words) ? s.src[i + 1] : 0u;
+        const uint32_t x = __builtin_amdgcn_alignbit(hi, s.src[i], (uint32_t)p & 31u);
+        v |= (x & low_bits(end - c)) << got;
+        got += end - c;
+        if (got >= want) return v;
+        c = (end == s.L) ? 0 : end;
+    }
+}
+
+// Output words of a code block: thread t builds words QM * t .. QM * t + QM - 1.
+template <int QM>
+__device__ __forceinline__ void dl_words(const dl_source& s, const rm_geometry& g, const uint32_t* seq, int emax_words,
+                                         uint32_t* __restrict__ dst)
+{
+    const uint32_t soff = (uint32_t)g.start & 31u;
+    const int groups = (g.EQ + 31) >> 5;
+    const int run_step = g.EQ % g.L;
+    for (int t = threadIdx.x; t < groups; t += blockDim.x) {
+        const int j0 = 32 * t, want = min(32, g.EQ - j0);
+        uint32_t run[QM];
+        int c = (g.c0 + j0) % g.L;
+#pragma unroll
+        for (int k = 0; k < QM; ++k) {
+            run[k] = circle_bits(s, c, want);
+            c += run_step;
+            if (c >= g.L) c -= g.L;
+        }
+#pragma unroll
+        for (int q = 0; q < QM; ++q) {
+            const int at = QM * t + q;
+            uint32_t w = 0;
+#pragma unroll
+            for (int b = 0; b < 32; ++b) w |= ((run[(32 * q + b) % QM] >> ((32 * q + b) / QM)) & 1u) << b;
+            // (the word after the last with output bits exists too)
+            if (seq && 32 * at < g.E) w ^= __builtin_amdgcn_alignbit(seq[at + 1], seq[at], soff);
+            if (at < emax_words) dst[at] = w & low_bits(max(0, g.E - 32 * at));
+        }
+    }
+    for (int w = QM * groups + (int)threadIdx.x; w < emax_words; w += blockDim.x) dst[w] = 0u;
+}
+
 __global__ __launch_bounds__(256) void dl_rate_match_kernel(const PerTbParams* __restrict__ prms,
                                                             const uint32_t* const* __restrict__ cw, int max_cbs,
                                                             int emax_words, int scrambling,
                                                             uint32_t* __restrict__ out)
 {
-    extern __shared__ uint32_t dl_lds[];
+    extern __shared__ uint32_t dl_seq[];  // scrambling words of the code block, one more than its E bits reach
     const int t = blockIdx.y, r = blockIdx.x;
     const PerTbParams& p = prms[t];
     const int C = __builtin_amdgcn_readfirstlane((int)p.num_CBs);
@@ -43,46 +109,32 @@ __global__ __launch_bounds__(256) void dl_rate_match_kernel(const PerTbParams* _
         rm_make_uniform(g);
     }
     const int N = __builtin_amdgcn_readfirstlane((int)p.N);
-    const int tid = threadIdx.x, nthr = blockDim.x;
     uint32_t* dst = out + ((size_t)t * max_cbs + r) * emax_words;
     // a CB that does not fit its slot or the kernel's buffers stays zero
     const bool ok = prm_ok && g.E > 0 && g.E <= 32 * emax_words && g.Ncb <= N && N <= DL_RM_MAX_N && g.L > 0 &&
                     g.Kd >= 0 && g.c0 >= 0 && g.c0 < g.L;
-    const int words_in = (N + 31) >> 5;
-    uint32_t* cb_in = dl_lds;
-    uint32_t* seq = dl_lds + words_in;
-    if (ok) {
-        const uint32_t* src = cw[t] + (size_t)r * words_in;
-        for (int w = tid; w < words_in; w += nthr) cb_in[w] = src[w];
-        if (scrambling) {  // the CB's words of c
-            const uint32_t w_base = (uint32_t)g.start >> 5;
-            const int nw = (int)(((uint32_t)(g.start + g.E - 1) >> 5) - w_base + 1u);
-            if (tid < 64) gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w_base, nw, seq);
-            if (tid == 0) seq[nw] = 0u;
-        }
+    if (!ok) {
+        for (int w = threadIdx.x; w < emax_words; w += blockDim.x) dst[w] = 0u;
+        return;
     }
-    __syncthreads();
-    const int e_words = ok ? (g.E + 31) >> 5 : 0;
-    const int soff = g.start & 31;
-    for (int w = tid; w < emax_words; w += nthr) {
-        uint32_t v = 0;
-        if (w < e_words) {
-            const int nb = min(32, g.E - 32 * w);
-            for (int b = 0; b < nb; ++b) {
-                const int i = 32 * w + b;
-                const int j = i / g.Qm, k = i - j * g.Qm;
-                const int m = k * g.EQ + j;
-                const int c = (g.c0 + m) % g.L;
-                const int pos = (c < g.Kd) ? c : c + g.F;
-                uint32_t bit = (cb_in[pos >> 5] >> (pos & 31)) & 1u;
-                if (scrambling) {
-                    const int n = soff + i;
-                    bit ^= (seq[n >> 5] >> (n & 31)) & 1u;
-                }
-                v |= bit << b;
-            }
+    const int words_in = (N + 31) >> 5;
+    const dl_source s{cw[t] + (size_t)r * words_in, words_in, g.L, g.Kd, g.F};
+    if (scrambling) {
+        const uint32_t w_base = (uint32_t)g.start >> 5;
+        const int nw = (int)(((uint32_t)(g.start + g.E - 1) >> 5) - w_base + 1u);
+        if (threadIdx.x < 64) {
+            gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w_base, nw, dl_seq);
+            if (threadIdx.x == 0) dl_seq[nw] = 0u;
         }
-        dst[w] = v;
+        __syncthreads();
+    }
+    const uint32_t* seq = scrambling ? dl_seq : nullptr;
+    switch (Qm) {  // (uniform)
+    case 8: dl_words<8>(s, g, seq, emax_words, dst); break;
+    case 6: dl_words<6>(s, g, seq, emax_words, dst); break;
+    case 4: dl_words<4>(s, g, seq, emax_words, dst); break;
+    case 2: dl_words<2>(s, g, seq, emax_words, dst); break;
+    default: dl_words<1>(s, g, seq, emax_words, dst);
     }
 }
 
@@ -95,11 +147,11 @@ cuphyStatus_t dl_rate_match(const PerTbParams* d_prms, int num_tbs, const uint32
     if (num_tbs == 0) return CUPHY_STATUS_SUCCESS;
     if (!d_prms || !d_cw || !d_out) return CUPHY_STATUS_INVALID_ARGUMENT;
     const int emax_words = emax / 32;
-    const size_t lds = ((size_t)(DL_RM_MAX_N + 31) / 32 + (scrambling ? (size_t)emax_words + 2 : 0)) * sizeof(uint32_t);
-    if (lds > 64u * 1024u && hipFuncSetAttribute((const void*)&dl_rate_match_kernel,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-        return CUPHY_STATUS_INTERNAL_ERROR;
-    hipLaunchKernelGGL(dl_rate_match_kernel, dim3((unsigned)max_cbs, (unsigned)num_tbs), dim3(256), lds, strm, d_prms,
+    // the words of E <= emax scrambling bits from any bit of a word on, and one more
+    const size_t lds = scrambling ? ((size_t)emax_words + 2) * sizeof(uint32_t) : 0;
+    // a thread per 32 symbols: one wave holds 16,384 bits at 8 bits per symbol
+    const unsigned block = emax_words <= 512 ? 64u : 256u;
+    hipLaunchKernelGGL(dl_rate_match_kernel, dim3((unsigned)max_cbs, (unsigned)num_tbs), dim3(block), lds, strm, d_prms,
                        d_cw, max_cbs, emax_words, scrambling ? 1 : 0, d_out);
     return hipGetLastError() == hipSuccess ? CUPHY_STATUS_SUCCESS : CUPHY_STATUS_INTERNAL_ERROR;
 }

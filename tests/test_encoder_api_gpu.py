@@ -163,3 +163,34 @@ def test_encode_then_rate_match_chain(enc):
     got = out.cpu().numpy()[0]
     for r in range(p.num_CBs):
         assert np.array_equal(words_to_bits(got[r], got.shape[1] * 32)[:ref[r].size], ref[r]), r
+
+
+# (bg, Zc, CBs, K', Qm, layers, E per CB, rv, scrambling): fewer symbols than a
+# word, remainders of 32 symbols, Qm = 1, runs that cross the filler hole and
+# the wrap (short circles several times within a word), a sequence far from
+# its start (2.5 M bits)
+DL_EDGES = [(2, 2, 2, 16, 2, 1, 6, 0, True), (2, 2, 1, 16, 8, 1, 1000, 3, True), (1, 3, 2, 60, 1, 1, 31, 1, True),
+            (1, 3, 1, 60, 6, 2, 504, 2, False), (2, 52, 3, 480, 1, 1, 2049, 0, True), (1, 384, 1, 8448, 8, 4, 9088, 0, True),
+            (1, 208, 2, 4400, 4, 1, 4 * 33, 2, True), (1, 384, 100, 8424, 6, 1, 25344, 1, True)]
+
+
+@pytest.mark.parametrize("case", DL_EDGES)
+def test_dl_rate_match_edges(case):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from aerial_amd.encoder import dl_rate_match
+    from aerial_amd.pusch import make_tb_params
+    bg, Zc, C, Kp, Qm, Nl, E, rv, scr = case
+    print("[case] DL rate matching BG%d Zc=%d CBs=%d K'=%d Qm=%d Nl=%d E=%d rv=%d scr=%d" % case, flush=True)
+    p, _ = make_tb_params(bg, Zc, C, Kp, Qm, Nl, C * E, rv)
+    p.cinit = (0x3C6EF35 * (E + 1)) & 0x7FFFFFFF
+    cw = np.random.RandomState(E).randint(0, 2, (C, p.N)).astype(np.uint8)
+    words = np.stack([O.pack_bits(x) for x in cw])
+    emax = (E + 31) // 32 * 32 + 64
+    out = dl_rate_match([p], [torch.from_numpy(words.view(np.int32)).cuda()], emax, scrambling=scr)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()[0]
+    for r, ref in enumerate(dl_reference(p, cw, p.cinit, scr)):
+        bits = words_to_bits(got[r], emax)
+        assert np.array_equal(bits[:E], ref), (case, r)
+        assert not bits[E:].any(), (case, r)
