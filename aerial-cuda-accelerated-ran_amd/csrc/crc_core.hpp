@@ -1,9 +1,9 @@
 // Device core of the CRC checks (TS 38.212 5.1, zero initial value), shared
-// by the PUSCH CRC-decode kernels and the fused slot kernel.  A thread
-// computes the remainder of its contiguous chunk of words byte-wise with a
-// 256-entry table, then multiplies it by x^(32 * words after the chunk)
-// mod g with a table of x^(32*2^j) mod g; chunk results are XOR-combined
-// (CRC linearity).  All tables are built at compile time.
+// by the PUSCH CRC-decode kernels and the fused slot kernel.  Every thread
+// computes the remainder of some of the message's words, shifted by the bits
+// after them, and the shares are XOR-combined (CRC linearity): the CRC-decode
+// kernels give a thread every S-th word (strided_crc), the fused kernel one
+// word.  All tables are built at compile time.
 #pragma once
 
 #include "nr_ldpc_common.hpp"
@@ -35,7 +35,6 @@ constexpr uint32_t gf2_mulmod(uint32_t a, uint32_t b, crc_poly p)
 
 struct crc_tables {
     uint32_t byte[3][256];   // byte-wise step: reg' = (reg << 8) ^ T[(reg >> (L-8)) ^ b]
-    uint32_t pow32[3][24];   // x^(32 * 2^j) mod g
 };
 
 constexpr uint32_t byte_entry(uint32_t v, crc_poly p)
@@ -50,32 +49,14 @@ constexpr crc_tables make_crc_tables()
 {
     crc_tables t{};
     const crc_poly ps[3] = {CRC24A_P, CRC24B_P, CRC16_P};
-    for (int k = 0; k < 3; ++k) {
+    for (int k = 0; k < 3; ++k)
         for (uint32_t v = 0; v < 256; ++v) t.byte[k][v] = byte_entry(v, ps[k]);
-        // x^32 mod g, then repeated squaring
-        uint32_t x32 = 1;
-        for (int i = 0; i < 32; ++i) x32 = gf2_mulmod(x32, 2u, ps[k]);
-        t.pow32[k][0] = x32;
-        for (int j = 1; j < 24; ++j) t.pow32[k][j] = gf2_mulmod(t.pow32[k][j - 1], t.pow32[k][j - 1], ps[k]);
-    }
     return t;
 }
 
 static __device__ const crc_tables g_crc_tables = make_crc_tables();
 
 enum { K_CRC24A = 0, K_CRC24B = 1, K_CRC16 = 2 };
-
-__device__ __forceinline__ uint32_t dmulmod(uint32_t a, uint32_t b, int L, uint32_t g)
-{
-    const uint32_t mask = (1u << L) - 1u;
-    uint32_t r = 0;
-    for (int i = L - 1; i >= 0; --i) {
-        const uint32_t top = (r >> (L - 1)) & 1u;
-        r = ((r << 1) & mask) ^ (top ? g : 0u);
-        if ((b >> i) & 1u) r ^= a;
-    }
-    return r;
-}
 
 // a*b mod g for a compile-time polynomial (fully unrolled).
 template <int L, uint32_t G>
@@ -104,36 +85,91 @@ __device__ __forceinline__ uint32_t rbit8x4(uint32_t w)
     return w;
 }
 
-// Remainder of `nw` message words (bytes in memory order, each byte MSB-first
-// in the message) held by the workgroup; `word(i)` yields message word i.
-template <typename WordFn>
-__device__ uint32_t block_crc(int nw, int kind, WordFn word, uint32_t* lds_red)
+// Multiplication of a 32-bit (unreduced) value by x^(32 * S) mod g, by
+// bytes: v * x^(32 S) = XOR over b of step[b][byte b of v]; and the factors
+// x^(32 t + L) of the last word of thread t of S.
+template <int S> struct crc_stride_table {
+    uint32_t step[4][256];
+    uint32_t last[S];
+};
+template <int S> constexpr crc_stride_table<S> make_crc_stride_table(crc_poly p)
 {
-    const crc_poly p = kind == K_CRC24A ? CRC24A_P : (kind == K_CRC24B ? CRC24B_P : CRC16_P);
-    const uint32_t* T = g_crc_tables.byte[kind];
-    const int nt = blockDim.x, tid = threadIdx.x;
-    const int per = (nw + nt - 1) / nt;
-    const int w0 = min(nw, tid * per), w1 = min(nw, w0 + per);
-    uint32_t reg = 0;
-    for (int w = w0; w < w1; ++w) {
-        const uint32_t v = word(w);
-        for (int b = 0; b < 4; ++b) {
-            const uint32_t byte = (v >> (8 * b)) & 0xFFu;
-            reg = ((reg << 8) & ((1u << p.L) - 1u)) ^ T[((reg >> (p.L - 8)) ^ byte) & 0xFFu];
+    crc_stride_table<S> t{};
+    const uint32_t mask = (1u << p.L) - 1u;
+    uint32_t x32 = 1, xs = 1;  // x^32, x^(32 S)
+    for (int i = 0; i < 32; ++i) x32 = gf2_mulmod(x32, 2u, p);
+    for (int i = S; i > 1; i >>= 1) xs = (i == S) ? gf2_mulmod(x32, x32, p) : gf2_mulmod(xs, xs, p);
+    uint32_t v = xs;
+    for (int b = 0; b < 4; ++b)
+        for (int i = 0; i < 8; ++i) {
+            for (int n = 0; n < (1 << i); ++n) t.step[b][(1 << i) + n] = t.step[b][n] ^ v;
+            v = ((v << 1) & mask) ^ (((v >> (p.L - 1)) & 1u) ? p.g : 0u);
         }
+    v = 1;
+    for (int i = 0; i < p.L; ++i) v = ((v << 1) & mask) ^ (((v >> (p.L - 1)) & 1u) ? p.g : 0u);
+    for (int n = 0; n < S; ++n) {
+        t.last[n] = v;
+        for (int b = 0; b < 4; ++b) v = ((v << 8) & mask) ^ byte_entry((v >> (p.L - 8)) & 0xFFu, p);
     }
-    // shift by the words that follow this chunk: x^(32 * (nw - w1))
-    uint32_t m = (uint32_t)(nw - w1);
-    for (int j = 0; m && reg; ++j, m >>= 1)
-        if (m & 1u) reg = dmulmod(reg, g_crc_tables.pow32[kind][j], p.L, p.g);
-    // XOR-reduce over the workgroup
-    for (int off = 32; off > 0; off >>= 1) reg ^= __shfl_xor(reg, off, 64);
-    if ((tid & 63) == 0) lds_red[tid >> 6] = reg;
-    __syncthreads();
+    return t;
+}
+
+// v * f mod g, v any 32-bit value, f < 2^L.
+template <int L, uint32_t G> __device__ __forceinline__ uint32_t mulmod32(uint32_t v, uint32_t f)
+{
+    constexpr uint32_t mask = (1u << L) - 1u;
     uint32_t r = 0;
-    for (int i = 0; i < (nt + 63) / 64; ++i) r ^= lds_red[i];
-    __syncthreads();
-    return r;
+#pragma unroll
+    for (int i = 31; i >= 0; --i) {
+        const uint32_t top = (uint32_t)((int32_t)(r << (31 - (L - 1))) >> 31);
+        const uint32_t bit = (uint32_t)((int32_t)(v << (31 - i)) >> 31);
+        r = (r << 1) ^ (top & G) ^ (bit & f);
+    }
+    return r & mask;
+}
+
+// Reduction of x over the wave, returned in every lane: within each row of
+// 16 lanes by DPP (lane pairs, quads, half rows, rows: register-to-register,
+// no LDS round trip), then across the four rows by readlane.  Every lane
+// of the wave must be active (workgroups of whole waves, called in uniform
+// control flow).
+template <typename Op> __device__ __forceinline__ uint32_t wave_reduce(uint32_t x, Op op)
+{
+    x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
+    x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
+    x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x140, 0xF, 0xF, false));  // row_mirror
+    const auto at = [&](int l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, l); };
+    return op(op(at(0), at(16)), op(at(32), at(48)));
+}
+__device__ __forceinline__ uint32_t wave_xor(uint32_t x)
+{
+    return wave_reduce(x, [](uint32_t a, uint32_t b) { return a ^ b; });
+}
+
+// Share of the remainder of nw message words (`word(i)` = message word i,
+// its first bit the most significant) that thread t of S holds: the words
+// nw - 1 - t - S * i, by Horner's rule from the first, step(b, x) =
+// x * x^(8 b + 32 S) mod g from the stride table, then shifted to the end
+// with last = x^(32 t + L).  XOR over the threads gives the remainder.  The S
+// threads read consecutive words; a step is four independent table reads.
+template <int S, typename Word, typename Step, typename Mul>
+__device__ __forceinline__ uint32_t strided_crc(int nw, int t, Word word, Step step, uint32_t last, Mul mul)
+{
+    constexpr int U = 4;  // words in flight
+    uint32_t v = 0;
+    for (int i = (nw + S - 1) / S - 1; i >= 0; i -= U) {
+        uint32_t w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = (i - u) * S + t;  // words from the end
+            w[u] = (i >= u && e < nw) ? word(nw - 1 - e) : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i >= u) v = step(0, v & 255u) ^ step(1, (v >> 8) & 255u) ^ step(2, (v >> 16) & 255u) ^ step(3, v >> 24) ^ w[u];
+    }
+    return mul(v, last);
 }
 
 // Byte-granular shift factors: x^(8m) mod g for m < CRC_SHIFT_LO (shifts
@@ -170,40 +206,6 @@ constexpr crc_shift_tables make_crc_shift_tables()
 }
 
 static __device__ const crc_shift_tables g_crc_shift = make_crc_shift_tables();
-
-__device__ __forceinline__ uint32_t crc_poly_of(int kind) { return kind == K_CRC24A ? CRC24A_P.g : (kind == K_CRC24B ? CRC24B_P.g : CRC16_P.g); }
-__device__ __forceinline__ int crc_len_of(int kind) { return kind == K_CRC16 ? 16 : 24; }
-
-// Remainder of the nbytes message bytes byte_at(0 .. nbytes-1) (MSB-first
-// bytes), nbytes <= CRC_SHIFT_LO, computed by the workgroup with the byte
-// table T of the kind (in LDS): every thread a contiguous chunk, shifted by
-// x^(8 * bytes after it) with one multiplication, XOR-reduced.
-template <typename ByteFn>
-__device__ uint32_t block_crc_bytes(int nbytes, int kind, ByteFn byte_at, const uint32_t* T, uint32_t* lds_red)
-{
-    const int L = crc_len_of(kind);
-    const uint32_t g = crc_poly_of(kind);
-    const uint32_t mask = (1u << L) - 1u;
-    const int nt = blockDim.x, tid = threadIdx.x;
-    const int per = (nbytes + nt - 1) / nt;
-    const int b0 = min(nbytes, tid * per), b1 = min(nbytes, b0 + per);
-    uint32_t reg = 0;
-    for (int b = b0; b < b1; ++b) reg = ((reg << 8) & mask) ^ T[((reg >> (L - 8)) ^ byte_at(b)) & 0xFFu];
-    if (reg && nbytes > b1) reg = dmulmod(reg, g_crc_shift.lo[kind][nbytes - b1], L, g);
-    for (int off = 32; off > 0; off >>= 1) reg ^= __shfl_xor(reg, off, 64);
-    if ((tid & 63) == 0) lds_red[tid >> 6] = reg;
-    __syncthreads();
-    uint32_t r = 0;
-    for (int i = 0; i < (nt + 63) / 64; ++i) r ^= lds_red[i];
-    __syncthreads();
-    return r;
-}
-
-// x^(8n) mod g24A for n < 256 KiB.
-__device__ __forceinline__ uint32_t crc24a_shift_bytes(uint32_t n)
-{
-    return dmulmod(g_crc_shift.lo[K_CRC24A][n & 1023u], g_crc_shift.tb_hi[(n >> 10) & 255u], 24, CRC24A_P.g);
-}
 
 // CRC bits attached to each CB: 24 (CRC24B) when the TB is segmented.
 __device__ __forceinline__ int cb_crc_bits(const PerTbParams& p)

@@ -24,7 +24,8 @@ struct crc_descriptor {
 void* crc_cb_kernel_ptr();
 void* crc_tb_kernel_ptr();
 
-constexpr unsigned CRC_CB_BLOCK = 64;
-constexpr unsigned CRC_TB_BLOCK = 256;
+constexpr int CRC_CBS_PER_BLOCK = 4;  // code blocks (waves) per workgroup of the CB kernel
+constexpr unsigned CRC_CB_BLOCK = 64 * CRC_CBS_PER_BLOCK;
+constexpr unsigned CRC_TB_BLOCK = 1024;
 
 }  // namespace nrldpc

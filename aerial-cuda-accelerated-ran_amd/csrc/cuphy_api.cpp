@@ -651,7 +651,9 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxCrcDecode(cuphyPuschRxCrcDecodeHndl_t
     pCbCrcLaunchCfg->desc = pGpuDesc;
     pCbCrcLaunchCfg->kernelArgs[0] = &pCbCrcLaunchCfg->desc;
     set_node(pCbCrcLaunchCfg->kernelNodeParamsDriver, nrldpc::crc_cb_kernel_ptr(),
-             dim3(std::max(1u, cmax), std::max<unsigned>(1, nSchUes), 1), dim3(nrldpc::CRC_CB_BLOCK),
+             dim3((std::max(1u, cmax) + nrldpc::CRC_CBS_PER_BLOCK - 1) / nrldpc::CRC_CBS_PER_BLOCK,
+                  std::max<unsigned>(1, nSchUes), 1),
+             dim3(nrldpc::CRC_CB_BLOCK),
              pCbCrcLaunchCfg->kernelArgs);
     pTbCrcLaunchCfg->desc = pGpuDesc;
     pTbCrcLaunchCfg->kernelArgs[0] = &pTbCrcLaunchCfg->desc;

@@ -292,3 +292,43 @@ def test_crc_decode_matches_oracle(reverse):
     # pass/fail pattern: only the corrupted TBs fail
     assert [int(got_tb[t] != 0) for t in range(len(refs))] == [0, 1, 0, 0, 1, 0]
     crc.close()
+
+
+def test_crc_decode_many_shapes():
+    """90 TBs of one setup (more than a wave's lanes of TBs before a TB), 1 to
+    9 code blocks and one TB of 150: every alignment of a block's bytes in
+    its TB, one to 264 words per block, CRC16 / CRC24A / CRC24B; random words,
+    so that the remainders are arbitrary values."""
+    _need_gpu()
+    from aerial_amd.pusch import CrcDecode, make_tb_params
+    rng = np.random.RandomState(12)
+    shapes = [(1, 32), (1, 40), (2, 40), (1, 8448), (3, 8448), (150, 8424)]
+    shapes += [(int(rng.randint(1, 10)), 8 * int(rng.randint(5, 1057))) for _ in range(84)]
+    print("[case] crc %d TBs" % len(shapes), flush=True)
+    params, words, refs = [], [], []
+    for C, Kp in shapes:
+        bg = 1 if Kp > 3840 else 2
+        Zc = next(z for z in sorted({a << j for a in (2, 3, 5, 7, 9, 11, 13, 15) for j in range(8)})
+                  if (22 if bg == 1 else 10) * z >= Kp)
+        params.append(make_tb_params(bg, Zc, C, Kp, 2, 1, C * 4000, 0)[0])
+        w = rng.randint(0, 1 << 32, (C, O.WORDS_PER_CB), dtype=np.uint64).astype(np.uint32)
+        w[:, (Kp + 31) // 32:] = 0
+        if Kp % 32:
+            w[:, Kp // 32] &= np.uint32((1 << (Kp % 32)) - 1)
+        words.append(w)
+        refs.append(O.crc_desegment(w.reshape(-1), C, Kp))
+    ncb = sum(C for C, _ in shapes)
+    cb_crc = torch.full((ncb,), -1, dtype=torch.int32, device="cuda")
+    tb_crc = torch.full((len(params),), -1, dtype=torch.int32, device="cuda")
+    nby = sum(len(r[1]) for r in refs)
+    tb_bytes = torch.full((nby + 64,), 0xAB, dtype=torch.uint8, device="cuda")
+    crc = CrcDecode(reverse_bytes=True)
+    crc.run(params, torch.from_numpy(np.concatenate(words).reshape(-1).view(np.int32).copy()).cuda(), cb_crc, tb_bytes,
+            tb_crc)
+    torch.cuda.synchronize()
+    assert np.array_equal(cb_crc.cpu().numpy().view(np.uint32), np.concatenate([r[0] for r in refs]))
+    assert np.array_equal(tb_crc.cpu().numpy().view(np.uint32), np.array([r[2] for r in refs], np.uint32))
+    got = tb_bytes.cpu().numpy()
+    assert np.array_equal(got[:nby], np.concatenate([np.asarray(r[1]) for r in refs]))
+    assert np.all(got[nby:] == 0xAB)
+    crc.close()
