@@ -557,6 +557,7 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxRateMatch(cuphyPuschRxRateMatchHndl_t
     const rm_object& o = static_cast<const rm_object&>(*puschRxRateMatchHndl);
     nrldpc::rm_descriptor& d = *static_cast<nrldpc::rm_descriptor*>(pCpuDesc);
     uint32_t cmax = 0;
+    std::array<uint32_t, MAX_N_TBS_SUPPORTED> max_e;
     for (uint32_t i = 0; i < nSchUes; ++i) {
         const uint16_t ue = pSchUserIdxsCpu[i];
         const PerTbParams& p = pTbPrmsCpu[ue];
@@ -567,12 +568,14 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxRateMatch(cuphyPuschRxRateMatchHndl_t
         else
             d.llr_in[i] = (p.nDmrsCdmGrpsNoData == 1 ? pTPrmCdm1RmIn : pTPrmRmIn)[p.userGroupIndex].pAddr;
         cmax = std::max(cmax, p.num_CBs);
-        if (o.descrambling && !p.uciOnPuschFlag && rm_max_E(p) > nrldpc::RM_MAX_DESCR_E)
+        max_e[i] = rm_max_E(p);
+        if (o.descrambling && !p.uciOnPuschFlag && max_e[i] > nrldpc::RM_MAX_DESCR_E)
             return CUPHY_STATUS_UNSUPPORTED_CONFIG;  // more descrambling bits per CB than the kernel holds
     }
     d.out = ppRmOut;
     d.tb_prms = pTbPrmsGpu;
     d.descrambling_on = o.descrambling ? 1 : 0;
+    d.lds_bytes = nrldpc::rm_lds_bytes(o.fpconfig, max_e.data(), nSchUes, o.descrambling);
     if (enableCpuToGpuDescrAsyncCpy &&
         hipMemcpyAsync(pGpuDesc, pCpuDesc, sizeof(nrldpc::rm_descriptor), hipMemcpyHostToDevice, strm) != hipSuccess)
         return CUPHY_STATUS_MEMCPY_ERROR;
@@ -580,6 +583,7 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxRateMatch(cuphyPuschRxRateMatchHndl_t
     pLaunchCfg->kernelArgs[0] = &pLaunchCfg->desc;
     set_node(pLaunchCfg->kernelNodeParamsDriver, nrldpc::rm_kernel(o.fpconfig, o.descrambling), dim3(std::max(1u, cmax), std::max<unsigned>(1, nSchUes), 1),
              dim3(nrldpc::RM_BLOCK), pLaunchCfg->kernelArgs);
+    pLaunchCfg->kernelNodeParamsDriver.sharedMemBytes = (unsigned)d.lds_bytes;
     set_node(pLaunchCfg->resetKernelNodeParamsDriver, nrldpc::rm_noop_kernel(), dim3(1), dim3(64), pLaunchCfg->kernelArgs);
     set_node(pLaunchCfg->clampKernelNodeParamsDriver, nrldpc::rm_noop_kernel(), dim3(1), dim3(64), pLaunchCfg->kernelArgs);
     if (nSchUes == 0) pLaunchCfg->kernelNodeParamsDriver.func = nrldpc::rm_noop_kernel();

@@ -1,7 +1,7 @@
 // Host/device interface of the PUSCH de-rate-match kernel (derate_match.hip).
 #pragma once
 
-#include <hip/hip_runtime_api.h>
+#include <hip/hip_runtime.h>
 
 #include "cuphy_hip.h"
 
@@ -15,6 +15,7 @@ struct rm_descriptor {
     void** out;                               // HARQ buffer of each UE index
     const PerTbParams* tb_prms;               // device copy, indexed by UE index
     int descrambling_on;
+    int lds_bytes;                            // dynamic LDS of the launch (rm_lds_bytes)
 };
 
 // Kernel of a FP configuration (0: fp32->fp32, 1: fp16->fp32, 2: fp32->fp16,
@@ -28,5 +29,17 @@ constexpr unsigned RM_BLOCK = 256;
 // may start anywhere in a word).
 constexpr int RM_SEQ_WORDS = 12288;
 constexpr int RM_MAX_DESCR_E = 32 * (RM_SEQ_WORDS - 1);
+
+// Dynamic LDS of a launch whose TBs have at most max_e[i] bits per CB: each
+// CB's descrambling words and, up to RM_LDS_LIMIT bytes in all (the size a
+// kernel gets without asking for more), its LLRs.
+constexpr int RM_LDS_LIMIT = 64 * 1024;
+int rm_lds_bytes(int fpconfig, const uint32_t* max_e, int n, bool descrambling);
+
+// Whether a CB of E LLRs of `elem` bytes fits after seq_words words.
+__host__ __device__ inline bool rm_staged_fits(int E, int elem, uint32_t seq_words, uint32_t lds_words)
+{
+    return (uint64_t)seq_words + ((uint64_t)(uint32_t)E * (uint32_t)elem + 3u) / 4u <= lds_words;
+}
 
 }  // namespace nrldpc

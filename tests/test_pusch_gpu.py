@@ -332,3 +332,52 @@ def test_crc_decode_many_shapes():
     assert np.array_equal(got[:nby], np.concatenate([np.asarray(r[1]) for r in refs]))
     assert np.all(got[nby:] == 0xAB)
     crc.close()
+
+
+# (bg, Zc, CBs, K', Qm, layers, E per CB, rv, UE LLR offset in values, harq offset in values)
+RM_EDGES = [(2, 2, 3, 16, 1, 1, 5, 0, 0, 0),              # fewer LLRs than a 16-byte group, circle of 96 positions
+            (2, 2, 1, 16, 2, 1, 700, 3, 0, 0),             # every position seven times and more
+            (1, 13, 2, 264, 6, 2, 12 * 37, 1, 0, 0),       # odd sizes, wrap and filler inside groups
+            (1, 384, 2, 8448, 8, 1, 25344, 0, 0, 0),       # the whole buffer exactly once
+            (1, 384, 1, 8448, 8, 1, 32768, 2, 0, 0),       # the most LLRs staged in binary16
+            (1, 384, 1, 8448, 8, 1, 32776, 2, 0, 0),       # one symbol more: over memory
+            (1, 208, 2, 4400, 4, 2, 8000, 2, 3, 0),        # LLRs not aligned to a symbol's load
+            (2, 104, 2, 1000, 8, 1, 2400, 3, 0, 5)]        # HARQ buffer not aligned to 16 bytes
+
+
+@pytest.mark.parametrize("fp,descr", [(3, False), (3, True), (0, True)])
+@pytest.mark.parametrize("case", RM_EDGES)
+def test_derate_match_edges(case, fp, descr):
+    """First transmission, then two combined, at the edges of the staged
+    form: groups of 16 bytes, LDS limit, alignment, repetition."""
+    _need_gpu()
+    from aerial_amd.pusch import DeRateMatch, make_tb_params
+    bg, Zc, C, Kp, Qm, Nl, E, rv, in_off, out_off = case
+    print("[case] derate edges BG%d Zc=%d C=%d K'=%d Qm=%d Nl=%d E=%d rv=%d offsets %d %d" % case
+          + " fp=%d descr=%d" % (fp, descr), flush=True)
+    half = fp == 3
+    dt = torch.float16 if half else torch.float32
+    rm = DeRateMatch(fp_config=fp, descrambling=descr)
+    p, _ = make_tb_params(bg, Zc, C, Kp, Qm, Nl, C * E, rv)
+    size, n = C * p.Ncb_padded, 2 * Zc + p.Ncb
+    ref = np.zeros(size, np.float32)
+    harq = torch.full((size + out_off,), 55.0, dtype=dt, device="cuda")[out_off:]
+    for tx in range(3):
+        p, _ = make_tb_params(bg, Zc, C, Kp, Qm, Nl, C * E, (rv + 2 * tx) % 4, ndi=1 if tx == 0 else 0)
+        p.cinit = 0x155AA3 if descr else 0
+        ocfg = O.rm_cfg(bg=bg, Zc=Zc, C=C, Qm=Qm, Nl=Nl, G=C * E, K=p.K, F=p.F, Ncb=p.Ncb, Ncb_padded=p.Ncb_padded,
+                        k0=p.k0, ndi=p.ndi, descramble=int(descr), cinit=p.cinit)
+        llr = tb_llrs(max(C * E, 50), 90 + tx)[:C * E]
+        if half:
+            llr = llr.astype(np.float16).astype(np.float32)
+        O.derate_match(ocfg, llr, ref, fp16=half)
+        buf = torch.from_numpy(qam_stride_layout(llr, Qm, Nl, Nl, list(range(Nl)))).cuda().to(dt)
+        x = torch.zeros(buf.numel() + in_off, dtype=dt, device="cuda")[in_off:]
+        x.copy_(buf)
+        rm.run([p], [x], [harq])
+        torch.cuda.synchronize()
+        got = harq.float().cpu().numpy().reshape(C, -1)
+        exp = ref.reshape(C, -1)
+        assert np.array_equal(got[:, :n].view(np.uint32), exp[:, :n].view(np.uint32)), tx
+        assert np.all(got[:, n:] == 55.0), "padding written"
+    rm.close()
