@@ -1,0 +1,42 @@
+"""Upload of a call's small host structures (parameters, descriptors, pointer
+arrays) as one block: packed in page-locked host memory, copied to the device
+by one asynchronous copy on the launching stream.  Separate copies from
+pageable memory each wait for the stream's earlier work before the call can
+go on, so that a call's host time and its kernels never overlap.  Both blocks
+come from torch's caching allocators, which hand the host block out again
+only after the copy has run and the device block in the stream's order."""
+import contextlib
+import ctypes as C
+
+import torch
+
+_ALIGN = 64
+
+
+class UploadBlock:
+    """Space for parts of the given sizes; part i at host(i) / dev(i)."""
+
+    def __init__(self, sizes):
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("host parameters cannot be uploaded while the stream is being captured")
+        self._off, n = [], 0
+        for s in sizes:
+            self._off.append(n)
+            n += (s + _ALIGN - 1) // _ALIGN * _ALIGN
+        self._host = torch.empty(max(n, 1), dtype=torch.uint8, pin_memory=True)
+        self._dev = torch.empty(max(n, 1), dtype=torch.uint8, device="cuda")
+        self._hptr, self._dptr = self._host.data_ptr(), self._dev.data_ptr()
+
+    def host(self, i):
+        return self._hptr + self._off[i]
+
+    def dev(self, i):
+        return C.c_void_p(self._dptr + self._off[i])
+
+    def send(self):
+        self._dev.copy_(self._host, non_blocking=True)
+
+
+def on_stream(stream):
+    """Context in which blocks belong to the launching stream."""
+    return torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext()

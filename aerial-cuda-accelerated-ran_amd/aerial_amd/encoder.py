@@ -16,8 +16,9 @@ import torch
 
 from . import _hip
 from . import _lib as L
+from ._upload import UploadBlock, on_stream
 from .decoder import _stream_handle
-from .pusch import params_to_device, set_per_tb_params
+from .pusch import put_params, set_per_tb_params
 
 
 def pack_bits(bits):
@@ -68,10 +69,8 @@ class LdpcEncoder:
         dsz, dal, wsz = C.c_size_t(), C.c_size_t(), C.c_size_t()
         L.check("cuphyLDPCEncodeGetDescrInfo",
                 self._lib.cuphyLDPCEncodeGetDescrInfo(C.byref(dsz), C.byref(dal), max_tbs, C.byref(wsz)))
-        self.cpu_desc = (C.c_uint8 * dsz.value)()
-        self.gpu_desc = torch.zeros(dsz.value, dtype=torch.uint8, device="cuda")
-        self.h_ws = (C.c_uint8 * wsz.value)()
-        self.d_ws = torch.zeros(wsz.value, dtype=torch.uint8, device="cuda")
+        self.cpu_desc = (C.c_uint8 * dsz.value)()  # (the kernel takes it by value)
+        self._ws_bytes = wsz.value
         self.cfg = L.LDPCEncodeLaunchConfig()
 
     def encode_words(self, bg, Z, info_words, num_rows=0, rv=0, stream=None):
@@ -85,18 +84,23 @@ class LdpcEncoder:
         rows = num_rows if (rv == 0 and 0 < num_rows < (46 if bg == 1 else 42)) else (46 if bg == 1 else 42)
         nbits = (nsys + rows) * Z - (2 * Z if self.puncturing else 0)
         out_words = (nbits + 31) // 32
-        outs = [torch.empty((ncw, out_words), dtype=torch.int32, device="cuda") for _ in range(n)]
+        # contiguous tensors of one allocation
+        outs = list(torch.empty((n, ncw, out_words), dtype=torch.int32, device="cuda").unbind(0))
         tin = _BitTensor(in_words * 32, ncw, in_words * 32)
         tout = _BitTensor(out_words * 32, ncw, out_words * 32)
         in_ptrs = (C.c_void_p * n)(*[x.data_ptr() for x in info_words])
         out_ptrs = (C.c_void_p * n)(*[o.data_ptr() for o in outs])
-        st = self._lib.cuphySetupLDPCEncode(
-            C.byref(self.cfg), tin.h, None, tout.h, None, bg, Z, int(self.puncturing), num_rows, rv, 1, n,
-            C.cast(in_ptrs, C.c_void_p), C.cast(out_ptrs, C.c_void_p), C.cast(self.h_ws, C.c_void_p),
-            C.c_void_p(self.d_ws.data_ptr()), C.cast(self.cpu_desc, C.c_void_p), C.c_void_p(self.gpu_desc.data_ptr()),
-            1, _stream_handle(stream))
-        L.check("cuphySetupLDPCEncode", st)
-        _hip.launch_node(self.cfg.m_kernelNodeParams, _stream_handle(stream))
+        with on_stream(stream):
+            ws = UploadBlock((self._ws_bytes,))  # the TBs' addresses
+            sh = _stream_handle(stream)
+            st = self._lib.cuphySetupLDPCEncode(
+                C.byref(self.cfg), tin.h, None, tout.h, None, bg, Z, int(self.puncturing), num_rows, rv, 1, n,
+                C.cast(in_ptrs, C.c_void_p), C.cast(out_ptrs, C.c_void_p), C.c_void_p(ws.host(0)), ws.dev(0),
+                C.cast(self.cpu_desc, C.c_void_p), None, 0, sh)
+            L.check("cuphySetupLDPCEncode", st)
+            ws.send()
+            _hip.launch_node(self.cfg.m_kernelNodeParams, sh)
+        self._ws = ws
         return outs
 
     def encode(self, code_blocks, tb_sizes, code_rates, redundancy_versions):
@@ -123,11 +127,21 @@ def dl_rate_match(params, coded_words, emax, scrambling=False, stream=None):
     (num_tbs, max_cbs, emax/32) int32 words, CB r of TB t in its slot."""
     n = len(params)
     max_cbs = max(p.num_CBs for p in params)
-    _, dev = params_to_device(params)
-    ptrs = torch.tensor([w.data_ptr() for w in coded_words], dtype=torch.int64, device="cuda")
-    out = torch.full((n, max_cbs, emax // 32), -1, dtype=torch.int32, device="cuda")
-    st = L.lib().cuphyHipDlRateMatch(C.c_void_p(dev.data_ptr()), n, C.c_void_p(ptrs.data_ptr()), max_cbs, emax,
-                                     int(scrambling), C.c_void_p(out.data_ptr()), _stream_handle(stream))
+    # a CB slot that no code block of its TB fills stays -1 (the kernel writes every word of the others)
+    shape = (n, max_cbs, emax // 32)
+    if all(p.num_CBs == max_cbs for p in params):
+        out = torch.empty(shape, dtype=torch.int32, device="cuda")
+    else:
+        out = torch.full(shape, -1, dtype=torch.int32, device="cuda")
+    with on_stream(stream):
+        blk = UploadBlock((n * C.sizeof(L.PerTbParams), 8 * n))
+        put_params(blk.host(0), params)
+        ptrs = (C.c_uint64 * n).from_address(blk.host(1))
+        for i, w in enumerate(coded_words):
+            ptrs[i] = w.data_ptr()
+        blk.send()
+        st = L.lib().cuphyHipDlRateMatch(blk.dev(0), n, blk.dev(1), max_cbs, emax, int(scrambling),
+                                         C.c_void_p(out.data_ptr()), _stream_handle(stream))
     L.check("cuphyHipDlRateMatch", st)
-    out._keep = (dev, ptrs)  # the argument buffers live until the caller synchronizes
+    out._keep = blk  # the argument buffers live as long as the result
     return out

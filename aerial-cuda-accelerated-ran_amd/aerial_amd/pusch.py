@@ -13,6 +13,7 @@ import torch
 
 from . import _hip
 from . import _lib as L
+from ._upload import UploadBlock, on_stream
 from .decoder import _stream_handle
 
 LLR_MAX_ABS = 10000.0
@@ -97,6 +98,14 @@ def params_to_device(params):
     return arr, torch.from_numpy(host).cuda()
 
 
+def put_params(address, params):
+    """PerTbParams array at a host address."""
+    arr = (L.PerTbParams * len(params)).from_address(address)
+    for i, p in enumerate(params):
+        arr[i] = p
+    return arr
+
+
 class DeRateMatch:
     """cuphyCreate/Setup/DestroyPuschRxRateMatch + launch of its kernel nodes."""
 
@@ -111,8 +120,7 @@ class DeRateMatch:
         sz, al = C.c_size_t(), C.c_size_t()
         L.check("cuphyPuschRxRateMatchGetDescrInfo",
                 self._lib.cuphyPuschRxRateMatchGetDescrInfo(C.byref(sz), C.byref(al)))
-        self.cpu_desc = (C.c_uint8 * sz.value)()
-        self.gpu_desc = torch.zeros(sz.value, dtype=torch.uint8, device="cuda")
+        self._desc_bytes = sz.value
         self.cfg = L.RateMatchLaunchCfg()
 
     def close(self):
@@ -124,21 +132,25 @@ class DeRateMatch:
         """params: list of PerTbParams (UE index = list index); llr_in: one
         device tensor per user group; harq_out: one device tensor per UE."""
         n = len(params)
-        self._host_prms, self._dev_prms = params_to_device(params)
         idx = (C.c_uint16 * n)(*range(n))
         tin = (L.TensorPrm * len(llr_in))()
         for i, t in enumerate(llr_in):
             tin[i].pAddr = t.data_ptr()
-        self._out_ptrs = torch.tensor([t.data_ptr() for t in harq_out], dtype=torch.int64).cuda()
-        st = self._lib.cuphySetupPuschRxRateMatch(
-            self.h, n, idx, self._host_prms, C.c_void_p(self._dev_prms.data_ptr()), tin, tin,
-            C.cast(C.c_void_p(self._out_ptrs.data_ptr()), C.POINTER(C.c_void_p)), C.cast(self.cpu_desc, C.c_void_p),
-            C.c_void_p(self.gpu_desc.data_ptr()), 1, C.c_void_p(C.addressof(self.cfg)), _stream_handle(stream))
-        L.check("cuphySetupPuschRxRateMatch", st)
-        sh = _stream_handle(stream)
-        _hip.launch_node(self.cfg.resetKernelNodeParamsDriver, sh)
-        _hip.launch_node(self.cfg.kernelNodeParamsDriver, sh)
-        _hip.launch_node(self.cfg.clampKernelNodeParamsDriver, sh)
+        with on_stream(stream):
+            blk = UploadBlock((self._desc_bytes, n * C.sizeof(L.PerTbParams), len(harq_out) * 8))
+            prms = put_params(blk.host(1), params)
+            ptrs = (C.c_uint64 * len(harq_out)).from_address(blk.host(2))
+            for i, t in enumerate(harq_out):
+                ptrs[i] = t.data_ptr()
+            sh = _stream_handle(stream)
+            st = self._lib.cuphySetupPuschRxRateMatch(
+                self.h, n, idx, prms, blk.dev(1), tin, tin, C.cast(blk.dev(2), C.POINTER(C.c_void_p)),
+                C.c_void_p(blk.host(0)), blk.dev(0), 0, C.c_void_p(C.addressof(self.cfg)), sh)
+            L.check("cuphySetupPuschRxRateMatch", st)
+            blk.send()
+            # (the library's reset and clamp nodes are empty kernels: nothing to launch)
+            _hip.launch_node(self.cfg.kernelNodeParamsDriver, sh)
+        self._block = blk
 
 
 class CrcDecode:
@@ -150,8 +162,7 @@ class CrcDecode:
         L.check("cuphyCreatePuschRxCrcDecode", self._lib.cuphyCreatePuschRxCrcDecode(C.byref(self.h), int(reverse_bytes)))
         sz, al = C.c_size_t(), C.c_size_t()
         L.check("cuphyPuschRxCrcDecodeGetDescrInfo", self._lib.cuphyPuschRxCrcDecodeGetDescrInfo(C.byref(sz), C.byref(al)))
-        self.cpu_desc = (C.c_uint8 * sz.value)()
-        self.gpu_desc = torch.zeros(sz.value, dtype=torch.uint8, device="cuda")
+        self._desc_bytes = sz.value
         self.cb_cfg = L.CrcDecodeLaunchCfg()
         self.tb_cfg = L.CrcDecodeLaunchCfg()
 
@@ -162,15 +173,18 @@ class CrcDecode:
 
     def run(self, params, cb_words, cb_crc, tb_bytes, tb_crc, stream=None):
         n = len(params)
-        self._host_prms, self._dev_prms = params_to_device(params)
         idx = (C.c_uint16 * n)(*range(n))
-        st = self._lib.cuphySetupPuschRxCrcDecode(
-            self.h, n, idx, C.c_void_p(cb_crc.data_ptr()), C.c_void_p(tb_bytes.data_ptr()),
-            C.c_void_p(cb_words.data_ptr()), C.c_void_p(tb_crc.data_ptr()), self._host_prms,
-            C.c_void_p(self._dev_prms.data_ptr()), C.cast(self.cpu_desc, C.c_void_p),
-            C.c_void_p(self.gpu_desc.data_ptr()), 1, C.c_void_p(C.addressof(self.cb_cfg)), C.c_void_p(C.addressof(self.tb_cfg)),
-            _stream_handle(stream))
-        L.check("cuphySetupPuschRxCrcDecode", st)
-        sh = _stream_handle(stream)
-        _hip.launch_node(self.cb_cfg.kernelNodeParamsDriver, sh)
-        _hip.launch_node(self.tb_cfg.kernelNodeParamsDriver, sh)
+        with on_stream(stream):
+            blk = UploadBlock((self._desc_bytes, n * C.sizeof(L.PerTbParams)))
+            prms = put_params(blk.host(1), params)
+            sh = _stream_handle(stream)
+            st = self._lib.cuphySetupPuschRxCrcDecode(
+                self.h, n, idx, C.c_void_p(cb_crc.data_ptr()), C.c_void_p(tb_bytes.data_ptr()),
+                C.c_void_p(cb_words.data_ptr()), C.c_void_p(tb_crc.data_ptr()), prms, blk.dev(1),
+                C.c_void_p(blk.host(0)), blk.dev(0), 0, C.c_void_p(C.addressof(self.cb_cfg)),
+                C.c_void_p(C.addressof(self.tb_cfg)), sh)
+            L.check("cuphySetupPuschRxCrcDecode", st)
+            blk.send()
+            _hip.launch_node(self.cb_cfg.kernelNodeParamsDriver, sh)
+            _hip.launch_node(self.tb_cfg.kernelNodeParamsDriver, sh)
+        self._block = blk
