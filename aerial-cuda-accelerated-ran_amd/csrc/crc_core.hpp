@@ -18,6 +18,7 @@ struct crc_poly {
 constexpr crc_poly CRC24A_P{0x864CFBu, 24};
 constexpr crc_poly CRC24B_P{0x800063u, 24};
 constexpr crc_poly CRC16_P{0x1021u, 16};
+enum { K_CRC24A = 0, K_CRC24B = 1, K_CRC16 = 2 };
 
 // a*b mod g (both < 2^L), carry-less
 constexpr uint32_t gf2_mulmod(uint32_t a, uint32_t b, crc_poly p)
@@ -33,10 +34,6 @@ constexpr uint32_t gf2_mulmod(uint32_t a, uint32_t b, crc_poly p)
     return r;
 }
 
-struct crc_tables {
-    uint32_t byte[3][256];   // byte-wise step: reg' = (reg << 8) ^ T[(reg >> (L-8)) ^ b]
-};
-
 constexpr uint32_t byte_entry(uint32_t v, crc_poly p)
 {
     const uint32_t mask = (1u << p.L) - 1u;
@@ -45,45 +42,8 @@ constexpr uint32_t byte_entry(uint32_t v, crc_poly p)
     return r;
 }
 
-constexpr crc_tables make_crc_tables()
-{
-    crc_tables t{};
-    const crc_poly ps[3] = {CRC24A_P, CRC24B_P, CRC16_P};
-    for (int k = 0; k < 3; ++k)
-        for (uint32_t v = 0; v < 256; ++v) t.byte[k][v] = byte_entry(v, ps[k]);
-    return t;
-}
-
-static __device__ const crc_tables g_crc_tables = make_crc_tables();
-
-enum { K_CRC24A = 0, K_CRC24B = 1, K_CRC16 = 2 };
-
-// a*b mod g for a compile-time polynomial (fully unrolled).
-template <int L, uint32_t G>
-__device__ __forceinline__ uint32_t cmulmod(uint32_t a, uint32_t b)
-{
-    constexpr uint32_t mask = (1u << L) - 1u;
-    // bit i of b and bit L-1 of r as all-ones / all-zero masks (sign-extending
-    // field extracts); bits of r above L-1 are left to fall out of the mask
-    // at the end, so that each step is a shift and two masked XORs
-    uint32_t r = 0;
-#pragma unroll
-    for (int i = L - 1; i >= 0; --i) {
-        const uint32_t top = (uint32_t)((int32_t)(r << (31 - (L - 1))) >> 31);
-        const uint32_t bit = (uint32_t)((int32_t)(b << (31 - i)) >> 31);
-        r = (r << 1) ^ (top & G) ^ (bit & a);
-    }
-    return r & mask;
-}
-
-__device__ __forceinline__ uint32_t rbit8x4(uint32_t w)
-{
-    // reverse the bits inside each byte (byte order kept)
-    w = ((w >> 1) & 0x55555555u) | ((w & 0x55555555u) << 1);
-    w = ((w >> 2) & 0x33333333u) | ((w & 0x33333333u) << 2);
-    w = ((w >> 4) & 0x0F0F0F0Fu) | ((w & 0x0F0F0F0Fu) << 4);
-    return w;
-}
+// The bits inside each byte reversed (byte order kept).
+__device__ __forceinline__ uint32_t rbit8x4(uint32_t w) { return __builtin_bswap32(__builtin_bitreverse32(w)); }
 
 // Multiplication of a 32-bit (unreduced) value by x^(32 * S) mod g, by
 // bytes: v * x^(32 S) = XOR over b of step[b][byte b of v]; and the factors
@@ -114,20 +74,6 @@ template <int S> constexpr crc_stride_table<S> make_crc_stride_table(crc_poly p)
     return t;
 }
 
-// v * f mod g, v any 32-bit value, f < 2^L.
-template <int L, uint32_t G> __device__ __forceinline__ uint32_t mulmod32(uint32_t v, uint32_t f)
-{
-    constexpr uint32_t mask = (1u << L) - 1u;
-    uint32_t r = 0;
-#pragma unroll
-    for (int i = 31; i >= 0; --i) {
-        const uint32_t top = (uint32_t)((int32_t)(r << (31 - (L - 1))) >> 31);
-        const uint32_t bit = (uint32_t)((int32_t)(v << (31 - i)) >> 31);
-        r = (r << 1) ^ (top & G) ^ (bit & f);
-    }
-    return r & mask;
-}
-
 // Reduction of x over the wave, returned in every lane: within each row of
 // 16 lanes by DPP (lane pairs, quads, half rows, rows: register-to-register,
 // no LDS round trip), then across the four rows by readlane.  Every lane
@@ -147,14 +93,80 @@ __device__ __forceinline__ uint32_t wave_xor(uint32_t x)
     return wave_reduce(x, [](uint32_t a, uint32_t b) { return a ^ b; });
 }
 
+// Lane index, opaque: what depends on it alone (table loads, addresses) is then
+// computed where it is used instead of being hoisted out of a persistent
+// kernel's item loop into registers held across the decode.
+__device__ __forceinline__ uint32_t opaque_lane()
+{
+    uint32_t t = threadIdx.x & 63u;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+// Remainder of carry-less products, on a wave: the products' XOR over the
+// lanes is reduced once, lane i contributing x^(L + i) mod g where bit L + i
+// of it is set.
+struct crc_fold_table {
+    uint32_t k[3][64];  // x^(L + i) mod g of CRC24A, CRC24B, CRC16
+};
+constexpr crc_fold_table make_crc_fold_table()
+{
+    crc_fold_table t{};
+    const crc_poly ps[3] = {CRC24A_P, CRC24B_P, CRC16_P};
+    for (int q = 0; q < 3; ++q) {
+        const uint32_t mask = (1u << ps[q].L) - 1u;
+        uint32_t v = ps[q].g;  // x^L mod g
+        for (int i = 0; i < 64; ++i) {
+            t.k[q][i] = v;
+            v = ((v << 1) & mask) ^ (((v >> (ps[q].L - 1)) & 1u) ? ps[q].g : 0u);
+        }
+    }
+    return t;
+}
+static __device__ const crc_fold_table g_crc_fold = make_crc_fold_table();
+
+// XOR over the wave of the 64-bit p, mod g (degree L, p < 2^(L + 64)), the
+// same value in every lane; fold: the lane's entry of the polynomial's fold
+// table.
+template <int L> __device__ __forceinline__ uint32_t wave_fold(uint32_t lane, uint32_t lo, uint32_t hi, uint32_t fold)
+{
+    const uint64_t c = ((uint64_t)wave_xor(hi) << 32) | wave_xor(lo);
+    const uint32_t bit = (lane < 64u - (uint32_t)L) ? (uint32_t)(c >> (lane + (uint32_t)L)) & 1u : 0u;
+    return ((uint32_t)c & ((1u << L) - 1u)) ^ wave_xor((0u - bit) & fold);
+}
+
+// XOR over the lanes of v * f mod g (v any 32-bit value, f < 2^24): 32
+// independent masked shifts per lane, one reduction.
+template <int L>
+__device__ __forceinline__ uint32_t wave_sum_products(uint32_t lane, uint32_t v, uint32_t f, uint32_t fold)
+{
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const uint32_t m = (uint32_t)((int32_t)(v << (31 - i)) >> 31);
+        lo ^= m & (f << i);
+        if (i > 8) hi ^= m & (f >> (32 - i));
+    }
+    return wave_fold<L>(lane, lo, hi, fold);
+}
+
+// a * b mod g for uniform a, b < 2^24 and a polynomial of degree 24: lane i
+// takes bit i of a.
+__device__ __forceinline__ uint32_t wave_mulmod24(uint32_t lane, uint32_t a, uint32_t b, uint32_t fold)
+{
+    const uint64_t p = (lane < 24u && ((a >> lane) & 1u)) ? (uint64_t)b << lane : 0u;
+    return wave_fold<24>(lane, (uint32_t)p, (uint32_t)(p >> 32), fold);
+}
+
 // Share of the remainder of nw message words (`word(i)` = message word i,
 // its first bit the most significant) that thread t of S holds: the words
 // nw - 1 - t - S * i, by Horner's rule from the first, step(b, x) =
-// x * x^(8 b + 32 S) mod g from the stride table, then shifted to the end
-// with last = x^(32 t + L).  XOR over the threads gives the remainder.  The S
-// threads read consecutive words; a step is four independent table reads.
-template <int S, typename Word, typename Step, typename Mul>
-__device__ __forceinline__ uint32_t strided_crc(int nw, int t, Word word, Step step, uint32_t last, Mul mul)
+// x * x^(8 b + 32 S) mod g from the stride table.  Multiplied by
+// x^(32 t + L) (the table's `last`) and XORed over the threads it gives the
+// remainder.  The S threads read consecutive words; a step is four
+// independent table reads.
+template <int S, typename Word, typename Step>
+__device__ __forceinline__ uint32_t strided_crc(int nw, int t, Word word, Step step)
 {
     constexpr int U = 4;  // words in flight
     uint32_t v = 0;
@@ -169,7 +181,7 @@ __device__ __forceinline__ uint32_t strided_crc(int nw, int t, Word word, Step s
         for (int u = 0; u < U; ++u)
             if (i >= u) v = step(0, v & 255u) ^ step(1, (v >> 8) & 255u) ^ step(2, (v >> 16) & 255u) ^ step(3, v >> 24) ^ w[u];
     }
-    return mul(v, last);
+    return v;
 }
 
 // Byte-granular shift factors: x^(8m) mod g for m < CRC_SHIFT_LO (shifts

@@ -68,17 +68,10 @@ __device__ __forceinline__ tb_layout layout_of(const crc_descriptor& d, int slot
 template <typename Word>
 __device__ __forceinline__ uint32_t wave_crc(int nw, int kind, Word word, const uint32_t (*table)[256])
 {
-    const auto step = [&](int b, uint32_t x) { return table[b][x]; };
-    const int t = (int)(threadIdx.x & 63u);
-    const uint32_t last = g_cb_stride[kind].last[t];
-    uint32_t v;
-    if (kind == K_CRC16)
-        v = strided_crc<64>(nw, t, word, step, last, mulmod32<CRC16_P.L, CRC16_P.g>);
-    else if (kind == K_CRC24B)
-        v = strided_crc<64>(nw, t, word, step, last, mulmod32<CRC24B_P.L, CRC24B_P.g>);
-    else
-        v = strided_crc<64>(nw, t, word, step, last, mulmod32<CRC24A_P.L, CRC24A_P.g>);
-    return wave_xor(v);
+    const uint32_t t = threadIdx.x & 63u;
+    const uint32_t last = g_cb_stride[kind].last[t], fold = g_crc_fold.k[kind][t];
+    const uint32_t v = strided_crc<64>(nw, (int)t, word, [&](int b, uint32_t x) { return table[b][x]; });
+    return kind == K_CRC16 ? wave_sum_products<16>(t, v, last, fold) : wave_sum_products<24>(t, v, last, fold);
 }
 
 __global__ __launch_bounds__(CRC_CB_BLOCK) void crc_cb_kernel(const crc_descriptor* __restrict__ desc)
@@ -136,16 +129,18 @@ __global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(const crc_descript
     if (p.num_CBs <= 1) return;
     const int t = threadIdx.x;
     (&table[0][0])[t] = (&g_tb_stride.step[0][0])[t];
-    const uint32_t last = g_tb_stride.last[t];
+    const uint32_t last = g_tb_stride.last[t], fold = g_crc_fold.k[K_CRC24A][t & 63];
     const tb_layout l = layout_of(d, slot);
     const int Kp = (int)(p.K - p.F);
     const int data_bytes = (Kp - 24 + 7) / 8;
     const int nw = ((int)p.num_CBs * data_bytes + 3) / 4;
     const uint32_t* tbw = reinterpret_cast<const uint32_t*>(d.tb_out + l.tb_byte_base);
     __syncthreads();
-    const uint32_t v = wave_xor(strided_crc<CRC_TB_BLOCK>(
-        nw, t, [&](int w) { return __builtin_bswap32(tbw[w]); },
-        [&](int b, uint32_t x) { return table[b][x]; }, last, mulmod32<CRC24A_P.L, CRC24A_P.g>));
+    const uint32_t v = wave_sum_products<24>(
+        (uint32_t)t & 63u,
+        strided_crc<CRC_TB_BLOCK>(
+            nw, t, [&](int w) { return __builtin_bswap32(tbw[w]); }, [&](int b, uint32_t x) { return table[b][x]; }),
+        last, fold);
     if ((t & 63) == 0) red[t >> 6] = v;
     __syncthreads();
     if (t < 64) {

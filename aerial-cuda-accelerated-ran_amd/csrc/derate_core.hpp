@@ -49,14 +49,19 @@ __device__ __forceinline__ rm_geometry rm_geometry_of(const PerTbParams& p, int 
     // the larger size compares with encodedSize as rate_matching.cu:345; it is used only for r > rr,
     // i.e. when q1 is not a multiple of C, where q*nq*C < total <= encodedSize holds either way
     const int Eh = El + nq * ((long long)q * nq * C < (long long)p.encodedSize ? 1 : 0);
+    // (E / Qm and start / Qm without dividing: El = Nl * Qm * q, Eh = El or Nl * Qm more)
+    const int sl = g.Nl * q, sh = sl + (Eh > El ? g.Nl : 0);
+    int first;  // the CB's first symbol
     if (cb_in_tb <= rr) {
         g.E = El;
-        g.start = cb_in_tb * El;
+        g.EQ = sl;
+        first = cb_in_tb * sl;
     } else {
         g.E = Eh;
-        g.start = (rr + 1) * El + (cb_in_tb - rr - 1) * Eh;
+        g.EQ = sh;
+        first = (rr + 1) * sl + (cb_in_tb - rr - 1) * sh;
     }
-    g.EQ = g.E / g.Qm;
+    g.start = first * g.Qm;
     g.Zc = (int)p.Zc;
     g.Ncb = (int)p.Ncb;
     g.F = (int)p.F;
@@ -65,7 +70,7 @@ __device__ __forceinline__ rm_geometry rm_geometry_of(const PerTbParams& p, int 
     const int k0 = (int)p.k0;
     g.c0 = (k0 < g.Kd) ? k0 : ((k0 <= g.Kd + g.F) ? g.Kd : k0 - g.F);
     g.ndi = p.ndi != 0;
-    g.adj = (g.start / g.Qm) * QAM_STRIDE;
+    g.adj = first * QAM_STRIDE;
     g.nbbu = (int)p.nBBULayers;
     g.uci = p.uciOnPuschFlag != 0;
     return g;

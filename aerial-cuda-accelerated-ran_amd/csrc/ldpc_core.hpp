@@ -746,38 +746,25 @@ __device__ __forceinline__ void store_hard(const T* __restrict__ app, int nbits,
     }
 }
 
-// Hard decisions as LSB-first 32-bit words into `out` (global) and into
-// `lds_words` (LDS), ending with a barrier.  Thread w builds word w from its
-// 32 APP values with 16-byte LDS reads (the buffer must hold whole groups of
+// Word w of a code block's hard decisions (APP <= 0 -> 1, LSB first) from its
+// 32 APP values, by 16-byte LDS reads (the buffer must hold whole groups of
 // 32 values); bits past nbits are 0.  Used by the fused slot kernel, whose
 // CRC pass reads the words back from LDS.
-template <typename T>
-__device__ __forceinline__ void store_hard_words(const T* __restrict__ app, int nbits, uint32_t* __restrict__ out,
-                                                 uint32_t* __restrict__ lds_words)
+template <typename T> __device__ __forceinline__ uint32_t hard_word(const T* __restrict__ app, int nbits, int w)
 {
     typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T))));
     constexpr int PER = 16 / (int)sizeof(T);  // values per 16-byte read
-    const int nwords = (nbits + 31) >> 5;
-    // opaque copy of the thread index: keeps the per-thread addresses from
-    // being hoisted out of a persistent kernel's item loop into registers
-    // held across the decode
-    int w0 = (int)threadIdx.x;
-    asm volatile("" : "+v"(w0));
-    for (int w = w0; w < nwords; w += blockDim.x) {
-        const vec_t* src = reinterpret_cast<const vec_t*>(app + 32 * w);
-        uint32_t word = 0;
+    const vec_t* src = reinterpret_cast<const vec_t*>(app + 32 * w);
+    uint32_t word = 0;
 #pragma unroll
-        for (int q = 0; q < 32 / PER; ++q) {
-            const vec_t v = src[q];
+    for (int q = 0; q < 32 / PER; ++q) {
+        const vec_t v = src[q];
 #pragma unroll
-            for (int e = 0; e < PER; ++e) word |= (uint32_t)(v[e] <= (T)0) << (q * PER + e);
-        }
-        const int tail = nbits - 32 * w;  // valid bits of this word
-        if (tail < 32) word &= (1u << tail) - 1u;
-        out[w] = word;
-        lds_words[w] = word;
+        for (int e = 0; e < PER; ++e) word |= (uint32_t)(v[e] <= (T)0) << (q * PER + e);
     }
-    __syncthreads();
+    const int tail = nbits - 32 * w;  // valid bits of this word
+    if (tail < 32) word &= (1u << tail) - 1u;
+    return word;
 }
 
 // Buffers of one code block of a group.

@@ -44,9 +44,20 @@
 
 namespace nrldpc {
 
+// Thread index, opaque: see opaque_lane.
+__device__ __forceinline__ int opaque_tid()
+{
+    int t = (int)threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
 constexpr uint32_t FUSED_CB_ERROR = 0xFFFFFFFFu;  // CRC value of a CB/TB whose parameters were rejected
 constexpr uint32_t TB_ACC_ERROR = 0x80000000u;    // accumulator flag: a CB of the TB was rejected
 constexpr int SLOT_CB_WORDS = MAX_DECODED_CODE_BLOCK_BIT_SIZE / 32;  // 264: decoded-word stride per CB
+
+static __device__ const crc_stride_table<64> g_wave_stride[3] = {
+    make_crc_stride_table<64>(CRC24A_P), make_crc_stride_table<64>(CRC24B_P), make_crc_stride_table<64>(CRC16_P)};
 
 template <typename TI> __device__ __forceinline__ float llr_as_float(TI v) { return (float)v; }
 
@@ -54,68 +65,109 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
 // LDS state of a workgroup besides the HARQ/APP array.
 struct fused_lds {
-    uint32_t words[SLOT_CB_WORDS];       // hard bits of the current CB
-    uint32_t crc_t[3][256];              // byte tables of the three CRCs
-    uint32_t shift[3][CRC_SHIFT_LO];     // x^(8m) mod g of the three CRCs
-    uint32_t red[2][8];
+    // hard bits of the item's CBs, one after another, each in whole words
+    uint32_t words[SLOT_CB_WORDS + FUSED_MAX_GROUP];
+    uint32_t step[3][4][256];            // CRC step tables of the three kinds (crc_stride_table<64>)
     uint32_t cb_flags[FUSED_MAX_GROUP];  // per-CB early-termination flags of a group
     uint32_t cb_iters[FUSED_MAX_GROUP];  // iterations each CB of a group ran
     int item, next;
 };
 
-// Remainder of one word's 4 message bytes (MSB-first bytes) with byte table T.
-template <int L>
-__device__ __forceinline__ uint32_t crc_word(uint32_t w, const uint32_t* T)
+// A lane's factors of a CRC: its last word's (crc_stride_table) and its fold
+// table entry.
+struct crc_lane {
+    uint32_t last, fold;
+};
+__device__ __forceinline__ crc_lane crc_lane_of(uint32_t lane, int kind)
 {
-    constexpr uint32_t mask = (1u << L) - 1u;
-    uint32_t reg = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) reg = ((reg << 8) & mask) ^ T[((reg >> (L - 8)) ^ (w >> (8 * b))) & 0xFFu];
-    return reg;
+    return {g_wave_stride[kind].last[lane], g_crc_fold.k[kind][lane]};
 }
 
-// The CB CRC (kind K of L bits over nb_cb = 4 * words bytes) and the CB's
-// TB-CRC24A share (over its db payload bytes, before the shift to its
-// place in the TB) in one pass: thread t takes word t, shifts its two
-// remainders by x^(8 * bytes after it) with factors from LDS, and both are
-// XOR-reduced together.
-template <int L, uint32_t G>
-__device__ __forceinline__ void cb_and_share_crc(const fused_lds& sh, const uint32_t* T, const uint32_t* S, int nb_cb,
-                                                 int db, uint32_t* red0, uint32_t* red1, uint32_t& crc,
-                                                 uint32_t& share)
+// Remainder of nw message words (the calling wave's 64 lanes, every 64th word
+// each: strided_crc), polynomial of degree L with step table `step`; word(i):
+// the i-th, its first bit the most significant.
+template <int L, typename Word>
+__device__ __forceinline__ uint32_t wave_crc(const uint32_t (*step)[256], int nw, Word word, uint32_t lane,
+                                             const crc_lane& f)
 {
-    const int t = threadIdx.x;
-    uint32_t rc = 0, rs = 0;
-    if (4 * t < nb_cb) {
-        // the two remainders as independent straight-line chains (a shift
-        // of 0 bytes multiplies by x^0 = 1), so that their table lookups
-        // and products interleave
-        const uint32_t w = rbit8x4(sh.words[t]);
-        const uint32_t* TA = sh.crc_t[K_CRC24A];
-        rc = crc_word<L>(w, T);
-        if (4 * t + 4 <= db) {
-            rs = crc_word<24>(w, TA);
-        } else if (4 * t < db) {  // the payload's last, partial word: bytes [4t, db)
-            for (int b = 0; b < db - 4 * t; ++b)
-                rs = ((rs << 8) & 0xFFFFFFu) ^ TA[((rs >> 16) ^ (w >> (8 * b))) & 0xFFu];
-        }
-        const int nb = max(0, min(4, db - 4 * t));
-        rc = cmulmod<L, G>(rc, S[nb_cb - 4 * t - 4]);
-        rs = cmulmod<24, CRC24A_P.g>(rs, sh.shift[K_CRC24A][max(0, db - 4 * t - nb)]);
+    const uint32_t v = strided_crc<64>(nw, (int)lane, word, [&](int b, uint32_t x) { return step[b][x]; });
+    return wave_sum_products<L>(lane, v, f.last, f.fold);
+}
+
+__device__ __forceinline__ void load_crc_steps(fused_lds& sh)
+{
+    for (int i = threadIdx.x; i < 3 * 1024; i += blockDim.x)
+        (&sh.step[0][0][0])[i] = (&g_wave_stride[i >> 10].step[0][0])[i & 1023];
+}
+
+// x^(-8 n) mod g24A, n = 0 .. 3 (g has a constant term: x^-1 = (g + 1) / x).
+constexpr uint32_t crc24a_unshift(int n)
+{
+    uint32_t v = 1;
+    for (int i = 0; i < 8 * n; ++i) v = gf2_mulmod(v, ((1u << 24) | CRC24A_P.g) >> 1, CRC24A_P);
+    return v;
+}
+
+// What the last steps of a TB's CBs share.
+struct cb_tail {
+    int Kp, kind, data_bytes, C;
+    uint32_t lane;            // of the calling thread
+    crc_lane cb, tb;          // the CB CRC's kind; CRC24A
+};
+
+// CB CRC of the decoded words (LDS), by the calling wave.
+__device__ __forceinline__ uint32_t cb_crc_of(const fused_lds& sh, const uint32_t* words, const cb_tail& t)
+{
+    const auto message = [&](int i) { return __builtin_bitreverse32(words[i]); };
+    const int nw = (t.Kp + 31) / 32;
+    return t.kind == K_CRC16 ? wave_crc<16>(sh.step[t.kind], nw, message, t.lane, t.cb)
+                             : wave_crc<24>(sh.step[t.kind], nw, message, t.lane, t.cb);
+}
+
+// Bytes from the end of a CB's share (payload filled up to whole words) to its
+// place in the TB: negative where the fill reaches past it.
+__device__ __forceinline__ int share_shift(int C, int data_bytes, int cb_in_tb)
+{
+    return (C * data_bytes + 3) / 4 * 4 - (cb_in_tb + 1) * data_bytes - (-data_bytes & 3);
+}
+
+// The CB's share of the TB CRC, by the calling wave.  TB CRC = XOR over CBs of
+// crc(payload bytes of CB c) * x^(8 * TB bytes after them), the TB zero-padded
+// to whole words (CRC linearity); the payload's last word is filled up with
+// zeros, which the shift to its place takes back.
+__device__ __forceinline__ uint32_t tb_share_of(const fused_lds& sh, const uint32_t* words, const cb_tail& t,
+                                                int cb_in_tb)
+{
+    const int nw = (t.data_bytes + 3) / 4;
+    const uint32_t keep = 0xFFFFFFFFu << (8 * (-t.data_bytes & 3));
+    const uint32_t part = wave_crc<24>(
+        sh.step[K_CRC24A], nw,
+        [&](int i) {
+            const uint32_t w = __builtin_bitreverse32(words[i]);
+            return i + 1 < nw ? w : w & keep;
+        },
+        t.lane, t.tb);
+    const int n = share_shift(t.C, t.data_bytes, cb_in_tb);
+    const uint32_t f = n < 0 ? (n == -1 ? crc24a_unshift(1) : n == -2 ? crc24a_unshift(2) : crc24a_unshift(3))
+                             : wave_mulmod24(t.lane, g_crc_shift.lo[K_CRC24A][n & 1023],
+                                             g_crc_shift.tb_hi[(n >> 10) & 255], t.tb.fold);
+    return wave_mulmod24(t.lane, part, f, t.tb.fold);
+}
+
+// The CB's payload bytes, by thread t of n: whole aligned words of the
+// destination, each from two decoded words, single bytes only at both ends.
+__device__ __forceinline__ void put_tb_bytes(const cuphyHipPuschSlotTb_t& job, int r, const uint32_t* words,
+                                             const cb_tail& tl, int t, int n)
+{
+    uint8_t* const dst = job.tb_bytes + (size_t)r * tl.data_bytes;
+    const int head = min(tl.data_bytes, (int)((0u - (uint32_t)(uintptr_t)dst) & 3u));
+    const int nfull = (tl.data_bytes - head) >> 2, tail = head + 4 * nfull;
+    for (int i = t; i < nfull; i += n) {
+        const uint32_t lo = rbit8x4(words[i]), hi = head ? rbit8x4(words[i + 1]) : 0u;
+        *reinterpret_cast<uint32_t*>(dst + head + 4 * i) = __builtin_amdgcn_alignbyte(hi, lo, (uint32_t)head);
     }
-    rc = wave_xor(rc);
-    rs = wave_xor(rs);
-    if ((t & 63) == 0) {
-        red0[t >> 6] = rc;
-        red1[t >> 6] = rs;
-    }
-    __syncthreads();
-    crc = share = 0;
-    for (int i = 0; i < (int)((blockDim.x + 63) / 64); ++i) {
-        crc ^= red0[i];
-        share ^= red1[i];
-    }
-    __syncthreads();
+    const int b = t < head ? t : tail + t - head;
+    if (t < head + tl.data_bytes - tail) dst[b] = (uint8_t)(rbit8x4(words[b >> 2]) >> (8 * (b & 3)));
 }
 
 // Combine this transmission's E LLRs of the CB into the LDS circular buffer
@@ -134,7 +186,7 @@ __device__ __forceinline__ void combine_tx(_Float16* __restrict__ cbuf, const TI
     for (int pass = 0; pass < npass; ++pass) {
         const int i0 = pass * g.L;
         const int span = min(g.L, g.E - i0);
-        int d = threadIdx.x;
+        int d = opaque_tid();
         if (d < span) {
             int c = g.c0 + d;  // circle position, kept in [0, L)
             while (c >= g.L) c -= g.L;
@@ -222,7 +274,7 @@ __device__ __forceinline__ void combine_symbols(_Float16* __restrict__ cbuf, con
     constexpr int NB = 4;  // symbols per thread in flight
     const int nthr = blockDim.x;
     const vec_t* sym = reinterpret_cast<const vec_t*>(in + g.adj);
-    for (int j0 = threadIdx.x; j0 < g.EQ; j0 += NB * nthr) {
+    for (int j0 = opaque_tid(); j0 < g.EQ; j0 += NB * nthr) {
         vec_t v[NB];
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
@@ -259,6 +311,102 @@ __device__ __forceinline__ void combine_symbols(_Float16* __restrict__ cbuf, con
     __syncthreads();
 }
 
+// Combining as combine_symbols where, besides, none of the Qm runs of EQ
+// positions wraps around the circle or crosses the filler: bit k of symbol j
+// then goes to position at(k) + j with a uniform at(k).  A first transmission
+// (ndi) reads nothing, its sum is LLR + 0.  Per LLR one add for the address,
+// convert, scale, round and add, instead of about 25 operations with the wrap
+// and filler tests; int8 LLRs whose scale keeps them within the clamp are not
+// clamped on their own.
+template <int QM, typename TI, bool DESCR>
+__device__ __forceinline__ void combine_runs(_Float16* __restrict__ cbuf, const TI* __restrict__ in,
+                                             const rm_geometry& g, float scale, const uint32_t* __restrict__ seq,
+                                             int soff)
+{
+    typedef typename slot_vec<TI>::type vec_t;
+    constexpr int NB = 4;  // symbols per thread in flight
+    const bool clamp = !(std::is_same<TI, int8_t>::value && __builtin_fabsf(scale) <= LLR_MAX_ABS / 128.0f);
+    const int nthr = blockDim.x;
+    const vec_t* sym = reinterpret_cast<const vec_t*>(in + g.adj);
+    int at[QM];
+    int c0 = g.c0, EQ = g.EQ;  // (opaque: not hoisted out of the switch over the modulation orders)
+    asm volatile("" : "+s"(c0), "+s"(EQ));
+#pragma unroll
+    for (int k = 0; k < QM; ++k) {
+        int c = c0 + k * EQ;
+        if (c >= g.L) c -= g.L;
+        at[k] = (c >= g.Kd) ? c + g.F : c;
+    }
+    for (int j0 = opaque_tid(); j0 < EQ; j0 += NB * nthr) {
+        vec_t v[NB];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const int j = j0 + u * nthr;
+            if (j < EQ) v[u] = sym[j];
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const int j = j0 + u * nthr;
+            if (j >= EQ) break;
+            _Float16 x[QM];
+#pragma unroll
+            for (int k = 0; k < QM; ++k) x[k] = (_Float16)(llr_as_float(v[u][k]) * scale);
+            if (clamp) {
+#pragma unroll
+                for (int k = 0; k < QM; ++k) x[k] = rm_num<_Float16>::clamp(x[k]);
+            }
+            if (DESCR) {  // bits n0 .. n0 + Qm - 1, n0 = soff + j * Qm (word n0/32 + 1 exists)
+                const int n0 = soff + j * QM;
+                const uint32_t bits = __builtin_amdgcn_alignbit(seq[(n0 >> 5) + 1], seq[n0 >> 5], (uint32_t)n0 & 31u);
+#pragma unroll
+                for (int k = 0; k < QM; ++k) x[k] = u2h((uint16_t)(h2u(x[k]) ^ ((bits << (15 - k)) & 0x8000u)));
+            }
+            if (g.ndi) {  // (0 + a clamped value is within the bounds)
+#pragma unroll
+                for (int k = 0; k < QM; ++k) cbuf[at[k] + j] = (_Float16)0.0f + x[k];
+            } else {
+                _Float16 prev[QM];
+#pragma unroll
+                for (int k = 0; k < QM; ++k) prev[k] = cbuf[at[k] + j];
+#pragma unroll
+                for (int k = 0; k < QM; ++k) cbuf[at[k] + j] = rm_num<_Float16>::clamp(prev[k] + x[k]);
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// Whether none of the Qm runs wraps or crosses the filler (E <= L).
+__device__ __forceinline__ bool runs_whole(const rm_geometry& g)
+{
+    int c = g.c0;
+    bool whole = true;
+    for (int k = 0; k < g.Qm; ++k) {
+        if (c >= g.L) c -= g.L;
+        whole = whole && c + g.EQ <= g.L && (c >= g.Kd || c + g.EQ <= g.Kd || g.F == 0);
+        c += g.EQ;
+    }
+    return whole;
+}
+
+// RUNS: the one-CB kernels, whose per-CB operations bound them (64-cell int8
+// slot with the tasks of step 6: 600 -> 572 us); the kernels of groups, bound by
+// their slowest CB, ran 436 -> 445 us on 64 UEs with it (registers).
+template <typename TI, bool DESCR, bool RUNS>
+__device__ __forceinline__ void combine_once(_Float16* __restrict__ cbuf, const TI* __restrict__ in,
+                                             const rm_geometry& g, float scale, const uint32_t* __restrict__ seq,
+                                             int soff)
+{
+    if (!RUNS || !runs_whole(g)) return combine_symbols<TI, DESCR>(cbuf, in, g, scale, seq, soff);
+    switch (g.Qm) {  // (uniform) modulation order as a constant
+    case 8: return combine_runs<8, TI, DESCR>(cbuf, in, g, scale, seq, soff);
+    case 6: return combine_runs<6, TI, DESCR>(cbuf, in, g, scale, seq, soff);
+    case 4: return combine_runs<4, TI, DESCR>(cbuf, in, g, scale, seq, soff);
+    case 2: return combine_runs<2, TI, DESCR>(cbuf, in, g, scale, seq, soff);
+    default: return combine_symbols<TI, DESCR>(cbuf, in, g, scale, seq, soff);
+    }
+}
+
 // Words of the descrambling sequence covering a CB's rate-matched bits
 // [start, start + E): from word start / 32 to word (start + E - 1) / 32.
 __device__ __forceinline__ int rm_seq_words(const rm_geometry& g)
@@ -270,7 +418,7 @@ __device__ __forceinline__ int rm_seq_words(const rm_geometry& g)
 // transmission combined (descrambled with `seq` when descr), the buffer
 // written back to HBM and converted in place to the decoder's APP array of
 // nval values.  Ends with a barrier.
-template <typename TI>
+template <typename TI, bool RUNS>
 __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_t* __restrict__ seq,
                                               const cuphyHipPuschSlotTb_t& job, const PerTbParams& p,
                                               const rm_geometry& g, int r, int nh, int nval, bool descr)
@@ -280,7 +428,7 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
     _Float16* harq = static_cast<_Float16*>(job.harq) + (size_t)r * ncb_padded;
     const TI* in = static_cast<const TI*>(job.llr);
     _Float16* cbuf = hb + 2 * Zc;
-    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int tid = opaque_tid(), nthr = blockDim.x;
     // 16-byte vector path when the HBM buffer is 16-byte aligned (LDS is)
     const bool vec = ((uintptr_t)harq & 15u) == 0;
     const int nv = vec ? nh / 8 : 0;
@@ -316,16 +464,16 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
     const bool sym_path = !g.uci && g.Nl == g.nbbu && g.E <= g.L &&
                           ((uintptr_t)(in + g.adj) % sizeof(typename slot_vec<TI>::type)) == 0;
     const int soff = g.start & 31;
-    if (descr) {
-        if (sym_path)
-            combine_symbols<TI, true>(cbuf, in, g, job.llr_scale, seq, soff);
+    const float scale = job.llr_scale;
+    if (!sym_path) {
+        if (descr)
+            combine_tx<TI, true>(cbuf, in, g, p, scale, seq, soff);
         else
-            combine_tx<TI, true>(cbuf, in, g, p, job.llr_scale, seq, soff);
+            combine_tx<TI, false>(cbuf, in, g, p, scale, seq, soff);
+    } else if (descr) {
+        combine_once<TI, true, RUNS>(cbuf, in, g, scale, seq, soff);
     } else {
-        if (sym_path)
-            combine_symbols<TI, false>(cbuf, in, g, job.llr_scale, seq, soff);
-        else
-            combine_tx<TI, false>(cbuf, in, g, p, job.llr_scale, seq, soff);
+        combine_once<TI, false, RUNS>(cbuf, in, g, scale, seq, soff);
     }
 
     // ---- 3. write back the HARQ buffer; APP = clamp(HARQ), +0 for -0 ----
@@ -335,12 +483,8 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
         half8_t v = reinterpret_cast<const half8_t*>(hb)[n];
         reinterpret_cast<half8_t*>(harq)[n] = v;
         if (n * 8 < nval) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                _Float16 a = v[e];
-                if (do_clamp) a = __builtin_fmaxf16(__builtin_fminf16(a, cl), -cl);
-                v[e] = (a == (_Float16)0) ? (_Float16)0 : a;
-            }
+            if (do_clamp) v = __builtin_elementwise_max(__builtin_elementwise_min(v, (half8_t)cl), (half8_t)(-cl));
+            v = v + (half8_t)(_Float16)0.0f;  // -0 -> +0
             reinterpret_cast<half8_t*>(hb)[n] = v;  // values past nval are not read by the decoder
         }
     }
@@ -364,7 +508,7 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
 // run CB by CB with the whole workgroup; the decode runs the group side by
 // side (lanes [c * Zc, (c + 1) * Zc) on CB c, each CB stopping on its own
 // syndrome: results as decoded alone); hard decisions and CRCs again CB by
-// CB.  Returns, in every thread, the XOR of the CBs' shares of the TB
+// CB.  Returns, in the completing thread, the XOR of the CBs' shares of the TB
 // CRC24A (each the remainder of the CB's payload bytes shifted to their
 // place in the TB; for a one-CB TB its CRC, which is the TB CRC), or
 // TB_ACC_ERROR when the group's parameters do not fit the launch (then only
@@ -383,7 +527,7 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     const int Zc = g0.Zc;
     const int bg = __builtin_amdgcn_readfirstlane((int)p.bg);
     const int nsys = bg == 1 ? 22 : 10;
-    const int mb = job.num_parity_nodes;
+    const int mb = __builtin_amdgcn_readfirstlane((int)job.num_parity_nodes);
     const int nh = 2 * Zc + g0.Ncb;
     const int nval = (nsys + mb) * Zc;
     const int arr = max(nh, nval);
@@ -405,7 +549,8 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     const bool ok = (bg == 1 || bg == 2) && z_index(Zc) >= 0 && mb >= 4 && mb <= (bg == 1 ? 46 : 42) &&
                     mb <= MAXR && count == count_in && count >= 1 && count <= FUSED_MAX_GROUP &&
                     count * Zc <= (int)blockDim.x &&
-                    (count - 1) * S + arr <= lds_values && Kb * Zc <= 32 * (int)SLOT_CB_WORDS && e_ok &&
+                    (count - 1) * S + arr <= lds_values && Kb * Zc <= 32 * (int)SLOT_CB_WORDS &&
+                    count * ((Kb * Zc + 31) >> 5) <= (int)(sizeof(sh.words) / sizeof(sh.words[0])) && e_ok &&
                     (!descr || seq_at + 2 * (nw_max + 1) <= lds_values);
     const int tid = threadIdx.x, nthr = blockDim.x;
     if (!ok) {
@@ -423,7 +568,7 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
             g = rm_geometry_of(p, cb0 + c);
             rm_make_uniform(g);
         }
-        fused_combine<TI>(hb + c * S, seq, job, p, g, r0 + c, nh, nval, descr);
+        fused_combine<TI, !GROUPED>(hb + c * S, seq, job, p, g, r0 + c, nh, nval, descr);
     }
 
     // ---- 4. decode -------------------------------------------------------
@@ -434,8 +579,8 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     dj.Z = Zc;
     dj.mb = mb;
     dj.Kb = Kb;
-    dj.max_iter = job.max_iterations;
-    dj.early_term = (job.flags & CUPHY_LDPC_DECODE_EARLY_TERM) != 0;
+    dj.max_iter = __builtin_amdgcn_readfirstlane((int)job.max_iterations);
+    dj.early_term = (__builtin_amdgcn_readfirstlane((int)job.flags) & CUPHY_LDPC_DECODE_EARLY_TERM) != 0;
     dj.clamp = job.clamp_value;
     dj.alpha_f32 = job.norm.f32;
     dj.alpha_f16 = (uint16_t)(job.norm.f16x2 & 0xFFFFu);
@@ -444,59 +589,65 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     const int iters = (bg == 1) ? run_iterations<1, _Float16, MAXR>(hb, dj, count, S, flags, cb_it)
                                 : run_iterations<2, _Float16, MAXR>(hb, dj, count, S, flags, cb_it);
 
-    // ---- 5-6. per CB: hard decisions, CB CRC, TB bytes, TB-CRC share --------
-    const int Kp = (int)(p.K - p.F);
+    // ---- 5. hard decisions of all CBs into LDS and memory --------------------
+    const int tt = opaque_tid();
+    const int nbits = Kb * Zc, nwc = (nbits + 31) >> 5;
     const int kind = cb_crc_kind(p);
-    const int data_bytes = cb_data_bytes(p);
-    const uint32_t* words = sh.words;
-    auto byte_of = [&](int b) { return (rbit8x4(words[b >> 2]) >> (8 * (b & 3))) & 0xFFu; };
-    uint32_t acc = 0;
-    for (int c = 0; c < count; ++c) {
-        const int r = r0 + c, cb_in_tb = cb0 + c;
-        store_hard_words<_Float16>(hb + c * S, Kb * Zc, job.cb_bits + (size_t)r * SLOT_CB_WORDS, sh.words);
-        if (job.cb_iterations && tid == 0) job.cb_iterations[r] = (uint8_t)(count == 1 ? iters : (int)sh.cb_iters[c]);
-        uint32_t crc, part;
-        if (kind == K_CRC16)
-            cb_and_share_crc<16, CRC16_P.g>(sh, sh.crc_t[kind], sh.shift[kind], 4 * ((Kp + 31) / 32), data_bytes,
-                                            sh.red[0], sh.red[1], crc, part);
-        else if (kind == K_CRC24B)
-            cb_and_share_crc<24, CRC24B_P.g>(sh, sh.crc_t[kind], sh.shift[kind], 4 * ((Kp + 31) / 32), data_bytes,
-                                             sh.red[0], sh.red[1], crc, part);
-        else
-            cb_and_share_crc<24, CRC24A_P.g>(sh, sh.crc_t[kind], sh.shift[kind], 4 * ((Kp + 31) / 32), data_bytes,
-                                             sh.red[0], sh.red[1], crc, part);
-        if (tid == 0) {
-            job.cb_crc[r] = crc;
-            if (cb_in_tb == 0) {
-                const int bytes = C * data_bytes;
-                for (int b = bytes; b < (bytes + 3) / 4 * 4; ++b) job.tb_bytes[b] = 0;
-            }
-        }
-        if (C > 1) {
-            // TB CRC = XOR over CBs of crc(payload bytes of CB c) * x^(8 * TB
-            // bytes after them), the TB zero-padded to whole words (CRC linearity)
-            const uint32_t total = (uint32_t)((C * data_bytes + 3) / 4 * 4);
-            const uint32_t after = total - (uint32_t)(cb_in_tb + 1) * (uint32_t)data_bytes;
-            // uniform operands: the two products run on the scalar unit
-            part = (uint32_t)__builtin_amdgcn_readfirstlane((int)part);
-            if (part && after) {
-                const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.shift[K_CRC24A][after & 1023u]);
-                part = cmulmod<24, CRC24A_P.g>(part,
-                                               cmulmod<24, CRC24A_P.g>(lo, g_crc_shift.tb_hi[(after >> 10) & 255u]));
-            }
-            acc ^= part;
-            // the group's share goes into the TB's accumulator now, so that
-            // the atomic's round trip overlaps the byte stores below
-            // (complete_cb raises the TB's count once it has returned)
-            if (c + 1 == count && tid == 0)
-                xor_prev = __hip_atomic_fetch_xor(tbw + 2u * job.share_offset, acc, __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_AGENT);
-        }
-        for (int b = tid; b < data_bytes; b += nthr) job.tb_bytes[(size_t)r * data_bytes + b] = (uint8_t)byte_of(b);
-        if (C == 1) return crc;
-        if (c + 1 < count) __syncthreads();  // the words in LDS are the next CB's
+    const uint32_t lane = (uint32_t)tt & 63u;
+    // (the CRCs' factors are loaded while the words are made)
+    const cb_tail tail{(int)(p.K - p.F), kind, cb_data_bytes(p), C, lane, crc_lane_of(lane, kind),
+                       crc_lane_of(lane, K_CRC24A)};
+    for (int i = tt; i < count * nwc; i += nthr) {
+        const int c = (GROUPED && count > 1) ? i / nwc : 0, w = i - c * nwc;
+        const uint32_t word = hard_word<_Float16>(hb + c * S, nbits, w);
+        job.cb_bits[(size_t)(r0 + c) * SLOT_CB_WORDS + w] = word;
+        sh.words[i] = word;
     }
-    return acc;
+    if (job.cb_iterations && tt < count) job.cb_iterations[r0 + tt] = (uint8_t)(count == 1 ? iters : (int)sh.cb_iters[tt]);
+    __syncthreads();
+
+    // ---- 6. CB CRC, TB bytes, TB-CRC share -----------------------------------
+    // A task per wave: the CBs' TB-CRC shares, then their CRCs, then their
+    // bytes (a one-CB TB: its CRC, which is the TB CRC, and its bytes), so that
+    // wave 0, whose first lane completes the TB, has the share or the TB CRC.
+    // (A word per thread with two 24-step products each, all waves alike, was
+    // 15 % of the kernel's vector instructions.)
+    const int wave = __builtin_amdgcn_readfirstlane(tt >> 6);
+    const bool lane0 = lane == 0;
+    uint32_t result = 0, prev = 0;
+    const bool one = !GROUPED || count == 1;  // (then all waves past the CRCs' share the bytes)
+    const int first_task = C > 1 ? 0 : 1;
+    for (int task = wave + first_task; one || task < 3 * count; task += nthr >> 6) {
+        const int what = one ? min(task, 2) : task / count;
+        const int c = one ? 0 : task - what * count;
+        const uint32_t* const words = sh.words + c * nwc;
+        if (what == 0) {
+            const uint32_t share = tb_share_of(sh, words, tail, cb0 + c);
+            // into the TB's accumulator now, so that the atomic's round trip
+            // overlaps the other tasks (complete_cb raises the TB's count)
+            if (lane0)
+                prev = __hip_atomic_fetch_xor(tbw + 2u * job.share_offset, share, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+        } else if (what == 1) {
+            result = cb_crc_of(sh, words, tail);
+            if (lane0) {
+                job.cb_crc[r0 + c] = result;
+                if (cb0 + c == 0) {
+                    const int bytes = C * tail.data_bytes;
+                    for (int b = bytes; b < (bytes + 3) / 4 * 4; ++b) job.tb_bytes[b] = 0;
+                }
+            }
+        } else {
+            const int skip = one ? 64 * (2 - first_task) : tt & ~63;
+            put_tb_bytes(job, r0 + c, words, tail, tt - skip, one ? nthr - skip : 64);
+        }
+        if (one) break;
+    }
+    // the other waves' shares are in the accumulator (their old values
+    // returned) before the caller's barrier; wave 0 hands its own on
+    if (GROUPED && wave > 0) asm volatile("" : : "v"(prev) : "memory");
+    xor_prev = prev;
+    return result;
 }
 
 // Workspace words of a TB (after the queue words): TB-CRC accumulator at
@@ -557,8 +708,7 @@ void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
     _Float16* hb = reinterpret_cast<_Float16*>(lds_raw);
     uint32_t* queue = ws;
     uint32_t* tbw = ws + FUSED_WS_QUEUE_WORDS;
-    for (int i = threadIdx.x; i < 3 * 256; i += blockDim.x) (&sh.crc_t[0][0])[i] = (&g_crc_tables.byte[0][0])[i];
-    for (int i = threadIdx.x; i < 3 * CRC_SHIFT_LO; i += blockDim.x) (&sh.shift[0][0])[i] = (&g_crc_shift.lo[0][0])[i];
+    load_crc_steps(sh);
     if (threadIdx.x == 0) sh.item = (int)atomicAdd(&queue[0], 1u);
     __syncthreads();
     for (;;) {
@@ -671,8 +821,7 @@ __global__ __launch_bounds__(384) void pusch_serve_resident(const serve_ring_hdr
     __shared__ PerTbParams s_prm;
     _Float16* hb = reinterpret_cast<_Float16*>(lds_raw);
     const int tid = threadIdx.x, nthr = blockDim.x;
-    for (int i = tid; i < 3 * 256; i += nthr) (&sh.crc_t[0][0])[i] = (&g_crc_tables.byte[0][0])[i];
-    for (int i = tid; i < 3 * CRC_SHIFT_LO; i += nthr) (&sh.shift[0][0])[i] = (&g_crc_shift.lo[0][0])[i];
+    load_crc_steps(sh);
     const uint64_t t_start = wall_clock64();
     bool first = true;
     for (;;) {
