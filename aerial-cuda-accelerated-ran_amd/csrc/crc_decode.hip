@@ -10,8 +10,7 @@
 //     copied into the TB byte buffer, MSB-first per byte when reverseBytes
 //     (bit 32w + i of the decoder output = bit i of word w);
 //   TB kernel -- CRC24A over the assembled TB bytes (zero-padded to whole
-//     words), one workgroup per TB, remainder 0 = pass (C = 1: the CB
-//     kernel's remainder).
+//     words), remainder 0 = pass (C = 1: the CB kernel's remainder).
 // Layouts as in the reference: CBs of TB y start at word sum_{i<y} C_i*264;
 // TB y's bytes start at sum_{i<y} roundup4(C_i * data_bytes_i).
 // CRC arithmetic (TS 38.212 5.1, zero initial value): thread t of S takes
@@ -22,14 +21,15 @@
 // One wave per code block, four to a workgroup (they share the TB's step
 // table in LDS); the TB's bytes go out as aligned words, each assembled from
 // two decoded words, with single bytes only at a block's ends.  The TB kernel
-// gives each TB one workgroup of 1,024 threads.  The offsets of a TB are sums
-// over the TBs before it, taken by the lanes of the wave.  Both kernels are
-// bound by their dependent loads (descriptor, parameters, words), not by the
-// 2 KB per code block.  Measured on 20 TBs of 140 BG1 Zc = 384 code blocks,
-// against contiguous chunks per thread with byte tables in global memory, one
-// loop over the TBs before and byte stores: CB kernel 30 -> 10.5 us, TB kernel
-// 73 -> 18 us (8 words in flight instead of 4, or 8 copies of the step table
-// against LDS bank conflicts, changed nothing).
+// gives each TB CRC_TB_PARTS workgroups, whose remainders meet in an XOR in the
+// descriptor (one workgroup reads 147 KB at 18 us, whatever its loads in flight).
+// The offsets of a TB are sums over the TBs before it, taken by the lanes of
+// the wave.  Both kernels are bound by their dependent loads (descriptor,
+// parameters, words), not by the 2 KB per code block.  Measured on 20 TBs of
+// 140 BG1 Zc = 384 code blocks, against contiguous chunks per thread with byte
+// tables in global memory, one loop over the TBs before and byte stores: CB
+// kernel 30 -> 9 us, TB kernel 73 -> 10 us (both with about 4 us that an empty
+// kernel measures the same way).
 #include "crc_core.hpp"
 #include "crc_decode.hpp"
 
@@ -39,8 +39,6 @@ namespace nrldpc {
 static __device__ const crc_stride_table<64> g_cb_stride[3] = {
     make_crc_stride_table<64>(CRC24A_P), make_crc_stride_table<64>(CRC24B_P), make_crc_stride_table<64>(CRC16_P)};
 static __device__ const crc_stride_table<CRC_TB_BLOCK> g_tb_stride = make_crc_stride_table<CRC_TB_BLOCK>(CRC24A_P);
-
-static_assert(CRC_TB_BLOCK == 4 * 256, "a thread per entry of the step table");
 
 struct tb_layout {
     int cb_word_base, cb_count_base, tb_byte_base;
@@ -119,7 +117,7 @@ __global__ __launch_bounds__(CRC_CB_BLOCK) void crc_cb_kernel(const crc_descript
     }
 }
 
-__global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(const crc_descriptor* __restrict__ desc)
+__global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(crc_descriptor* __restrict__ desc)
 {
     __shared__ uint32_t table[4][256];
     __shared__ uint32_t red[CRC_TB_BLOCK / 64];
@@ -128,25 +126,44 @@ __global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(const crc_descript
     const PerTbParams& p = d.tb_prms[d.sch_user_idxs[slot]];
     if (p.num_CBs <= 1) return;
     const int t = threadIdx.x;
-    (&table[0][0])[t] = (&g_tb_stride.step[0][0])[t];
+    for (int i = t; i < 4 * 256; i += CRC_TB_BLOCK) (&table[0][0])[i] = (&g_tb_stride.step[0][0])[i];
     const uint32_t last = g_tb_stride.last[t], fold = g_crc_fold.k[K_CRC24A][t & 63];
     const tb_layout l = layout_of(d, slot);
     const int Kp = (int)(p.K - p.F);
     const int data_bytes = (Kp - 24 + 7) / 8;
     const int nw = ((int)p.num_CBs * data_bytes + 3) / 4;
-    const uint32_t* tbw = reinterpret_cast<const uint32_t*>(d.tb_out + l.tb_byte_base);
+    // this workgroup's words [w0, w1) of the TB
+    const int per = (nw + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int w0 = min(nw, per * (int)blockIdx.y), w1 = min(nw, w0 + per);
+    const uint32_t* tbw = reinterpret_cast<const uint32_t*>(d.tb_out + l.tb_byte_base) + w0;
     __syncthreads();
     const uint32_t v = wave_sum_products<24>(
         (uint32_t)t & 63u,
         strided_crc<CRC_TB_BLOCK>(
-            nw, t, [&](int w) { return __builtin_bswap32(tbw[w]); }, [&](int b, uint32_t x) { return table[b][x]; }),
+            w1 - w0, t, [&](int w) { return __builtin_bswap32(tbw[w]); },
+            [&](int b, uint32_t x) { return table[b][x]; }),
         last, fold);
     if ((t & 63) == 0) red[t >> 6] = v;
     __syncthreads();
-    if (t < 64) {
-        const uint32_t crc = wave_xor(t < (int)(CRC_TB_BLOCK / 64) ? red[t] : 0u);
-        if (t == 0) d.tb_crc_out[slot] = crc;
-    }
+    if (t >= 64) return;
+    uint32_t crc = 0;
+    for (int i = 0; i < (int)(CRC_TB_BLOCK / 64); ++i) crc ^= red[i];
+    // shifted by the words after the part
+    const uint32_t n = 4u * (uint32_t)(nw - w1);
+    crc = wave_mulmod24((uint32_t)t, crc,
+                        wave_mulmod24((uint32_t)t, g_crc_shift.lo[K_CRC24A][n & 1023u],
+                                      g_crc_shift.tb_hi[(n >> 10) & 255u], fold),
+                        fold);
+    if (t != 0) return;
+    // XORed into the TB's accumulator before the part is counted; the last
+    // part takes the sum and puts both words back to zero
+    uint32_t prev = __hip_atomic_fetch_xor(&desc->tb_acc[slot], crc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" : "+v"(prev) : : "memory");
+    if (__hip_atomic_fetch_add(&desc->tb_parts[slot], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+        gridDim.y - 1u)
+        return;
+    d.tb_crc_out[slot] = __hip_atomic_exchange(&desc->tb_acc[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&desc->tb_parts[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 void* crc_cb_kernel_ptr() { return (void*)&crc_cb_kernel; }

@@ -331,6 +331,16 @@ def test_crc_decode_many_shapes():
     got = tb_bytes.cpu().numpy()
     assert np.array_equal(got[:nby], np.concatenate([np.asarray(r[1]) for r in refs]))
     assert np.all(got[nby:] == 0xAB)
+    # the TB kernel launched again from the same setup gives the same values
+    from aerial_amd import _hip
+    from aerial_amd.decoder import _stream_handle
+    for _ in range(2):
+        tb_crc.fill_(-1)
+        _hip.launch_node(crc.tb_cfg.kernelNodeParamsDriver, _stream_handle(None))
+        torch.cuda.synchronize()
+        want = np.array([r[2] for r in refs], np.uint32)
+        many = np.array([C > 1 for C, _ in shapes])  # (a one-CB TB's CRC is the CB kernel's)
+        assert np.array_equal(tb_crc.cpu().numpy().view(np.uint32)[many], want[many])
     crc.close()
 
 
