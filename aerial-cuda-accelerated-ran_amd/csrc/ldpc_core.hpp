@@ -101,10 +101,8 @@ template <int BG> constexpr uint64_t kBarrierMask = barrier_mask<bg_traits<BG>>(
 // compressed binary32 row state the slot row_slot[r].  Rows r < NR only.
 template <int BG, int NR> struct pair_plan {
     int group[64];
-    int row_slot[64];
     int pair_slot[64];  // binary16: first message slot of the row (even; rows padded to even degree)
     int edges[2];
-    int rows[2];
     int padded_edges[2];
 };
 template <int BG, int NR> constexpr pair_plan<BG, NR> make_pair_plan()
@@ -116,16 +114,56 @@ template <int BG, int NR> constexpr pair_plan<BG, NR> make_pair_plan()
         const bool first = (r == 0) || ((kBarrierMask<BG> >> r) & 1ull);
         const int g = first ? (p.edges[1] < p.edges[0] ? 1 : 0) : 1 - prev;
         p.group[r] = g;
-        p.row_slot[r] = p.rows[g];
         p.pair_slot[r] = p.padded_edges[g];
         p.edges[g] += BGT::row_start(r + 1) - BGT::row_start(r);
         p.padded_edges[g] += (BGT::row_start(r + 1) - BGT::row_start(r) + 1) & ~1;
-        p.rows[g] += 1;
         prev = g;
     }
     return p;
 }
 template <int BG, int NR> constexpr pair_plan<BG, NR> kPairPlan = make_pair_plan<BG, NR>();
+
+// binary32 state of a kernel holding NR block rows in PAIR lane groups: rows of
+// at most explicit_degree edges keep every edge's message (slot[r]: the first
+// of them), the others their compressed state (slot[r]: the row's).  An
+// explicit message costs about half the operations per edge (no rebuilding
+// of the previous one, no argmin); a row of D edges costs D registers then
+// instead of 3, so the degree is what the kernel's registers hold at its
+// occupancy: 168 per lane with two lane groups (three waves per SIMD), 256 with
+// one, 128 with at most SMALL_MAXR rows.  Measured, 8 code blocks Zc = 384,
+// all rows, two lane groups: BG1 213.6 -> 202.3 us, BG2 141.3 -> 120.2 us; 700
+// blocks BG2 R = 0.5 219 -> 190 us; no change where the rows' latency bounds
+// (BG1 Zc = 128: 151.2 -> 150.2 us).
+template <int BG, int NR, int PAIR> struct f32_plan {
+    bool is_explicit[64];
+    int slot[64];
+    int messages, rows;  // registers' worth of the larger lane group
+};
+constexpr int f32_explicit_degree(int BG, int NR, int PAIR)
+{
+    if (NR <= SMALL_MAXR) return BG == 1 ? 5 : 6;
+    if (PAIR == 2) return BG == 1 ? 5 : 10;
+    return BG == 1 ? 4 : 6;
+}
+template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> make_f32_plan()
+{
+    using BGT = bg_traits<BG>;
+    f32_plan<BG, NR, PAIR> p{};
+    int messages[2] = {0, 0}, rows[2] = {0, 0};
+    const pair_plan<BG, NR> pp = make_pair_plan<BG, NR>();
+    for (int r = 0; r < NR; ++r) {
+        const int g = (PAIR == 2) ? pp.group[r] : 0;
+        const int d = BGT::row_start(r + 1) - BGT::row_start(r);
+        p.is_explicit[r] = d <= f32_explicit_degree(BG, NR, PAIR);
+        int& next = p.is_explicit[r] ? messages[g] : rows[g];
+        p.slot[r] = next;
+        next += p.is_explicit[r] ? d : 1;
+    }
+    p.messages = messages[0] > messages[1] ? messages[0] : messages[1];
+    p.rows = rows[0] > rows[1] ? rows[0] : rows[1];
+    return p;
+}
+template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> kF32Plan = make_f32_plan<BG, NR, PAIR>();
 
 // binary16 message slots: row r's edges from padded_row_start(r) on, every
 // row's degree rounded up to even, so that each pair of a row's edges is one
@@ -318,6 +356,67 @@ __device__ __forceinline__ void process_row(float*, BP __restrict__ base, shift_
     st_n1[RS] = a1;
     st_n2[RS] = a2;
     st_meta[RS] = fs | (idx << 27);
+}
+
+// binary32 row with explicit messages st[S0 .. S0 + D): the update of the
+// binary16 rows, one edge per register.  With min1 / min2 the row's two
+// smallest |t|, g = min(|t|, min2) is min1 exactly for the argmin edge and min2
+// for every other one, so other = (min1 + min2) - g in integer arithmetic on
+// the bit patterns is the magnitude the edge takes (ties: min1 == min2, as the
+// first-index rule gives); the product with +-alpha has the magnitude
+// alpha * other rounded the same.  |t| is masked once, so that the minima
+// take the two-operand encodings, which issue at twice the rate of the
+// three-operand ones that an absolute-value modifier needs.
+__device__ __forceinline__ float fmin2(float a, float b)
+{
+    float r;
+    asm("v_min_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float fmax2(float a, float b)
+{
+    float r;
+    asm("v_max_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+template <int BG, int R, int NM, int S0, bool LM, typename BP, bool PK, bool SPL>
+__device__ __forceinline__ void process_row_explicit(BP __restrict__ base, shift_ptr sh, uint32_t zb, uint32_t zp,
+                                                     uint32_t Zb, float alpha, float (&st)[NM], uint32_t Pb)
+{
+    using BGT = bg_traits<BG>;
+    constexpr int E0 = BGT::row_start(R);
+    constexpr int D = BGT::row_start(R + 1) - E0;
+    constexpr uint32_t SIGN = 0x80000000u;
+    float t[D], a[D];
+    uint32_t off[D];
+    uint32_t mags = 0x7FFFFFFFu;
+    asm("" : "+s"(mags));
+    static_for<D>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        off[j] = edge_off<BG, E0 + j, float, LM, PK, SPL>(sh, zb, zp, Zb, Pb);
+        t[j] = lds_ld<float>(base, off[j]) - st[S0 + j];
+        a[j] = u2f(f2u(t[j]) & mags);
+    });
+    float m1 = fmin2(a[0], a[1]), m2 = fmax2(a[0], a[1]);
+    uint32_t par = f2u(t[0]) ^ f2u(t[1]);
+    static_for<D>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        if constexpr (j >= 2) {
+            m2 = fmin2(m2, fmax2(m1, a[j]));
+            m1 = fmin2(m1, a[j]);
+            par ^= f2u(t[j]);
+        }
+    });
+    const uint32_t S = f2u(m1) + f2u(m2);
+    const uint32_t Q = f2u(alpha) ^ (par & SIGN);
+    static_for<D>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        const float other = u2f(S - f2u(fmin2(a[j], m2)));
+        // Q ^ (t & SIGN) as one three-input bitwise instruction (table 0x6C: B ^ (A & C))
+        const float c = other * u2f(__builtin_amdgcn_bitop3_b32(f2u(t[j]), Q, SIGN, (unsigned char)0x6C));
+        lds_st<float>(base, off[j], t[j] + c);
+        st[S0 + j] = c;
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -571,22 +670,25 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
     const uint32_t tid = threadIdx.x;
     const T alpha = job_alpha<T>(job);
 
-    // C2V state: compressed per row (binary32) or explicit per edge (binary16)
-    constexpr int NRS = (PAIR == 2) ? (PP.rows[0] > PP.rows[1] ? PP.rows[0] : PP.rows[1]) : NR;
+    // C2V state: per row or per edge (binary32, f32_plan), per edge (binary16)
     // binary16 message slots: every row padded to an even number of edges
     constexpr int NEDGE = (PAIR == 2) ? (PP.padded_edges[0] > PP.padded_edges[1] ? PP.padded_edges[0]
                                                                                   : PP.padded_edges[1])
                                       : padded_row_start<BG>(NR);
     constexpr int NW = NEDGE / 2;
-    float st_n1[std::is_same<T, float>::value ? NRS : 1], st_n2[std::is_same<T, float>::value ? NRS : 1];
-    uint32_t st_meta[std::is_same<T, float>::value ? NRS : 1];
-    half2_t st_h[std::is_same<T, float>::value ? 1 : NW];
-    if constexpr (std::is_same<T, float>::value) {
+    constexpr bool F32 = std::is_same<T, float>::value;
+    constexpr f32_plan<BG, NR, PAIR> FP = kF32Plan<BG, NR, PAIR>;
+    constexpr int NRS = F32 && FP.rows > 0 ? FP.rows : 1, NM = F32 && FP.messages > 0 ? FP.messages : 1;
+    float st_n1[NRS], st_n2[NRS], st_f[NM];
+    uint32_t st_meta[NRS];
+    half2_t st_h[F32 ? 1 : NW];
+    if constexpr (F32) {
         static_for<NRS>([&](auto R) {
             st_n1[R] = 0.0f;
             st_n2[R] = 0.0f;
             st_meta[R] = 0;
         });
+        static_for<NM>([&](auto M) { st_f[M] = 0.0f; });
     } else {
         static_for<NW>([&](auto W) { st_h[W] = half2_t{(_Float16)0, (_Float16)0}; });
     }
@@ -648,12 +750,13 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
                 uint32_t Zr = Zb;
                 asm volatile("" : "+s"(shr), "+s"(Zr));
                 if (active && (PAIR == 1 || lgrp == (uint32_t)PP.group[R])) {
-                    constexpr int RS = (PAIR == 2) ? PP.row_slot[R] : R;
                     constexpr int S0 = (PAIR == 2) ? PP.pair_slot[R] : padded_row_start<BG>(R);
-                    if constexpr (std::is_same<T, float>::value)
-                        process_row<BG, R, NRS, RS, LM, decltype(lane_base), PK, SPL>(app, lane_base, shr, zb, zp, Zr,
-                                                                                      alpha, st_n1, st_n2, st_meta,
-                                                                                      Pb);
+                    if constexpr (F32 && FP.is_explicit[R])
+                        process_row_explicit<BG, R, NM, FP.slot[R], LM, decltype(lane_base), PK, SPL>(
+                            lane_base, shr, zb, zp, Zr, alpha, st_f, Pb);
+                    else if constexpr (F32)
+                        process_row<BG, R, NRS, FP.slot[R], LM, decltype(lane_base), PK, SPL>(
+                            app, lane_base, shr, zb, zp, Zr, alpha, st_n1, st_n2, st_meta, Pb);
                     else
                         process_row<BG, R, NW, S0, LM, decltype(lane_base), PK, SPL>(app, lane_base, shr, zb, zp, Zr,
                                                                                      alpha, st_h, Pb);
