@@ -360,7 +360,7 @@ cuphyStatus_t CUPHYWINAPI cuphyErrorCorrectionLDPCDecode(cuphyLDPCDecoder_t deco
     } else {
         d.config.flags &= ~(uint32_t)CUPHY_LDPC_DECODE_WRITE_SOFT_OUTPUTS;
     }
-    return nrldpc::decode_tb(d, strm);
+    return nrldpc::decode_tb(d, decoder->cu_count, strm);
 }
 
 cuphyStatus_t CUPHYWINAPI cuphyErrorCorrectionLDPCTransportBlockDecode(cuphyLDPCDecoder_t decoder,
@@ -381,7 +381,7 @@ cuphyStatus_t CUPHYWINAPI cuphyErrorCorrectionLDPCTransportBlockDecode(cuphyLDPC
             return CUPHY_STATUS_INVALID_ARGUMENT;
     if (decodeDesc->num_tbs == 0) return CUPHY_STATUS_SUCCESS;
     if (!nrldpc::config_supported(c)) return CUPHY_STATUS_UNSUPPORTED_CONFIG;
-    return nrldpc::decode_tb(*decodeDesc, strm);
+    return nrldpc::decode_tb(*decodeDesc, decoder->cu_count, strm);
 }
 
 // ---------------------------------------------------------------------------

@@ -97,8 +97,8 @@ template <int BG> constexpr uint64_t kBarrierMask = barrier_mask<bg_traits<BG>>(
 // alternate between the groups, and a segment's first row goes to the
 // group holding fewer edges so far (the per-lane message state is then
 // about half the graph's).  Within its group a row's binary16 messages take
-// consecutive slots from pair_slot[r] (rows padded to even degree) and its
-// compressed binary32 row state the slot row_slot[r].  Rows r < NR only.
+// consecutive slots from pair_slot[r] (rows padded to even degree).  Rows
+// r < NR only.
 template <int BG, int NR> struct pair_plan {
     int group[64];
     int pair_slot[64];  // binary16: first message slot of the row (even; rows padded to even degree)
@@ -164,6 +164,26 @@ template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> make_f32_pl
     return p;
 }
 template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> kF32Plan = make_f32_plan<BG, NR, PAIR>();
+
+// Slots of the offsets of run_iterations' PRE form: the edges that need a
+// rotation, counted per lane group.
+template <int BG, int NR, int PAIR> struct offset_plan {
+    int slot[320];
+    int count;
+};
+template <int BG, int NR, int PAIR> constexpr offset_plan<BG, NR, PAIR> make_offset_plan()
+{
+    using BGT = bg_traits<BG>;
+    offset_plan<BG, NR, PAIR> p{};
+    const pair_plan<BG, NR> pp = make_pair_plan<BG, NR>();
+    int n[2] = {0, 0};
+    for (int r = 0; r < NR; ++r)
+        for (int e = BGT::row_start(r); e < BGT::row_start(r + 1); ++e)
+            if (!BGT::identity_edge(e)) p.slot[e] = n[PAIR == 2 ? pp.group[r] : 0]++;
+    p.count = n[0] > n[1] ? n[0] : n[1];
+    return p;
+}
+template <int BG, int NR, int PAIR> constexpr offset_plan<BG, NR, PAIR> kOffsetPlan = make_offset_plan<BG, NR, PAIR>();
 
 // binary16 message slots: row r's edges from padded_row_start(r) on, every
 // row's degree rounded up to even, so that each pair of a row's edges is one
@@ -306,12 +326,11 @@ __device__ __forceinline__ uint32_t edge_off(shift_ptr sh, uint32_t zb, uint32_t
 // (edge j at bit D-1-j).  Per edge: address 3, previous-message rebuild 4,
 // subtract 1, min/min2/parity 3, new message + write-back 6 VALU ops.
 // ---------------------------------------------------------------------------
-// RS: the row's state slot (R, or its slot within a row-pair lane group).
-template <int BG, int R, int NR, int RS = R, bool LM = false, typename BP = unsigned char*, bool PK = false,
-          bool SPL = false>
-__device__ __forceinline__ void process_row(float*, BP __restrict__ base, shift_ptr sh, uint32_t zb,
-                                            uint32_t zp, uint32_t Zb, float alpha, float (&st_n1)[NR], float (&st_n2)[NR],
-                                            uint32_t (&st_meta)[NR], uint32_t Pb = 0)
+// RS: the row's state slot (f32_plan).  off_of(j): byte offset of edge j's APP
+// value.
+template <int BG, int R, int NR, int RS, typename BP, typename Off>
+__device__ __forceinline__ void process_row(float*, BP __restrict__ base, const Off& off_of, float alpha,
+                                            float (&st_n1)[NR], float (&st_n2)[NR], uint32_t (&st_meta)[NR])
 {
     using BGT = bg_traits<BG>;
     constexpr int E0 = BGT::row_start(R);
@@ -323,7 +342,7 @@ __device__ __forceinline__ void process_row(float*, BP __restrict__ base, shift_
     const uint32_t oidx = om >> 27;
     static_for<D>([&](auto J) {
         constexpr int j = decltype(J)::value;
-        off[j] = edge_off<BG, E0 + j, float, LM, PK, SPL>(sh, zb, zp, Zb, Pb);
+        off[j] = off_of(J);
         const float mag = (oidx == (uint32_t)j) ? on2 : on1;
         const float old = u2f(f2u(mag) | ((om << (32 - D + j)) & 0x80000000u));
         t[j] = lds_ld<float>(base, off[j]) - old;
@@ -379,9 +398,9 @@ __device__ __forceinline__ float fmax2(float a, float b)
     asm("v_max_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-template <int BG, int R, int NM, int S0, bool LM, typename BP, bool PK, bool SPL>
-__device__ __forceinline__ void process_row_explicit(BP __restrict__ base, shift_ptr sh, uint32_t zb, uint32_t zp,
-                                                     uint32_t Zb, float alpha, float (&st)[NM], uint32_t Pb)
+template <int BG, int R, int NM, int S0, typename BP, typename Off>
+__device__ __forceinline__ void process_row_explicit(BP __restrict__ base, const Off& off_of, float alpha,
+                                                     float (&st)[NM])
 {
     using BGT = bg_traits<BG>;
     constexpr int E0 = BGT::row_start(R);
@@ -393,7 +412,7 @@ __device__ __forceinline__ void process_row_explicit(BP __restrict__ base, shift
     asm("" : "+s"(mags));
     static_for<D>([&](auto J) {
         constexpr int j = decltype(J)::value;
-        off[j] = edge_off<BG, E0 + j, float, LM, PK, SPL>(sh, zb, zp, Zb, Pb);
+        off[j] = off_of(J);
         t[j] = lds_ld<float>(base, off[j]) - st[S0 + j];
         a[j] = u2f(f2u(t[j]) & mags);
     });
@@ -472,10 +491,9 @@ __device__ __forceinline__ half2_t sub_pair(uint32_t v0, uint32_t v1, half2_t m)
 
 // S0: message slot of the row's first edge (even: padded_row_start(R), or
 // the row's pair_slot within a row-pair lane group).
-template <int BG, int R, int NW, int S0 = padded_row_start<BG>(R), bool LM = false, typename BP = unsigned char*,
-          bool PK = false, bool SPL = false>
-__device__ __forceinline__ void process_row(_Float16*, BP __restrict__ base, shift_ptr sh, uint32_t zb,
-                                            uint32_t zp, uint32_t Zb, _Float16 alpha, half2_t (&st)[NW], uint32_t Pb = 0)
+template <int BG, int R, int NW, int S0, typename BP, typename Off>
+__device__ __forceinline__ void process_row(_Float16*, BP __restrict__ base, const Off& off_of, _Float16 alpha,
+                                            half2_t (&st)[NW])
 {
     using BGT = bg_traits<BG>;
     constexpr int E0 = BGT::row_start(R);
@@ -494,10 +512,10 @@ __device__ __forceinline__ void process_row(_Float16*, BP __restrict__ base, shi
     static_for<P>([&](auto K) {
         constexpr int k = decltype(K)::value;
         constexpr int j0 = 2 * k, j1 = 2 * k + 1;
-        off[j0] = edge_off<BG, E0 + j0, _Float16, LM, PK, SPL>(sh, zb, zp, Zb, Pb);
+        off[j0] = off_of(std::integral_constant<int, j0>{});
         const uint32_t v0 = lds_ld<uint16_t>(base, off[j0]);
         if constexpr (j1 < D) {
-            off[j1] = edge_off<BG, E0 + j1, _Float16, LM, PK, SPL>(sh, zb, zp, Zb, Pb);
+            off[j1] = off_of(std::integral_constant<int, j1>{});
             const uint32_t v1 = lds_ld<uint16_t>(base, off[j1]);
             if constexpr (SDWA_PAIR)
                 t[k] = sub_pair(v0, v1, st[W0 + k]);
@@ -658,7 +676,12 @@ template <> __device__ __forceinline__ _Float16 job_alpha<_Float16>(const cb_job
 // and each lane holds the message state of its group's rows only.
 // LM: lane-major APP values from LDS address 0 (lm_pitch_bytes; count must
 // be 1, cb_flags two LDS words for the early-termination votes).
-template <int BG, typename T, int MAXR, int PAIR = 1, bool LM = (PAIR == 2)>
+// PRE (lane-major only): every edge's rotated lane offset in a register,
+// computed once.  A row then starts with its LDS reads instead of scalar
+// loads of its shifts, a multiplication and two vector operations per edge --
+// for launches of few small code blocks, whose time is the latency of one
+// row after another (a wave per SIMD has the registers).
+template <int BG, typename T, int MAXR, int PAIR = 1, bool LM = (PAIR == 2), bool PRE = false>
 __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job& job, int count = 1, int stride = 0,
                                               uint32_t* cb_flags = nullptr, uint32_t* cb_iters = nullptr)
 {
@@ -728,6 +751,28 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
     constexpr bool PK = !LM || sizeof(T) == 2;
 
     shift_ptr sh = (shift_ptr)(const void*)&g_shift_tables.v[BG - 1][z_index((int)Z)][0];
+    static_assert(!PRE || LM, "offsets in registers: lane-major layout");
+    constexpr offset_plan<BG, NR, PAIR> pre_plan = kOffsetPlan<BG, NR, PAIR>;
+    uint32_t pre[PRE ? pre_plan.count : 1];
+    if constexpr (PRE) {
+        const uint32_t zp = zlane * Pb, zb = PK ? lane_rot_base(zp, Zb) : zp;
+        static_for<pre_plan.count>([&](auto I) { pre[I] = 0u; });
+        static_for<NR>([&](auto Rc) {
+            constexpr int R = decltype(Rc)::value;
+            if (R < mb && (PAIR == 1 || lgrp == (uint32_t)PP.group[R]))
+                static_for<BGT::row_start(R + 1) - BGT::row_start(R)>([&](auto J) {
+                    constexpr int E = BGT::row_start(R) + decltype(J)::value;
+                    if constexpr (!BGT::identity_edge(E))
+                        pre[pre_plan.slot[E]] = edge_off<BG, E, T, LM, PK, SPL>(sh, zb, zp, Zb, Pb) -
+                                                lm_col_offset(BG, BGT::col(E), (int)sizeof(T), SPL);
+                });
+        });
+        static_for<pre_plan.count>([&](auto I) {  // (opaque: not recomputed in the loop)
+            uint32_t v = pre[I];
+            asm volatile("" : "+v"(v));
+            pre[I] = v;
+        });
+    }
     int it = 0;
     while (it < job.max_iter) {
         ++it;
@@ -751,15 +796,19 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
                 asm volatile("" : "+s"(shr), "+s"(Zr));
                 if (active && (PAIR == 1 || lgrp == (uint32_t)PP.group[R])) {
                     constexpr int S0 = (PAIR == 2) ? PP.pair_slot[R] : padded_row_start<BG>(R);
+                    const auto off_of = [&](auto J) -> uint32_t {
+                        constexpr int E = BGT::row_start(R) + decltype(J)::value;
+                        if constexpr (PRE && !BGT::identity_edge(E))
+                            return pre[pre_plan.slot[E]] + lm_col_offset(BG, BGT::col(E), (int)sizeof(T), SPL);
+                        else
+                            return edge_off<BG, E, T, LM, PK, SPL>(shr, zb, zp, Zr, Pb);
+                    };
                     if constexpr (F32 && FP.is_explicit[R])
-                        process_row_explicit<BG, R, NM, FP.slot[R], LM, decltype(lane_base), PK, SPL>(
-                            lane_base, shr, zb, zp, Zr, alpha, st_f, Pb);
+                        process_row_explicit<BG, R, NM, FP.slot[R]>(lane_base, off_of, alpha, st_f);
                     else if constexpr (F32)
-                        process_row<BG, R, NRS, FP.slot[R], LM, decltype(lane_base), PK, SPL>(
-                            app, lane_base, shr, zb, zp, Zr, alpha, st_n1, st_n2, st_meta, Pb);
+                        process_row<BG, R, NRS, FP.slot[R]>(app, lane_base, off_of, alpha, st_n1, st_n2, st_meta);
                     else
-                        process_row<BG, R, NW, S0, LM, decltype(lane_base), PK, SPL>(app, lane_base, shr, zb, zp, Zr,
-                                                                                     alpha, st_h, Pb);
+                        process_row<BG, R, NW, S0>(app, lane_base, off_of, alpha, st_h);
                 }
                 // barrier before the next row only where it shares a column
                 // with the rows since the last barrier, and at the iteration end
@@ -909,7 +958,7 @@ __device__ __forceinline__ int decode_group(T* __restrict__ app, const cb_job& j
 // at z * pitch + column * sizeof(T).  PAIR = 2: row-pair mode (blockDim.x >=
 // 2 * roundup64(Z)); PAIR = 1: one lane group (blockDim.x >= Z).  flag: one
 // LDS word outside the values (the early-termination vote).
-template <int BG, typename T, typename TIn, int MAXR, int PAIR>
+template <int BG, typename T, typename TIn, int MAXR, int PAIR, bool PRE = false>
 __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job, const cb_buffers& b, uint32_t* flag)
 {
     const int Z = job.Z;
@@ -948,7 +997,7 @@ __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job,
         }
         __syncthreads();
     }
-    const int iters = run_iterations<BG, T, MAXR, PAIR, true>(app, job, 1, 0, flag);
+    const int iters = run_iterations<BG, T, MAXR, PAIR, true, PRE>(app, job, 1, 0, flag);
     const int nbits = job.Kb * Z;
     // hard decisions, 64 per wave per step by ballot (as store_hard); each
     // lane walks its (column, z) position instead of dividing per bit

@@ -62,8 +62,8 @@ __global__ __launch_bounds__(384) void ldpc_layered_tb(cuphyLDPCDecodeDesc_t des
 // workgroup, Z > 32, mb > 8): workgroup b decodes code word b with two lane
 // groups of roundup64(Z) lanes that take the column-disjoint block rows of
 // each barrier segment at the same time (run_iterations PAIR = 2).
-template <int BG, typename T, typename TIn>
-__global__ __launch_bounds__(768) void ldpc_layered_tb_pair(cuphyLDPCDecodeDesc_t desc)
+template <int BG, typename T, typename TIn, bool PRE>
+__device__ __forceinline__ void tb_pair(const cuphyLDPCDecodeDesc_t& desc)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const cb_job job = tb_job<TIn>(desc);
@@ -71,7 +71,31 @@ __global__ __launch_bounds__(768) void ldpc_layered_tb_pair(cuphyLDPCDecodeDesc_
     uint32_t* flag = reinterpret_cast<uint32_t*>(
         lds_raw + lm_app_bytes(BG, job.Z, bg_traits<BG>::NSYS + job.mb, (int)sizeof(T),
                                lm_split_layout((int)sizeof(T), 46)));
-    decode_lm<BG, T, TIn, 46, 2>(reinterpret_cast<T*>(lds_raw), job, tb_buffers<TIn>(desc, (int)blockIdx.x), flag);
+    decode_lm<BG, T, TIn, 46, 2, PRE>(reinterpret_cast<T*>(lds_raw), job, tb_buffers<TIn>(desc, (int)blockIdx.x), flag);
+}
+template <int BG, typename T, typename TIn>
+__global__ __launch_bounds__(768) void ldpc_layered_tb_pair(cuphyLDPCDecodeDesc_t desc)
+{
+    tb_pair<BG, T, TIn, false>(desc);
+}
+
+// The same with every edge's offset in a register (run_iterations PRE), for
+// workgroups whose waves have the registers for it: BG2 in binary16 holds 153,
+// three waves per SIMD; BG1 in binary16 254 and BG2 in binary32 207, two; BG1 in
+// binary32 278, one.  Used when every code block has a CU to itself; with more
+// code blocks the plain form's waves that share a CU hide each other's
+// latency.  Measured for 10 iterations, plain and this form: one code block BG2
+// Z = 64, 20 rows 53 and 48 us; eight BG1 Z = 128, 46 rows 119 and 107 us, in
+// binary32 151 (before explicit messages) and 135 us; eight BG2 Z = 384, 42 rows
+// 111 and 99 us; 256 BG1 Z = 128, 46 rows 122 and 110 us.
+template <int BG, typename T> constexpr int tb_pre_threads()
+{
+    return sizeof(T) == 2 ? (BG == 2 ? 768 : 512) : (BG == 2 ? 512 : 256);
+}
+template <int BG, typename T, typename TIn>
+__global__ __launch_bounds__((tb_pre_threads<BG, T>())) void ldpc_layered_tb_pair_pre(cuphyLDPCDecodeDesc_t desc)
+{
+    tb_pair<BG, T, TIn, true>(desc);
 }
 
 // Persistent heterogeneous decoder: each workgroup repeatedly takes the
@@ -153,13 +177,6 @@ __global__ __launch_bounds__(384) void ldpc_layered_persistent(cuphyHipLDPCWorkI
     }
 }
 
-// Row-pair persistent kernel (768 threads): every code block of the queue
-// decoded alone by two lane groups that take the independent block rows of
-// each barrier segment at the same time (run_iterations PAIR = 2), with 12
-// waves on the CU's 4 SIMDs.  For batches with fewer code blocks than CUs,
-// where the slot time is the slowest code block's decode time.  Same queue
-// protocol as ldpc_layered_persistent; a group's code blocks are decoded
-// one after another.
 // Body of the lane-major persistent kernels (PAIR = 2: row-pair, 768
 // threads; PAIR = 1: one lane group, one code block per workgroup of at
 // least roundup64(Z) threads).  No static LDS: the APP values start at LDS
@@ -277,18 +294,25 @@ void* select_tb_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math)
     return nullptr;
 }
 
-void* select_tb_pair_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math)
+// Row-pair kernel of a launch of `threads`-thread workgroups; own_cu: no more
+// workgroups than CUs.
+template <int BG, typename T, typename TIn> void* tb_pair_kernel(int threads, bool own_cu)
 {
-    if (bg == 1) {
-        if (llr_type == CUPHY_R_32F)
-            return fp16_math ? (void*)&ldpc_layered_tb_pair<1, _Float16, float> : (void*)&ldpc_layered_tb_pair<1, float, float>;
-        if (llr_type == CUPHY_R_16F) return (void*)&ldpc_layered_tb_pair<1, _Float16, _Float16>;
-    } else if (bg == 2) {
-        if (llr_type == CUPHY_R_32F)
-            return fp16_math ? (void*)&ldpc_layered_tb_pair<2, _Float16, float> : (void*)&ldpc_layered_tb_pair<2, float, float>;
-        if (llr_type == CUPHY_R_16F) return (void*)&ldpc_layered_tb_pair<2, _Float16, _Float16>;
-    }
-    return nullptr;
+    return own_cu && threads <= tb_pre_threads<BG, T>() ? (void*)&ldpc_layered_tb_pair_pre<BG, T, TIn>
+                                                        : (void*)&ldpc_layered_tb_pair<BG, T, TIn>;
+}
+template <int BG> void* tb_pair_kernel_of(cuphyDataType_t llr_type, bool fp16_math, int threads, bool own_cu)
+{
+    if (llr_type == CUPHY_R_32F)
+        return fp16_math ? tb_pair_kernel<BG, _Float16, float>(threads, own_cu)
+                         : tb_pair_kernel<BG, float, float>(threads, own_cu);
+    return llr_type == CUPHY_R_16F ? tb_pair_kernel<BG, _Float16, _Float16>(threads, own_cu) : nullptr;
+}
+void* select_tb_pair_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math, int threads, bool own_cu)
+{
+    return bg == 1   ? tb_pair_kernel_of<1>(llr_type, fp16_math, threads, own_cu)
+           : bg == 2 ? tb_pair_kernel_of<2>(llr_type, fp16_math, threads, own_cu)
+                     : nullptr;
 }
 
 void* select_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math, int mb)
@@ -338,7 +362,7 @@ static bool use_fp16_math(const cuphyLDPCDecodeConfigDesc_t& c)
 
 cuphyStatus_t check_lm_kernel(void* func);
 
-cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, launch_geometry& g)
+cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, int cu_count, launch_geometry& g)
 {
     const cuphyLDPCDecodeConfigDesc_t& c = desc.config;
     if (!config_supported(c)) return CUPHY_STATUS_UNSUPPORTED_CONFIG;
@@ -349,7 +373,10 @@ cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, launch_geometry& g)
     // form (two lane groups; the 46-row variant holds one 6-wave workgroup
     // per CU anyway, the row-pair one 12 waves)
     const bool pair = P == 1 && c.num_parity_nodes > SMALL_MAXR;
-    g.func = pair ? select_tb_pair_kernel(c.BG, c.llr_type, fp16) : select_kernel(c.BG, c.llr_type, fp16, c.num_parity_nodes);
+    g.block = pair ? dim3((unsigned)(2 * ((c.Z + 63) / 64 * 64))) : dim3((unsigned)((P * c.Z + 63) / 64 * 64));
+    g.grid = dim3((unsigned)((desc_codewords(desc) + P - 1) / P));
+    g.func = pair ? select_tb_pair_kernel(c.BG, c.llr_type, fp16, (int)g.block.x, (int)g.grid.x <= cu_count)
+                  : select_kernel(c.BG, c.llr_type, fp16, c.num_parity_nodes);
     if (!g.func) return CUPHY_STATUS_UNSUPPORTED_CONFIG;
     if (pair) {
         const cuphyStatus_t s = check_lm_kernel(g.func);
@@ -361,8 +388,6 @@ cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, launch_geometry& g)
     g.lds_bytes = pair ? (size_t)lm_app_bytes(c.BG, c.Z, nsys + c.num_parity_nodes, fp16 ? 2 : 4,
                                               lm_split_layout(fp16 ? 2 : 4, 46)) + 16u
                        : (size_t)P * stride * (fp16 ? 2u : 4u);
-    g.block = pair ? dim3((unsigned)(2 * ((c.Z + 63) / 64 * 64))) : dim3((unsigned)((P * c.Z + 63) / 64 * 64));
-    g.grid = dim3((unsigned)((desc_codewords(desc) + P - 1) / P));
     return CUPHY_STATUS_SUCCESS;
 }
 
@@ -402,10 +427,10 @@ cuphyStatus_t check_lm_kernel(void* func)
     return CUPHY_STATUS_SUCCESS;
 }
 
-cuphyStatus_t decode_tb(const cuphyLDPCDecodeDesc_t& desc, hipStream_t strm)
+cuphyStatus_t decode_tb(const cuphyLDPCDecodeDesc_t& desc, int cu_count, hipStream_t strm)
 {
     launch_geometry g;
-    cuphyStatus_t s = fill_launch(desc, g);
+    cuphyStatus_t s = fill_launch(desc, cu_count, g);
     if (s != CUPHY_STATUS_SUCCESS) return s;
     if (g.grid.x == 0) return CUPHY_STATUS_SUCCESS;
     if ((s = ensure_lds_attr(g.func, g.lds_bytes)) != CUPHY_STATUS_SUCCESS) return s;
@@ -462,7 +487,11 @@ cuphyStatus_t decode_batch(cuphyHipLDPCWorkItem_t* d_items, const uint32_t* d_gr
 cuphyStatus_t get_launch_config(cuphyLDPCDecodeLaunchConfig_t& lc)
 {
     launch_geometry g;
-    cuphyStatus_t s = fill_launch(lc.decode_desc, g);
+    // cu_count 0: the plain row-pair kernel.  hipGraphExecKernelNodeSetParams
+    // refuses a workgroup larger than the launch bounds of the function that the
+    // node holds at that moment, so a node may only hold functions that take
+    // every later size.
+    cuphyStatus_t s = fill_launch(lc.decode_desc, 0, g);
     if (s != CUPHY_STATUS_SUCCESS) return s;
     if ((s = ensure_lds_attr(g.func, g.lds_bytes)) != CUPHY_STATUS_SUCCESS) return s;
     lc.kernel_args[0] = &lc.decode_desc;

@@ -19,15 +19,16 @@ bool is_lifting_size(int Z);
 // (BG, Z, mb, Kb, LLR type) is decodable by the kernels of this library.
 bool config_supported(const cuphyLDPCDecodeConfigDesc_t& c);
 
-// Kernel and launch shape for a transport-block descriptor.
-cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, launch_geometry& g);
+// Kernel and launch shape for a transport-block descriptor on a GPU of
+// cu_count CUs (0: the kernels whose launch bounds take every block size).
+cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, int cu_count, launch_geometry& g);
 
 // Raise a kernel's dynamic-LDS limit above the 64 KB default, once per
 // (kernel, size) high-water mark.
 cuphyStatus_t ensure_lds_attr(void* func, size_t bytes);
 
 // Enqueue the decode of every code word of `desc` on `strm`.
-cuphyStatus_t decode_tb(const cuphyLDPCDecodeDesc_t& desc, hipStream_t strm);
+cuphyStatus_t decode_tb(const cuphyLDPCDecodeDesc_t& desc, int cu_count, hipStream_t strm);
 
 // Populate a kernel-node launch configuration (graph capture / driver launch).
 cuphyStatus_t get_launch_config(cuphyLDPCDecodeLaunchConfig_t& lc);

@@ -201,6 +201,32 @@ def test_early_termination_fp16_large_z(dec):
     assert_soft_equal(s_gpu, s_ref)
 
 
+# Row-pair transport blocks hold the offsets of their edges in registers where
+# every code block has a CU to itself and the workgroup's waves have the
+# registers; one code block more than CUs takes the plain form.
+OWN_CU = [(1, 36, 9), (1, 128, 46), (1, 144, 46), (1, 256, 46), (1, 256, 10), (1, 288, 20), (2, 36, 42), (2, 64, 9),
+          (2, 256, 42), (2, 288, 42), (2, 384, 42), (2, 384, 20)]
+
+
+@pytest.mark.parametrize("bg,Z,mb", OWN_CU)
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "fp32in_fp16math"])
+@pytest.mark.parametrize("et", [False, True])
+def test_code_blocks_up_to_and_above_the_cus(dec, bg, Z, mb, dtype, et):
+    from aerial_amd import _lib as L
+    _log("own CU: BG%d Z=%d mb=%d %s et=%d seed=23" % (bg, Z, mb, dtype, et))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    llr, _ = V.make_cbs(bg, Z, mb, 2, seed=23, snr_db=5.0 if et else 1.0)
+    if dtype == "fp16":
+        llr = V.to_half_rn(llr).astype(np.float32)
+    flags = L.CUPHY_LDPC_DECODE_EARLY_TERM if et else 0
+    h_ref, s_ref, _ = run_oracle(bg, Z, mb, llr, n_iter=5, et=et, mode=O.FP32 if dtype == "fp32" else O.FP16)
+    for n in (1, cus, cus + 1):
+        idx = np.arange(n) % 2
+        h, s = run_gpu(dec, bg, Z, mb, llr[idx], n_iter=5, dtype=dtype, flags=flags)
+        assert np.array_equal(h, h_ref[idx])
+        assert_soft_equal(s, s_ref[idx])
+
+
 def test_multi_tb_descriptor(dec):
     from aerial_amd import _lib as L
     from aerial_amd.decoder import LdpcDecodeConfig
