@@ -669,8 +669,8 @@ template <> __device__ __forceinline__ _Float16 job_alpha<_Float16>(const cb_job
 // syndrome (its lanes freeze, exactly as if decoded alone); `cb_flags` is
 // LDS scratch of `count` words for that (unused when count == 1).
 // cb_iters (optional, LDS, `count` words): iterations each code block ran.
-// PAIR = 2: row-pair mode for one code block (count must be 1, blockDim.x
-// >= 2 * roundup64(Z)): lanes [0, Z) and [Zw, Zw + Z) (Zw = roundup64(Z),
+// PAIR = 2: row-pair mode (blockDim.x >= 2 * roundup64(count * Z)): lanes
+// [0, count * Z) and [Zw, Zw + count * Z) (Zw = roundup64(count * Z),
 // wave-aligned) form two lane groups that process the rows of kPairPlan's
 // group 0 and group 1; rows of one barrier segment run at the same time,
 // and each lane holds the message state of its group's rows only.
@@ -719,13 +719,14 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
     // lane -> (code block, check row); row-pair mode: lane -> (lane group, check row)
     uint32_t cb, zlane, lgrp = 0;
     bool in_group;
+    if constexpr (LM) count = 1;
     if constexpr (PAIR == 2) {
-        const uint32_t Zw = (Z + 63u) & ~63u;
+        const uint32_t Zw = ((uint32_t)count * Z + 63u) & ~63u;
         lgrp = tid >= Zw ? 1u : 0u;
         zlane = tid - lgrp * Zw;
-        cb = 0;
-        in_group = zlane < Z && tid < 2u * Zw;
-        count = 1;
+        in_group = zlane < (uint32_t)count * Z && tid < 2u * Zw;
+        cb = (count == 1) ? 0u : zlane / Z;
+        zlane -= (in_group ? cb : 0u) * Z;
     } else {
         cb = (count == 1) ? (tid < Z ? 0u : 1u) : tid / Z;
         zlane = tid - (cb < (uint32_t)count ? cb : 0u) * Z;

@@ -515,7 +515,7 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
 // the error marker is written, into the CBs' CRCs).  The TB CRC itself is
 // written by complete_cb.  GROUPED = false: the one-CB form (count = 1 at
 // compile time, no group state; an item of several CBs is rejected).
-template <typename TI, int MAXR, bool GROUPED>
+template <typename TI, int MAXR, bool GROUPED, int PAIR>
 __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused_lds& sh,
                                                 const cuphyHipPuschSlotTb_t& job, const PerTbParams& p, int cb0,
                                                 int count_in, int lds_values, uint32_t* __restrict__ tbw,
@@ -548,7 +548,7 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     }
     const bool ok = (bg == 1 || bg == 2) && z_index(Zc) >= 0 && mb >= 4 && mb <= (bg == 1 ? 46 : 42) &&
                     mb <= MAXR && count == count_in && count >= 1 && count <= FUSED_MAX_GROUP &&
-                    count * Zc <= (int)blockDim.x &&
+                    count * Zc <= FUSED_BLOCK &&
                     (count - 1) * S + arr <= lds_values && Kb * Zc <= 32 * (int)SLOT_CB_WORDS &&
                     count * ((Kb * Zc + 31) >> 5) <= (int)(sizeof(sh.words) / sizeof(sh.words[0])) && e_ok &&
                     (!descr || seq_at + 2 * (nw_max + 1) <= lds_values);
@@ -586,8 +586,8 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     dj.alpha_f16 = (uint16_t)(job.norm.f16x2 & 0xFFFFu);
     uint32_t* const flags = (count > 1) ? sh.cb_flags : nullptr;
     uint32_t* const cb_it = (count > 1) ? sh.cb_iters : nullptr;
-    const int iters = (bg == 1) ? run_iterations<1, _Float16, MAXR>(hb, dj, count, S, flags, cb_it)
-                                : run_iterations<2, _Float16, MAXR>(hb, dj, count, S, flags, cb_it);
+    const int iters = (bg == 1) ? run_iterations<1, _Float16, MAXR, PAIR, false>(hb, dj, count, S, flags, cb_it)
+                                : run_iterations<2, _Float16, MAXR, PAIR, false>(hb, dj, count, S, flags, cb_it);
 
     // ---- 5. hard decisions of all CBs into LDS and memory --------------------
     const int tt = opaque_tid();
@@ -686,6 +686,13 @@ __device__ __forceinline__ void complete_cb(const cuphyHipPuschSlotTb_t& job, ui
         *job.tb_crc = tb_crc;
 }
 
+// Threads of a workgroup.  With all rows, whose registers leave one workgroup
+// per CU, two lane groups of FUSED_BLOCK (run_iterations PAIR = 2; 168 VGPRs, no
+// spills): every phase has twice the waves and the rows of a barrier segment run
+// side by side.  One group against two: 64 descrambled UEs with a retransmission
+// 429 -> 411 us, a served burst of 384 TBs 1083 -> 1041 us.
+constexpr int fused_threads(int maxr) { return maxr <= MID_MAXR ? FUSED_BLOCK : 2 * FUSED_BLOCK; }
+
 // Persistent fused slot kernel.  Workspace: queue state (2 words used of
 // FUSED_WS_QUEUE_WORDS), then two words per CB slot of the launch, of which
 // each TB uses the pair at its first slot (TB-CRC accumulator and count of
@@ -698,7 +705,7 @@ __device__ __forceinline__ void complete_cb(const cuphyHipPuschSlotTb_t& job, ui
 // high-rate variant ran one workgroup per CU.  (The middle variant's BG1
 // rows beyond 8 spill a few registers; BG2 rows, half as long, do not.)
 template <typename TI, int MAXR, bool GROUPED>
-__global__ __launch_bounds__(384) __attribute__((amdgpu_waves_per_eu(MAXR <= MID_MAXR ? 4 : 1)))
+__global__ __launch_bounds__(fused_threads(MAXR)) __attribute__((amdgpu_waves_per_eu(MAXR <= MID_MAXR ? 4 : 1)))
 void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
                                                         const uint32_t* __restrict__ items, int n_items,
                                                         int lds_values, uint32_t* __restrict__ ws)
@@ -709,6 +716,7 @@ void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
     uint32_t* queue = ws;
     uint32_t* tbw = ws + FUSED_WS_QUEUE_WORDS;
     load_crc_steps(sh);
+    constexpr int PAIR = MAXR <= MID_MAXR ? 1 : 2;
     if (threadIdx.x == 0) sh.item = (int)atomicAdd(&queue[0], 1u);
     __syncthreads();
     for (;;) {
@@ -723,7 +731,7 @@ void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
             const uint32_t C = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.num_CBs);
             if ((uint32_t)(cb + n) <= C) {
                 uint32_t xprev = 0;
-                const uint32_t part = fused_group<TI, MAXR, GROUPED>(hb, sh, job, p, cb, n, lds_values, tbw, xprev);
+                const uint32_t part = fused_group<TI, MAXR, GROUPED, PAIR>(hb, sh, job, p, cb, n, lds_values, tbw, xprev);
                 __syncthreads();  // every output of the group issued by every thread
                 if (threadIdx.x == 0) complete_cb(job, C, part, (uint32_t)n, tbw, xprev);
             }
@@ -849,7 +857,7 @@ __global__ __launch_bounds__(384) void pusch_serve_resident(const serve_ring_hdr
             const uint32_t C = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_prm.num_CBs);
             if ((uint32_t)(cb + n) <= C) {
                 uint32_t xprev = 0;
-                const uint32_t part = fused_group<TI, 46, true>(hb, sh, s_job, s_prm, cb, n, lds_values, tbw, xprev);
+                const uint32_t part = fused_group<TI, 46, true, 1>(hb, sh, s_job, s_prm, cb, n, lds_values, tbw, xprev);
                 __syncthreads();  // every output of the group issued by every thread
                 if (tid == 0) complete_cb(s_job, C, part, (uint32_t)n, tbw, xprev);
             }
@@ -1008,13 +1016,14 @@ cuphyStatus_t slot_decode(const cuphyHipPuschSlotTb_t* d_tbs, int n_tbs, const u
     cuphyStatus_t s = ensure_lds_attr(func, lds);  // also for an empty launch: prepares graph capture
     if (s != CUPHY_STATUS_SUCCESS) return s;
     if (n_items == 0) return CUPHY_STATUS_SUCCESS;
+    const int threads = fused_threads(max_parity_nodes);
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, func, 384, lds) != hipSuccess || per_cu < 1) per_cu = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, func, threads, lds) != hipSuccess || per_cu < 1) per_cu = 1;
     const int grid = std::min(n_items, std::max(1, cu_count) * per_cu);
     uint32_t* ws = static_cast<uint32_t*>(d_ws);
     void* args[6] = {const_cast<cuphyHipPuschSlotTb_t**>(&d_tbs), &n_tbs, const_cast<uint32_t**>(&d_items),
                      &n_items, &max_lds_values, &ws};
-    if (hipLaunchKernel(func, dim3((unsigned)grid), dim3(384), args, lds, strm) != hipSuccess)
+    if (hipLaunchKernel(func, dim3((unsigned)grid), dim3((unsigned)threads), args, lds, strm) != hipSuccess)
         return CUPHY_STATUS_INTERNAL_ERROR;
     return CUPHY_STATUS_SUCCESS;
 }
