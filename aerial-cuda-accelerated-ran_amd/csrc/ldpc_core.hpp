@@ -597,6 +597,40 @@ __device__ __forceinline__ uint32_t row_syndrome(BP __restrict__ base, shift_ptr
     return par;
 }
 
+// Place of the calling wave in the order in which a workgroup of 8 waves hands
+// its lanes to the rows of a code block.  The CU's 4 SIMDs get the waves of a
+// workgroup of 6 (Z > 320) as 2/2/1/1 and two such workgroups as 4/2/3/3 on 96 %
+// of the CUs (SIMD_ID of every wave), and a workgroup's barriers run at the pace
+// of its fullest SIMD.  8 waves are two per SIMD; places 6 and 7, which hold no
+// rows, are given to waves of SIMDs 2 and 3, in the CU's second workgroup of
+// SIMDs 0 and 1 (the place of its LDS tells it), which leaves 3/3/3/3.  Whatever
+// the placement, the 8 places are distinct.  scratch: 8 LDS words, free again
+// on return.
+constexpr uint32_t BALANCED_WAVES = 8;
+__device__ __forceinline__ uint32_t balanced_wave_place(uint32_t* scratch)
+{
+    constexpr int HW_ID_SIMD = 4 | (4 << 6) | ((2 - 1) << 11);      // HW_ID bits 5:4
+    constexpr int LDS_ALLOC_BASE = 6 | (0 << 6) | ((8 - 1) << 11);  // LDS_ALLOC bits 7:0
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t first = __builtin_amdgcn_s_getreg(LDS_ALLOC_BASE) != 0 ? 2u : 0u;  // SIMD of place 0
+    scratch[wave] = (uint32_t)__builtin_amdgcn_s_getreg(HW_ID_SIMD);
+    __syncthreads();
+    uint32_t simd[BALANCED_WAVES], key[BALANCED_WAVES], mine = 0, place = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < BALANCED_WAVES; ++i) {
+        simd[i] = __builtin_amdgcn_readfirstlane(scratch[i]) & 3u;
+        uint32_t before = 0;  // waves of the workgroup on this SIMD so far
+#pragma unroll
+        for (uint32_t j = 0; j < i; ++j) before += simd[j] == simd[i] ? 1u : 0u;
+        key[i] = (before * 4u + ((simd[i] - first) & 3u)) * BALANCED_WAVES + i;
+        mine = i == wave ? key[i] : mine;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < BALANCED_WAVES; ++i) place += key[i] < mine ? 1u : 0u;
+    __syncthreads();
+    return place;
+}
+
 // Everything one code block's decode needs, resolved from a TB descriptor
 // (transport-block kernel) or from a batch work item (persistent kernel).
 struct cb_job {
@@ -674,6 +708,7 @@ template <> __device__ __forceinline__ _Float16 job_alpha<_Float16>(const cb_job
 // wave-aligned) form two lane groups that process the rows of kPairPlan's
 // group 0 and group 1; rows of one barrier segment run at the same time,
 // and each lane holds the message state of its group's rows only.
+// tid: the thread's place among the lanes.
 // LM: lane-major APP values from LDS address 0 (lm_pitch_bytes; count must
 // be 1, cb_flags two LDS words for the early-termination votes).
 // PRE (lane-major only): every edge's rotated lane offset in a register,
@@ -683,14 +718,14 @@ template <> __device__ __forceinline__ _Float16 job_alpha<_Float16>(const cb_job
 // row after another (a wave per SIMD has the registers).
 template <int BG, typename T, int MAXR, int PAIR = 1, bool LM = (PAIR == 2), bool PRE = false>
 __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job& job, int count = 1, int stride = 0,
-                                              uint32_t* cb_flags = nullptr, uint32_t* cb_iters = nullptr)
+                                              uint32_t* cb_flags = nullptr, uint32_t* cb_iters = nullptr,
+                                              uint32_t tid = threadIdx.x)
 {
     using BGT = bg_traits<BG>;
     constexpr int NR = (MAXR < BGT::NROWS) ? MAXR : BGT::NROWS;
     constexpr pair_plan<BG, NR> PP = kPairPlan<BG, NR>;
     const uint32_t Z = (uint32_t)job.Z;
     const int mb = job.mb;
-    const uint32_t tid = threadIdx.x;
     const T alpha = job_alpha<T>(job);
 
     // C2V state: per row or per edge (binary32, f32_plan), per edge (binary16)
@@ -960,7 +995,8 @@ __device__ __forceinline__ int decode_group(T* __restrict__ app, const cb_job& j
 // 2 * roundup64(Z)); PAIR = 1: one lane group (blockDim.x >= Z).  flag: one
 // LDS word outside the values (the early-termination vote).
 template <int BG, typename T, typename TIn, int MAXR, int PAIR, bool PRE = false>
-__device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job, const cb_buffers& b, uint32_t* flag)
+__device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job, const cb_buffers& b, uint32_t* flag,
+                                         uint32_t tid = threadIdx.x, uint32_t nthr = blockDim.x)
 {
     const int Z = job.Z;
     const int ncol = bg_traits<BG>::NSYS + job.mb;
@@ -971,8 +1007,8 @@ __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job,
     // (per = blockDim.x / Z >= 1 column streams; coalesced over z)
     {
         const TIn* src = static_cast<const TIn*>(b.llr);
-        const int per = (int)blockDim.x / Z;
-        const int t = (int)threadIdx.x;
+        const int per = (int)nthr / Z;
+        const int t = (int)tid;
         const T clampv = (T)job.clamp;
         const bool do_clamp = job.clamp > 0.0f;
         if (t < per * Z) {
@@ -998,15 +1034,14 @@ __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job,
         }
         __syncthreads();
     }
-    const int iters = run_iterations<BG, T, MAXR, PAIR, true, PRE>(app, job, 1, 0, flag);
+    const int iters = run_iterations<BG, T, MAXR, PAIR, true, PRE>(app, job, 1, 0, flag, nullptr, tid);
     const int nbits = job.Kb * Z;
     // hard decisions, 64 per wave per step by ballot (as store_hard); each
     // lane walks its (column, z) position instead of dividing per bit
     {
         const int nwords = (nbits + 31) >> 5;
-        const int tid = (int)threadIdx.x;
-        const int lane = tid & 63;
-        const int nwaves = (int)((blockDim.x + 63u) >> 6);
+        const int lane = (int)tid & 63;
+        const int nwaves = (int)((nthr + 63u) >> 6);
         const int step = nwaves * 64;
         int n = (tid >> 6) * 64 + lane;
         int col = n / Z, z = n - col * Z;
@@ -1027,8 +1062,8 @@ __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job,
         }
     }
     if (b.soft) {
-        const int step = (int)blockDim.x;
-        int n = (int)threadIdx.x;
+        const int step = (int)nthr;
+        int n = (int)tid;
         int col = n / Z, z = n - col * Z;
         for (; n < nbits; n += step) {
             b.soft[n] = (_Float16)lds_at<T>(lds, (uint32_t)z * pitch + lm_col_offset(BG, col, (int)sizeof(T), SPL));

@@ -184,15 +184,22 @@ __global__ __launch_bounds__(384) void ldpc_layered_persistent(cuphyHipLDPCWorkI
 // dynamic allocation.
 template <typename T, typename TIn, int MAXR, int PAIR>
 __device__ __forceinline__ void persistent_lm(cuphyHipLDPCWorkItem_t* items, const uint32_t* __restrict__ group_first,
-                                              int n_groups, int lds_values, uint32_t* __restrict__ queue)
+                                              int n_groups, int lds_values, uint32_t* __restrict__ queue,
+                                              int rows_threads)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const uint32_t lds_bytes = (uint32_t)lds_values * (uint32_t)sizeof(T);
     int* const s_item = reinterpret_cast<int*>(lds_raw + lds_bytes - 16u);
     uint32_t* const flag = reinterpret_cast<uint32_t*>(lds_raw + lds_bytes - 8u);
     T* app = reinterpret_cast<T*>(lds_raw);
+    uint32_t tid = threadIdx.x;
+    if (PAIR == 1 && rows_threads < (int)blockDim.x) {
+        const uint32_t place = balanced_wave_place(reinterpret_cast<uint32_t*>(lds_raw));
+        if (place * 64u >= (uint32_t)rows_threads) return;  // (a barrier waits for the waves that have not ended)
+        tid = place * 64u + (tid & 63u);
+    }
     for (;;) {
-        if (threadIdx.x == 0) *s_item = (int)atomicAdd(&queue[0], 1u);
+        if (tid == 0) *s_item = (int)atomicAdd(&queue[0], 1u);
         __syncthreads();
         const int g = __builtin_amdgcn_readfirstlane(*s_item);
         __syncthreads();
@@ -207,20 +214,20 @@ __device__ __forceinline__ void persistent_lm(cuphyHipLDPCWorkItem_t* items, con
                 // lane-major APP values, below the last 16 bytes
                 const uint32_t need = lm_app_bytes(w.BG, job.Z, ((w.BG == 1) ? 22 : 10) + job.mb, (int)sizeof(T),
                                                    lm_split_layout((int)sizeof(T), MAXR));
-                if (need + 16u > lds_bytes || PAIR * ((job.Z + 63) & ~63) > (int)blockDim.x) st = CUPHY_HIP_ITEM_NO_FIT;
+                if (need + 16u > lds_bytes || PAIR * ((job.Z + 63) & ~63) > rows_threads) st = CUPHY_HIP_ITEM_NO_FIT;
             }
-            if (threadIdx.x == 0) w.status = st;
+            if (tid == 0) w.status = st;
             if (st == 0) {
                 const cb_buffers b{w.llr, w.out, static_cast<_Float16*>(w.soft)};
                 if (w.BG == 1)
-                    decode_lm<1, T, TIn, MAXR, PAIR>(app, job, b, flag);
+                    decode_lm<1, T, TIn, MAXR, PAIR>(app, job, b, flag, tid, (uint32_t)rows_threads);
                 else
-                    decode_lm<2, T, TIn, MAXR, PAIR>(app, job, b, flag);
+                    decode_lm<2, T, TIn, MAXR, PAIR>(app, job, b, flag, tid, (uint32_t)rows_threads);
             }
             __syncthreads();
         }
     }
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         __threadfence();
         const uint32_t done = atomicAdd(&queue[1], 1u);
         if (done == gridDim.x - 1) {
@@ -243,18 +250,17 @@ __global__ __launch_bounds__(768) void ldpc_layered_persistent_pair(cuphyHipLDPC
                                                                     int n_groups, int lds_values,
                                                                     uint32_t* __restrict__ queue)
 {
-    persistent_lm<T, TIn, MAXR, 2>(items, group_first, n_groups, lds_values, queue);
+    persistent_lm<T, TIn, MAXR, 2>(items, group_first, n_groups, lds_values, queue, (int)blockDim.x);
 }
 
 // One code block per workgroup (one lane group), lane-major APP values:
 // for launches without code-block groups.  Same queue protocol.
 template <typename T, typename TIn, int MAXR>
-__global__ __launch_bounds__(384) void ldpc_layered_persistent_lm(cuphyHipLDPCWorkItem_t* items,
-                                                                  const uint32_t* __restrict__ group_first,
-                                                                  int n_groups, int lds_values,
-                                                                  uint32_t* __restrict__ queue)
+__global__ __launch_bounds__(64 * BALANCED_WAVES)
+void ldpc_layered_persistent_lm(cuphyHipLDPCWorkItem_t* items, const uint32_t* __restrict__ group_first, int n_groups,
+                                int lds_values, uint32_t* __restrict__ queue, int rows_threads)
 {
-    persistent_lm<T, TIn, MAXR, 1>(items, group_first, n_groups, lds_values, queue);
+    persistent_lm<T, TIn, MAXR, 1>(items, group_first, n_groups, lds_values, queue, rows_threads);
 }
 
 // ---------------------------------------------------------------------------
@@ -461,7 +467,13 @@ cuphyStatus_t decode_batch(cuphyHipLDPCWorkItem_t* d_items, const uint32_t* d_gr
                                                                 : select_persistent_lm_kernel<46>(llr_type, f16))
                  : max_mb <= SMALL_MAXR ? select_persistent_kernel<SMALL_MAXR>(llr_type, f16)
                                         : select_persistent_kernel<46>(llr_type, f16);
-    const unsigned block = (unsigned)block_threads;
+    // 5 or 6 waves of which two workgroups share a CU: balanced over its SIMDs
+    // (the 46-row kernels' registers leave one workgroup per CU).  2,800 BG1
+    // Zc = 384 blocks of 4 rows: 322 -> 311 us; with the two spare waves kept for
+    // the barriers 327 us
+    const bool balance = lm && !pair && block_threads > 256 && max_mb <= SMALL_MAXR;
+    const unsigned block = balance ? 64u * BALANCED_WAVES : (unsigned)block_threads;
+    int rows_threads = block_threads;  // (of them, those that hold rows)
     // lane-major: APP rows padded to an odd number of words, at most 7 bytes
     // per lane beyond the values (Z <= 384), and 16 bytes of queue slot and
     // vote; the split layout of the binary16 46-row kernels needs its
@@ -477,8 +489,9 @@ cuphyStatus_t decode_batch(cuphyHipLDPCWorkItem_t* d_items, const uint32_t* d_gr
         per_cu = 1;
     const int grid = std::min(n_groups, std::max(1, cu_count) * per_cu);
     int lds_values = (int)(lds / elem);
-    void* args[5] = {&d_items, const_cast<uint32_t**>(&d_group_first),
-                     &n_groups, &lds_values, &d_queue};
+    // (the kernels without that parameter ignore the sixth)
+    void* args[6] = {&d_items, const_cast<uint32_t**>(&d_group_first),
+                     &n_groups, &lds_values, &d_queue, &rows_threads};
     if (hipLaunchKernel(func, dim3((unsigned)grid), dim3(block), args, lds, strm) != hipSuccess)
         return CUPHY_STATUS_INTERNAL_ERROR;
     return CUPHY_STATUS_SUCCESS;

@@ -519,7 +519,7 @@ template <typename TI, int MAXR, bool GROUPED, int PAIR>
 __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused_lds& sh,
                                                 const cuphyHipPuschSlotTb_t& job, const PerTbParams& p, int cb0,
                                                 int count_in, int lds_values, uint32_t* __restrict__ tbw,
-                                                uint32_t& xor_prev)
+                                                uint32_t& xor_prev, uint32_t row_wave)
 {
     const int count = GROUPED ? count_in : 1;
     rm_geometry g0 = rm_geometry_of(p, cb0);
@@ -586,8 +586,9 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
     dj.alpha_f16 = (uint16_t)(job.norm.f16x2 & 0xFFFFu);
     uint32_t* const flags = (count > 1) ? sh.cb_flags : nullptr;
     uint32_t* const cb_it = (count > 1) ? sh.cb_iters : nullptr;
-    const int iters = (bg == 1) ? run_iterations<1, _Float16, MAXR, PAIR, false>(hb, dj, count, S, flags, cb_it)
-                                : run_iterations<2, _Float16, MAXR, PAIR, false>(hb, dj, count, S, flags, cb_it);
+    const uint32_t row_tid = row_wave * 64u + (threadIdx.x & 63u);
+    const int iters = (bg == 1) ? run_iterations<1, _Float16, MAXR, PAIR, false>(hb, dj, count, S, flags, cb_it, row_tid)
+                                : run_iterations<2, _Float16, MAXR, PAIR, false>(hb, dj, count, S, flags, cb_it, row_tid);
 
     // ---- 5. hard decisions of all CBs into LDS and memory --------------------
     const int tt = opaque_tid();
@@ -690,8 +691,10 @@ __device__ __forceinline__ void complete_cb(const cuphyHipPuschSlotTb_t& job, ui
 // per CU, two lane groups of FUSED_BLOCK (run_iterations PAIR = 2; 168 VGPRs, no
 // spills): every phase has twice the waves and the rows of a barrier segment run
 // side by side.  One group against two: 64 descrambled UEs with a retransmission
-// 429 -> 411 us, a served burst of 384 TBs 1083 -> 1041 us.
-constexpr int fused_threads(int maxr) { return maxr <= MID_MAXR ? FUSED_BLOCK : 2 * FUSED_BLOCK; }
+// 429 -> 411 us, a served burst of 384 TBs 1083 -> 1041 us.  Where two workgroups
+// share a CU, 8 waves, of which lanes past FUSED_BLOCK hold no rows in the decode:
+// 64-cell int8 slot 572 -> 546 us (6 waves -> 8, balanced_wave_place).
+constexpr int fused_threads(int maxr) { return maxr <= MID_MAXR ? 64 * (int)BALANCED_WAVES : 2 * FUSED_BLOCK; }
 
 // Persistent fused slot kernel.  Workspace: queue state (2 words used of
 // FUSED_WS_QUEUE_WORDS), then two words per CB slot of the launch, of which
@@ -717,6 +720,10 @@ void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
     uint32_t* tbw = ws + FUSED_WS_QUEUE_WORDS;
     load_crc_steps(sh);
     constexpr int PAIR = MAXR <= MID_MAXR ? 1 : 2;
+    uint32_t row_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // one-CB form: bound by its instructions, 64-cell int8 slot 552 -> 546 us; groups
+    // leave few waves without rows (64 UEs 411 -> 418 us with it: registers)
+    if (PAIR == 1 && !GROUPED) row_wave = balanced_wave_place(sh.words);
     if (threadIdx.x == 0) sh.item = (int)atomicAdd(&queue[0], 1u);
     __syncthreads();
     for (;;) {
@@ -731,7 +738,8 @@ void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
             const uint32_t C = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.num_CBs);
             if ((uint32_t)(cb + n) <= C) {
                 uint32_t xprev = 0;
-                const uint32_t part = fused_group<TI, MAXR, GROUPED, PAIR>(hb, sh, job, p, cb, n, lds_values, tbw, xprev);
+                const uint32_t part = fused_group<TI, MAXR, GROUPED, PAIR>(hb, sh, job, p, cb, n, lds_values, tbw, xprev,
+                                                                         row_wave);
                 __syncthreads();  // every output of the group issued by every thread
                 if (threadIdx.x == 0) complete_cb(job, C, part, (uint32_t)n, tbw, xprev);
             }
@@ -857,7 +865,8 @@ __global__ __launch_bounds__(384) void pusch_serve_resident(const serve_ring_hdr
             const uint32_t C = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_prm.num_CBs);
             if ((uint32_t)(cb + n) <= C) {
                 uint32_t xprev = 0;
-                const uint32_t part = fused_group<TI, 46, true, 1>(hb, sh, s_job, s_prm, cb, n, lds_values, tbw, xprev);
+                const uint32_t part = fused_group<TI, 46, true, 1>(hb, sh, s_job, s_prm, cb, n, lds_values, tbw, xprev,
+                                                                (uint32_t)tid >> 6);
                 __syncthreads();  // every output of the group issued by every thread
                 if (tid == 0) complete_cb(s_job, C, part, (uint32_t)n, tbw, xprev);
             }

@@ -92,6 +92,36 @@ def test_batch_row_pair_equals_one_lane_group(dec, dtype):
             assert torch.equal(s1.view(torch.int16), s2.view(torch.int16)), (MIX[k], et)
 
 
+@pytest.mark.parametrize("et", [False, True])
+@pytest.mark.parametrize("bg,Z,mb", [(1, 384, 4), (1, 352, 8), (2, 320, 5)])
+def test_batch_two_workgroups_per_cu(dec, bg, Z, mb, et):
+    """More code blocks than CUs hold at once, in the high-rate kernel whose
+    workgroups are spread over the SIMDs: hard and soft outputs of the
+    transport-block kernel, the first code blocks as the oracle has them."""
+    from aerial_amd import _lib as L
+    from aerial_amd.batch import BatchDecoder
+    from aerial_amd.decoder import LdpcDecodeConfig
+    print("[case] batch high rate bg%d Z=%d mb=%d et=%d" % (bg, Z, mb, et), flush=True)
+    ncb, flags = 1100, L.CUPHY_LDPC_DECODE_EARLY_TERM if et else 0
+    llr = torch.randn((ncb, (V.nsys(bg) + mb) * Z), generator=torch.Generator().manual_seed(Z + mb)).mul_(6).half()
+    llr[::3] = llr[::3].abs() + 1  # (the all-zero code word: stops early)
+    dev = llr.cuda()
+    hard = [torch.full((ncb, (V.nsys(bg) * Z + 31) // 32), -1, dtype=torch.int32, device="cuda") for _ in range(2)]
+    soft = [torch.zeros((ncb, V.nsys(bg) * Z), dtype=torch.float16, device="cuda") for _ in range(2)]
+    tb = SimpleNamespace(bg=bg, Z=Z, mb=mb, ncb=ncb, llr=dev, out=hard[0])
+    b = BatchDecoder(dec, pack=False).build([tb], llr_type=L.CUPHY_R_16F, fp16_math=True, max_iterations=5,
+                                            flags=flags, soft=[soft[0]])
+    b.launch()
+    cfg = LdpcDecodeConfig(bg, Z, mb, llr_type=L.CUPHY_R_16F, max_iterations=5, alpha=0.8125, flags=flags)
+    dec.decode_tb(cfg, [dev], [hard[1]], [soft[1]])
+    torch.cuda.synchronize()
+    assert all(int(w.abs().sum().item()) == 0 for w in b.workspaces)
+    assert torch.equal(hard[0], hard[1]) and torch.equal(soft[0].view(torch.int16), soft[1].view(torch.int16))
+    ref = O.dec_cfg(bg, Z, mb, n_iter=5, alpha=0.8125, clamp=32.0, mode=O.FP16, early_term=et)
+    for i in range(4):
+        assert np.array_equal(hard[0][i].cpu().numpy().view(np.uint32), O.decode_cb(ref, llr[i].float().numpy())[0])
+
+
 def test_batch_order_independent(dec):
     from aerial_amd import _lib as L
     from aerial_amd.batch import BatchDecoder
