@@ -123,6 +123,33 @@ template <int BG, int NR> constexpr pair_plan<BG, NR> make_pair_plan()
 }
 template <int BG, int NR> constexpr pair_plan<BG, NR> kPairPlan = make_pair_plan<BG, NR>();
 
+// Block row R's own parity column: the last edge of every row from 4 on is the
+// only one of its column, with shift 0 in every lifting set.
+template <int BG> constexpr bool own_column(int R)
+{
+    using BGT = bg_traits<BG>;
+    const int last = BGT::row_start(R + 1) - 1;
+    for (int e = 0; e < BGT::row_start(BGT::NROWS); ++e)
+        if (e != last && BGT::col(e) == BGT::col(last)) return false;
+    return BGT::identity_edge(last);
+}
+// Slots of their APP values, counted per lane group.
+template <int BG, int NR> struct own_plan {
+    int slot[64];
+    int count;
+};
+template <int BG, int NR> constexpr own_plan<BG, NR> make_own_plan()
+{
+    own_plan<BG, NR> p{};
+    const pair_plan<BG, NR> pp = make_pair_plan<BG, NR>();
+    int n[2] = {0, 0};
+    for (int r = 0; r < NR; ++r)
+        if (own_column<BG>(r)) p.slot[r] = n[pp.group[r]]++;
+    p.count = n[0] > n[1] ? n[0] : n[1];
+    return p;
+}
+template <int BG, int NR> constexpr own_plan<BG, NR> kOwnPlan = make_own_plan<BG, NR>();
+
 // binary32 state of a kernel holding NR block rows in PAIR lane groups: rows of
 // at most explicit_degree edges keep every edge's message (slot[r]: the first
 // of them), the others their compressed state (slot[r]: the row's).  An
@@ -491,9 +518,11 @@ __device__ __forceinline__ half2_t sub_pair(uint32_t v0, uint32_t v1, half2_t m)
 
 // S0: message slot of the row's first edge (even: padded_row_start(R), or
 // the row's pair_slot within a row-pair lane group).
-template <int BG, int R, int NW, int S0, typename BP, typename Off>
+// OWN: the row's last edge is its own parity column (own_column), whose APP
+// value is `own` (low half) instead of LDS.
+template <int BG, int R, int NW, int S0, bool OWN, typename BP, typename Off>
 __device__ __forceinline__ void process_row(_Float16*, BP __restrict__ base, const Off& off_of, _Float16 alpha,
-                                            half2_t (&st)[NW])
+                                            half2_t (&st)[NW], uint32_t& own)
 {
     using BGT = bg_traits<BG>;
     constexpr int E0 = BGT::row_start(R);
@@ -512,11 +541,15 @@ __device__ __forceinline__ void process_row(_Float16*, BP __restrict__ base, con
     static_for<P>([&](auto K) {
         constexpr int k = decltype(K)::value;
         constexpr int j0 = 2 * k, j1 = 2 * k + 1;
-        off[j0] = off_of(std::integral_constant<int, j0>{});
-        const uint32_t v0 = lds_ld<uint16_t>(base, off[j0]);
+        const auto load = [&](auto J) -> uint32_t {
+            constexpr int j = decltype(J)::value;
+            if constexpr (OWN && j == D - 1) return own;
+            off[j] = off_of(J);
+            return lds_ld<uint16_t>(base, off[j]);
+        };
+        const uint32_t v0 = load(std::integral_constant<int, j0>{});
         if constexpr (j1 < D) {
-            off[j1] = off_of(std::integral_constant<int, j1>{});
-            const uint32_t v1 = lds_ld<uint16_t>(base, off[j1]);
+            const uint32_t v1 = load(std::integral_constant<int, j1>{});
             if constexpr (SDWA_PAIR)
                 t[k] = sub_pair(v0, v1, st[W0 + k]);
             else
@@ -569,22 +602,29 @@ __device__ __forceinline__ void process_row(_Float16*, BP __restrict__ base, con
         const half2_t sa = u2h2(__builtin_amdgcn_bitop3_b32(h22u(t[k]), Q, SIGNS, (unsigned char)0x6C));
         const half2_t c = other * sa;
         const uint32_t nv = h22u(t[k] + c);
-        lds_st<uint16_t>(base, off[j0], (uint16_t)nv);
-        if constexpr (j1 < D) lds_st<uint16_t>(base, off[j1], (uint16_t)(nv >> 16));
+        if constexpr (OWN && j0 == D - 1)
+            own = nv & 0xFFFFu;
+        else
+            lds_st<uint16_t>(base, off[j0], (uint16_t)nv);
+        if constexpr (OWN && j1 == D - 1)
+            own = nv >> 16;
+        else if constexpr (j1 < D)
+            lds_st<uint16_t>(base, off[j1], (uint16_t)(nv >> 16));
         st[W0 + k] = c;
     });
 }
 
 // Parity of check row R, lane z: hard bit = APP < 0 (syndrome_check.m:38-40).
+// OWN: as process_row.
 template <int BG, int R, typename T, bool LM = false, typename BP = unsigned char*, bool PK = false,
-          bool SPL = false>
+          bool SPL = false, bool OWN = false>
 __device__ __forceinline__ uint32_t row_syndrome(BP __restrict__ base, shift_ptr sh, uint32_t zb, uint32_t zp,
-                                                 uint32_t Zb, uint32_t Pb = 0)
+                                                 uint32_t Zb, uint32_t Pb = 0, uint32_t own = 0)
 {
     using BGT = bg_traits<BG>;
     constexpr int E0 = BGT::row_start(R);
-    constexpr int D = BGT::row_start(R + 1) - E0;
-    uint32_t par = 0;
+    constexpr int D = BGT::row_start(R + 1) - E0 - (OWN ? 1 : 0);
+    uint32_t par = OWN ? own & 0xFFFFu : 0u;
     static_for<D>([&](auto J) {
         constexpr int j = decltype(J)::value;
         const uint32_t off = edge_off<BG, E0 + j, T, LM, PK, SPL>(sh, zb, zp, Zb, Pb);
@@ -809,6 +849,29 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
             pre[I] = v;
         });
     }
+    // Row-pair binary16 kernels keep the APP values of the rows' own parity
+    // columns in registers: an LDS instruction takes 2.2 (read) to 2.5 ns (write)
+    // of the CU whatever its width, 9 us of an iteration's 15 (BG1 Zc = 384, all
+    // rows), and these columns are 42 of BG1's 316 edges, 38 of BG2's 197.
+    // Mixed slot of 16 UEs 153 -> 149 us, receive chain of 64 UEs 411 -> 396 us.
+    // Not in the kernels whose registers are full (one lane group, offsets in
+    // registers, binary32).
+    constexpr bool OWNS = PAIR == 2 && !F32 && !PRE;
+    constexpr own_plan<BG, NR> own_slots = kOwnPlan<BG, NR>;
+    constexpr int NOWN = OWNS && own_slots.count > 0 ? own_slots.count : 1;
+    uint32_t own[NOWN];
+    if constexpr (OWNS) {
+        static_for<NOWN>([&](auto I) { own[I] = 0u; });
+        static_for<NR>([&](auto Rc) {
+            constexpr int R = decltype(Rc)::value;
+            if constexpr (own_column<BG>(R)) {
+                constexpr int E = BGT::row_start(R + 1) - 1;
+                if (R < mb && active && lgrp == (uint32_t)PP.group[R])
+                    own[own_slots.slot[R]] =
+                        lds_ld<uint16_t>(lane_base, edge_off<BG, E, T, LM, PK, SPL>(sh, 0u, zlane * Pb, Zb, Pb));
+            }
+        });
+    }
     int it = 0;
     while (it < job.max_iter) {
         ++it;
@@ -844,7 +907,8 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
                     else if constexpr (F32)
                         process_row<BG, R, NRS, FP.slot[R]>(app, lane_base, off_of, alpha, st_n1, st_n2, st_meta);
                     else
-                        process_row<BG, R, NW, S0>(app, lane_base, off_of, alpha, st_h);
+                        process_row<BG, R, NW, S0, OWNS && own_column<BG>(R)>(
+                            app, lane_base, off_of, alpha, st_h, own[OWNS ? own_slots.slot[R] : 0]);
                 }
                 // barrier before the next row only where it shares a column
                 // with the rows since the last barrier, and at the iteration end
@@ -867,8 +931,9 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
                             uint32_t Zr = Zb;
                             asm volatile("" : "+s"(shr), "+s"(Zr));
                             if (active && (PAIR == 1 || lgrp == (uint32_t)PP.group[R]))
-                                fail |= row_syndrome<BG, R, T, LM, decltype(lane_base), PK, SPL>(lane_base, shr, zb,
-                                                                                                 zp, Zr, Pb);
+                                fail |= row_syndrome<BG, R, T, LM, decltype(lane_base), PK, SPL,
+                                                     OWNS && own_column<BG>(R)>(
+                                    lane_base, shr, zb, zp, Zr, Pb, own[OWNS ? own_slots.slot[R] : 0]);
                         }
                     }
                 });
