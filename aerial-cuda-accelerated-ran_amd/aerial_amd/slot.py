@@ -29,7 +29,7 @@ def half_bits(x):
     return int(torch.tensor([x], dtype=torch.float16).view(torch.int16).item()) & 0xFFFF
 
 
-FUSED_BLOCK = 384                    # threads of a fused-kernel workgroup
+FUSED_BLOCK = 384                    # lanes that hold rows, per lane group of a fused-kernel workgroup
 FUSED_MAX_GROUP = 16                 # CBs of one work item at most
 SLOT_MAX_LDS_VALUES = 68 * 384 + 2 * 12288
 

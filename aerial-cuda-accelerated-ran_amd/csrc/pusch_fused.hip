@@ -502,12 +502,12 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
 }
 
 // A group of `count` consecutive CBs cb0 .. cb0 + count - 1 of one TB
-// (count * Zc <= blockDim.x).  CB c's HARQ/APP array is at hb + c * S
+// (count * Zc <= FUSED_BLOCK).  CB c's HARQ/APP array is at hb + c * S
 // (S = max(2Zc + Ncb, (nsys + mb) * Zc), rounded up to whole 16-byte units
 // when count > 1); descrambling words follow the last array.  Steps 1-3
 // run CB by CB with the whole workgroup; the decode runs the group side by
-// side (lanes [c * Zc, (c + 1) * Zc) on CB c, each CB stopping on its own
-// syndrome: results as decoded alone); hard decisions and CRCs again CB by
+// side (lanes [c * Zc, (c + 1) * Zc) of each lane group on CB c, each CB stopping
+// on its own syndrome: results as decoded alone); hard decisions and CRCs again CB by
 // CB.  Returns, in the completing thread, the XOR of the CBs' shares of the TB
 // CRC24A (each the remainder of the CB's payload bytes shifted to their
 // place in the TB; for a one-CB TB its CRC, which is the TB CRC), or
@@ -702,11 +702,10 @@ constexpr int fused_threads(int maxr) { return maxr <= MID_MAXR ? 64 * (int)BALA
 // finished CBs; see complete_cb).  The next item index is fetched while the current CB is
 // worked on.  The queue is returned to 0 by the last workgroup to leave.
 // The high-rate variant (MAXR <= 8) and the middle one (MAXR <= 16) are
-// held to 4 waves per SIMD (at most 128 VGPRs): a 384-thread workgroup puts
-// its 6 waves 2/2/1/1 on the CU's SIMDs, so a second workgroup on the CU
-// needs 4 wave slots on two SIMDs; at its natural 157 VGPRs (3 slots) the
-// high-rate variant ran one workgroup per CU.  (The middle variant's BG1
-// rows beyond 8 spill a few registers; BG2 rows, half as long, do not.)
+// held to 4 waves per SIMD (at most 128 VGPRs): two workgroups of 8 waves fill
+// them.  At its natural 157 VGPRs (3 slots) the high-rate variant ran one
+// workgroup per CU.  (The middle variant's BG1 rows beyond 8 spill a few
+// registers; BG2 rows, half as long, do not.)
 template <typename TI, int MAXR, bool GROUPED>
 __global__ __launch_bounds__(fused_threads(MAXR)) __attribute__((amdgpu_waves_per_eu(MAXR <= MID_MAXR ? 4 : 1)))
 void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,

@@ -483,7 +483,7 @@ cuphyStatus_t CUPHYWINAPI cuphyHipPuschSlotDecodeGetWorkspaceSize(int num_cbs, s
  * CRC + TB assembly + TB CRC for num_cb_items work items in one persistent
  * launch.  d_cb_items[i] = (TB index << 16) | ((count - 1) << 12) | CB
  * index within the TB: the `count` (1..16) consecutive CBs from that index
- * on, decoded side by side in one 384-thread workgroup (count * Zc <= 384;
+ * on, decoded side by side in one workgroup (count * Zc <= 384;
  * each CB stops on its own syndrome, results as decoded alone); count = 1
  * gives one CB per item, (TB index << 16) | CB index (CB index < 4096).
  * Every CB of a TB must be in the launch exactly once.  A TB's CRC
