@@ -412,7 +412,9 @@ __device__ __forceinline__ void process_row(float*, BP __restrict__ base, const 
 // first-index rule gives); the product with +-alpha has the magnitude
 // alpha * other rounded the same.  |t| is masked once, so that the minima
 // take the two-operand encodings, which issue at twice the rate of the
-// three-operand ones that an absolute-value modifier needs.
+// three-operand ones that an absolute-value modifier needs.  NaNs (infinite
+// LLRs without a clamp give them: inf - inf) count as in the other rows, whose
+// minima start at +inf: the first edge's |t| is taken as min(|t|, +inf).
 __device__ __forceinline__ float fmin2(float a, float b)
 {
     float r;
@@ -425,14 +427,20 @@ __device__ __forceinline__ float fmax2(float a, float b)
     asm("v_max_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+// Sign bits that a row's edges may flip in alpha: none when alpha is negative
+// (a message is |alpha| * other or'ed with its sign, as in the other rows, and
+// so always negative then).
+__device__ __forceinline__ uint32_t explicit_signs(float alpha)
+{
+    return (__builtin_amdgcn_readfirstlane((int)f2u(alpha)) < 0) ? 0u : 0x80000000u;
+}
 template <int BG, int R, int NM, int S0, typename BP, typename Off>
 __device__ __forceinline__ void process_row_explicit(BP __restrict__ base, const Off& off_of, float alpha,
-                                                     float (&st)[NM])
+                                                     uint32_t signs, float (&st)[NM])
 {
     using BGT = bg_traits<BG>;
     constexpr int E0 = BGT::row_start(R);
     constexpr int D = BGT::row_start(R + 1) - E0;
-    constexpr uint32_t SIGN = 0x80000000u;
     float t[D], a[D];
     uint32_t off[D];
     uint32_t mags = 0x7FFFFFFFu;
@@ -443,7 +451,9 @@ __device__ __forceinline__ void process_row_explicit(BP __restrict__ base, const
         t[j] = lds_ld<float>(base, off[j]) - st[S0 + j];
         a[j] = u2f(f2u(t[j]) & mags);
     });
-    float m1 = fmin2(a[0], a[1]), m2 = fmax2(a[0], a[1]);
+    float first;  // min(|t|, +inf)
+    asm("v_min_f32_e32 %0, 0x7f800000, %1" : "=v"(first) : "v"(a[0]));
+    float m1 = fmin2(first, a[1]), m2 = fmax2(first, a[1]);
     uint32_t par = f2u(t[0]) ^ f2u(t[1]);
     static_for<D>([&](auto J) {
         constexpr int j = decltype(J)::value;
@@ -454,12 +464,12 @@ __device__ __forceinline__ void process_row_explicit(BP __restrict__ base, const
         }
     });
     const uint32_t S = f2u(m1) + f2u(m2);
-    const uint32_t Q = f2u(alpha) ^ (par & SIGN);
+    const uint32_t Q = f2u(alpha) ^ (par & signs);
     static_for<D>([&](auto J) {
         constexpr int j = decltype(J)::value;
         const float other = u2f(S - f2u(fmin2(a[j], m2)));
-        // Q ^ (t & SIGN) as one three-input bitwise instruction (table 0x6C: B ^ (A & C))
-        const float c = other * u2f(__builtin_amdgcn_bitop3_b32(f2u(t[j]), Q, SIGN, (unsigned char)0x6C));
+        // Q ^ (t & signs) as one three-input bitwise instruction (table 0x6C: B ^ (A & C))
+        const float c = other * u2f(__builtin_amdgcn_bitop3_b32(f2u(t[j]), Q, signs, (unsigned char)0x6C));
         lds_st<float>(base, off[j], t[j] + c);
         st[S0 + j] = c;
     });
@@ -767,6 +777,7 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
     const uint32_t Z = (uint32_t)job.Z;
     const int mb = job.mb;
     const T alpha = job_alpha<T>(job);
+    const uint32_t signs = std::is_same<T, float>::value ? explicit_signs((float)alpha) : 0u;
 
     // C2V state: per row or per edge (binary32, f32_plan), per edge (binary16)
     // binary16 message slots: every row padded to an even number of edges
@@ -903,7 +914,7 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
                             return edge_off<BG, E, T, LM, PK, SPL>(shr, zb, zp, Zr, Pb);
                     };
                     if constexpr (F32 && FP.is_explicit[R])
-                        process_row_explicit<BG, R, NM, FP.slot[R]>(lane_base, off_of, alpha, st_f);
+                        process_row_explicit<BG, R, NM, FP.slot[R]>(lane_base, off_of, alpha, signs, st_f);
                     else if constexpr (F32)
                         process_row<BG, R, NRS, FP.slot[R]>(app, lane_base, off_of, alpha, st_n1, st_n2, st_meta);
                     else

@@ -322,3 +322,67 @@ def test_launch_descriptor_runs(dec):
     assert rc == 0
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy().view(np.uint32), h_ref)
+
+
+# ---------------------------------------------------------------------------
+# binary32 rows on values that are not finite, and on a negative alpha
+# ---------------------------------------------------------------------------
+def _nan_of(r, a, b):
+    """The GPU's NaN of an invalid operation (inf - inf): all exponent bits,
+    the quiet bit and the sign, which takes part in the sign products."""
+    u = r.view(np.uint32)
+    u[np.isnan(r) & ~np.isnan(a) & ~np.isnan(b)] = 0xFFC00000
+    return r
+
+
+def model_fp32(bg, Z, mb, llr, n_iter, alpha):
+    """The binary32 decoder's rule, row by row, without a clamp: minima by
+    IEEE minNum / maxNum from +inf, the edges whose |t| equals min1 take
+    alpha * min2, the message's sign bit or'ed in.  (The oracle's
+    comparisons treat NaN otherwise.)"""
+    one, sign = np.float32, np.uint32(0x80000000)
+    app = (llr + one(0)).reshape(-1, Z).copy()
+    alpha, z = one(alpha), np.arange(Z)
+    rows = [O.edges(bg, Z, r) for r in range(mb)]
+    c2v = [np.zeros((len(e), Z), one) for e in rows]
+    with np.errstate(all="ignore"):
+        for _ in range(n_iter):
+            for e, msg in zip(rows, c2v):
+                at = [(c, (z + s) % Z) for c, s in e]
+                t = [_nan_of(app[p] - m, app[p], m) for p, m in zip(at, msg)]
+                m1 = m2 = np.full(Z, np.inf, one)
+                par = np.zeros(Z, np.uint32)
+                for x in t:
+                    m2 = np.fmin(m2, np.fmax(m1, np.abs(x)))
+                    m1 = np.fmin(m1, np.abs(x))
+                    par = par ^ x.view(np.uint32)
+                for j, (p, x) in enumerate(zip(at, t)):
+                    mag = np.where(np.abs(x) == m1, alpha * m2, alpha * m1).astype(one)
+                    msg[j] = (mag.view(np.uint32) | ((x.view(np.uint32) ^ par) & sign)).view(one)
+                    app[p] = _nan_of(x + msg[j], x, msg[j])
+    app = app.reshape(-1)[:V.nsys(bg) * Z]
+    return O.pack_bits((app <= 0).astype(np.uint8)), app.astype(np.float16)
+
+
+# row-pair kernels (mb > 8, Z > 32), the 8-row and the 46-row one-group kernels
+@pytest.mark.parametrize("bg,Z,mb", [(1, 64, 46), (2, 104, 20), (2, 64, 42), (2, 52, 8), (1, 72, 5), (1, 24, 20),
+                                     (2, 18, 42)])
+@pytest.mark.parametrize("kind", ["filler", "infinite", "nan", "negative_alpha"])
+def test_fp32_values_not_finite(dec, bg, Z, mb, kind):
+    _log("fp32 %s BG%d Z=%d mb=%d, no clamp, seed=17" % (kind, bg, Z, mb))
+    llr, _ = V.make_cbs(bg, Z, mb, 2, seed=17, snr_db=2.0, filler=2 * Z if kind == "filler" else 0)
+    rng = np.random.RandomState(bg * 1000 + Z)
+    flat, alpha = llr.reshape(-1), 0.8125
+    if kind == "infinite":
+        at = rng.randint(0, flat.size, flat.size // 5)
+        flat[at] = np.copysign(np.inf, flat[at])
+    elif kind == "nan":
+        flat[rng.randint(0, flat.size, flat.size // 50)] = np.nan
+    elif kind == "negative_alpha":
+        alpha = -0.8125
+    for n_iter in (1, 2, 5):
+        h, s = run_gpu(dec, bg, Z, mb, llr, n_iter=n_iter, alpha=alpha, clamp=0.0)
+        for c in range(2):
+            ref_h, ref_s = model_fp32(bg, Z, mb, llr[c], n_iter, alpha)
+            assert np.array_equal(h[c], ref_h), (n_iter, c)
+            assert np.array_equal(s[c], ref_s, equal_nan=True), (n_iter, c)
