@@ -575,7 +575,6 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxRateMatch(cuphyPuschRxRateMatchHndl_t
     d.out = ppRmOut;
     d.tb_prms = pTbPrmsGpu;
     d.descrambling_on = o.descrambling ? 1 : 0;
-    d.lds_bytes = nrldpc::rm_lds_bytes(o.fpconfig, max_e.data(), nSchUes, o.descrambling);
     if (enableCpuToGpuDescrAsyncCpy &&
         hipMemcpyAsync(pGpuDesc, pCpuDesc, sizeof(nrldpc::rm_descriptor), hipMemcpyHostToDevice, strm) != hipSuccess)
         return CUPHY_STATUS_MEMCPY_ERROR;
@@ -583,7 +582,8 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxRateMatch(cuphyPuschRxRateMatchHndl_t
     pLaunchCfg->kernelArgs[0] = &pLaunchCfg->desc;
     set_node(pLaunchCfg->kernelNodeParamsDriver, nrldpc::rm_kernel(o.fpconfig, o.descrambling), dim3(std::max(1u, cmax), std::max<unsigned>(1, nSchUes), 1),
              dim3(nrldpc::RM_BLOCK), pLaunchCfg->kernelArgs);
-    pLaunchCfg->kernelNodeParamsDriver.sharedMemBytes = (unsigned)d.lds_bytes;
+    pLaunchCfg->kernelNodeParamsDriver.sharedMemBytes =
+        (unsigned)nrldpc::rm_lds_bytes(o.fpconfig, max_e.data(), nSchUes, o.descrambling);
     set_node(pLaunchCfg->resetKernelNodeParamsDriver, nrldpc::rm_noop_kernel(), dim3(1), dim3(64), pLaunchCfg->kernelArgs);
     set_node(pLaunchCfg->clampKernelNodeParamsDriver, nrldpc::rm_noop_kernel(), dim3(1), dim3(64), pLaunchCfg->kernelArgs);
     if (nSchUes == 0) pLaunchCfg->kernelNodeParamsDriver.func = nrldpc::rm_noop_kernel();

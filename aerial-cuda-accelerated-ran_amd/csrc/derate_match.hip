@@ -19,9 +19,10 @@
 // order with a clamp after every addition -- so that the HARQ buffer is
 // written once, in 16-byte stores, and read once when combining.  The
 // reference uses atomicAdd in the wrap-around window plus a separate clamp
-// pass.  A CB whose LLRs do not fit the launch's LDS (RM_LDS_LIMIT: E above
-// 32,768 in binary16, 16,384 in binary32) walks the selected bits in passes of
-// L with a barrier between passes, straight from and to memory.
+// pass.  A CB whose LLRs do not fit the launch's LDS walks the selected bits in
+// passes of L with a barrier between passes, straight from and to memory
+// (RM_LDS_LIMIT: E above 32,768 in binary16 and 16,384 in binary32; the
+// sequence's words beside them: above 30,352 and 15,636 with descrambling).
 // Bound by HBM: 2,800 BG1 Zc = 384 CBs of 9,088 bits in binary16 move 197 MB in
 // a first transmission (39 us at the rate of a large copy) and 153 MB in a
 // retransmission.  Measured 37 us on average of the two, against 69 us for the passes with a
@@ -106,6 +107,15 @@ __device__ __forceinline__ void rm_stage(TO* __restrict__ llr, const TI* __restr
     }
 }
 
+// Whether c = c0 + d mod L of rm_position can be turned round to the d of a
+// circle position (rm_combine).  A limited buffer that ends inside a long filler
+// can have its start position past the circle's end (c0 > L); the passes
+// over memory take it as it is.
+__device__ __forceinline__ bool circle_inverts(const rm_geometry& g)
+{
+    return g.L <= 0 || (g.Kd >= 0 && g.c0 >= 0 && g.c0 <= g.L);
+}
+
 // Output positions from the staged LLRs: out[0, 2Zc) punctured, the circular
 // buffer after it.  Circle position c holds LLRs d, d + L, ... < E, d = (c -
 // c0) mod L.  A group of 16 bytes that is a run of consecutive d, all
@@ -170,10 +180,22 @@ __device__ __forceinline__ void rm_combine(TO* __restrict__ out, const TO* __res
     }
 }
 
+// Bytes of dynamic LDS that this launch got: hidden_dynamic_lds_size of the
+// implicit kernel arguments (code object version 5 and later).  Not taken from
+// the descriptor, which a caller may set up again for other TBs under a
+// kernel node that keeps the size of its own setup.
+__device__ __forceinline__ uint32_t launch_lds_bytes()
+{
+    constexpr int OFFSET = 120;
+    typedef const __attribute__((address_space(4))) uint32_t* arg_words;
+    return ((arg_words)__builtin_amdgcn_implicitarg_ptr())[OFFSET / 4];
+}
+
 template <typename TI, typename TO, bool DESCR>
 __global__ __launch_bounds__(RM_BLOCK) void derate_match_kernel(const rm_descriptor* __restrict__ desc)
 {
     extern __shared__ __align__(16) unsigned char rm_lds[];
+    __shared__ uint32_t seq_part[DESCR ? RM_SEQ_PART_WORDS : 1];
     const int cb_in_tb = blockIdx.x;
     const int tb_slot = blockIdx.y;
     const uint16_t ue = desc->sch_user_idxs[tb_slot];
@@ -184,52 +206,70 @@ __global__ __launch_bounds__(RM_BLOCK) void derate_match_kernel(const rm_descrip
     const TI* in = static_cast<const TI*>(desc->llr_in[tb_slot]);
     const rm_geometry g = rm_geometry_of(p, cb_in_tb);
 
-    // descrambling: words of c covering the CB's bits [start, start + E), and one more
-    const uint32_t lds_words = (uint32_t)desc->lds_bytes / 4u;
-    uint32_t* const seq = reinterpret_cast<uint32_t*>(rm_lds);
+    // descrambling: nw words of c, from w_first on, cover the CB's bits [start, start + E)
+    const uint32_t lds_words = launch_lds_bytes() / 4u;
+    uint32_t* seq = reinterpret_cast<uint32_t*>(rm_lds);
     const bool descr = DESCR && !g.uci;
-    uint32_t nw = 0;
-    if (descr) {
-        const uint32_t w_base = (uint32_t)g.start >> 5;
-        nw = min(((uint32_t)(g.start + g.E - 1) >> 5) - w_base + 1u, lds_words - 1u);
-        if (threadIdx.x < 64) {
-            gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w_base, (int)nw, seq);
+    const uint32_t w_first = (uint32_t)g.start >> 5;
+    const uint32_t nw = (descr && g.E > 0) ? ((uint32_t)(g.start + g.E - 1) >> 5) - w_first + 1u : 0u;
+    // (by one wave)
+    const auto make_words = [&](uint32_t w, uint32_t n) {
+        if (threadIdx.x < 64) gold_words_wave((uint32_t)__builtin_amdgcn_readfirstlane((int)p.cinit), w, (int)n, seq);
+    };
+    const uint32_t seq_words = descr ? (nw + 1u + 3u) & ~3u : 0u;  // one more word; the LLRs follow, 16-byte aligned
+    if (rm_staged_fits(g.E, (int)sizeof(TO), seq_words, lds_words) && circle_inverts(g)) {
+        if (descr) {
+            make_words(w_first, nw);
             if (threadIdx.x == 0) seq[nw] = 0u;
+            __syncthreads();
         }
-        __syncthreads();
-        nw = (nw + 1u + 3u) & ~3u;  // the LLRs follow, 16-byte aligned
-    }
-    if (rm_staged_fits(g.E, (int)sizeof(TO), nw, lds_words)) {
-        TO* const llr = reinterpret_cast<TO*>(seq + nw);
+        TO* const llr = reinterpret_cast<TO*>(seq + seq_words);
         rm_stage<TI, TO, DESCR>(llr, in, g, p, descr, seq);
         __syncthreads();
         rm_combine<TO>(out, llr, g);
         return;
     }
 
-    // LLRs beyond the LDS: passes of distinct positions over memory
+    // LLRs beyond the LDS: passes of distinct positions over memory, each in as
+    // many parts as the sequence takes to fit (one with the setup's own LDS)
     TO* cbuf = out + 2 * g.Zc;
-    const uint32_t w_first = (uint32_t)g.start >> 5;
+    uint32_t part_words = lds_words;
+    if (DESCR && lds_words < (uint32_t)RM_SEQ_PART_WORDS) {
+        seq = seq_part;
+        part_words = RM_SEQ_PART_WORDS;
+    }
+    const uint32_t nparts = DESCR && nw > part_words ? (nw + part_words - 1u) / part_words : 1u;
     const int npass = rm_num_passes(g);
     for (int pass = 0; pass < npass; ++pass) {
         const int i0 = pass * g.L;
         const int span = g.ndi && pass == 0 ? g.L : min(g.L, g.E - i0);
-        for (int d = threadIdx.x; d < span; d += blockDim.x) {
-            const int i = i0 + d;  // index in the de-interleaved sequence
-            const int o = rm_position(g, d);
-            if (i >= g.E) {  // ndi = 1, first pass: selected-bit positions not transmitted
-                cbuf[o] = (TO)0.0f;
-                continue;
+        for (uint32_t part = 0; part < nparts; ++part) {
+            const uint32_t w0 = part * part_words;
+            if (descr && (nparts > 1u || pass == 0)) {  // (after the barrier that ends the part before)
+                make_words(w_first + w0, min(part_words, nw - w0));
+                __syncthreads();
             }
-            TO v = rm_num<TO>::clamp(cvt_llr<TO, TI>(in[rm_input_index(g, p, i)]));
-            if (descr) {
-                const uint32_t n = (uint32_t)rm_tx_position(g, i) - (w_first << 5);
-                if ((seq[min(n >> 5, lds_words - 1u)] >> (n & 31u)) & 1u) v = -v;
+            for (int d = threadIdx.x; d < span; d += blockDim.x) {
+                const int i = i0 + d;  // index in the de-interleaved sequence
+                const int o = rm_position(g, d);
+                if (i >= g.E) {  // ndi = 1, first pass: selected-bit positions not transmitted
+                    if (part == 0) cbuf[o] = (TO)0.0f;
+                    continue;
+                }
+                bool flip = false;
+                if (descr) {
+                    const uint32_t n = (uint32_t)rm_tx_position(g, i) - (w_first << 5);
+                    const uint32_t w = (n >> 5) - w0;
+                    if (w >= part_words) continue;  // in another part
+                    flip = ((seq[w] >> (n & 31u)) & 1u) != 0;
+                }
+                TO v = rm_num<TO>::clamp(cvt_llr<TO, TI>(in[rm_input_index(g, p, i)]));
+                if (flip) v = -v;
+                const TO prev = (g.ndi && pass == 0) ? (TO)0.0f : cbuf[o];
+                cbuf[o] = rm_num<TO>::clamp(prev + v);
             }
-            const TO prev = (g.ndi && pass == 0) ? (TO)0.0f : cbuf[o];
-            cbuf[o] = rm_num<TO>::clamp(prev + v);
+            __syncthreads();
         }
-        __syncthreads();
     }
     if (g.ndi) {
         for (int n = threadIdx.x; n < g.F; n += blockDim.x) cbuf[g.Kd + n] = (TO)LLR_MAX_ABS;
@@ -267,7 +307,7 @@ int rm_lds_bytes(int fpconfig, const uint32_t* max_e, int n, bool descrambling)
         const uint32_t e = std::min(max_e[i], (uint32_t)RM_MAX_DESCR_E);
         // a CB's bits start anywhere in a word; one more word; 16-byte units
         const int seq = descrambling ? (int)(((31u + e) / 32u + 2u + 3u) & ~3u) : 0;
-        const int limit = RM_LDS_LIMIT / 4;
+        const int limit = (RM_LDS_LIMIT - (descrambling ? 4 * RM_SEQ_PART_WORDS : 0)) / 4;
         const int need = rm_staged_fits((int)e, elem, (uint32_t)seq, (uint32_t)limit)
                              ? seq + ((int)e * elem + 3) / 4
                              : seq;

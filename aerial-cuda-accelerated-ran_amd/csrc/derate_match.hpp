@@ -15,7 +15,6 @@ struct rm_descriptor {
     void** out;                               // HARQ buffer of each UE index
     const PerTbParams* tb_prms;               // device copy, indexed by UE index
     int descrambling_on;
-    int lds_bytes;                            // dynamic LDS of the launch (rm_lds_bytes)
 };
 
 // Kernel of a FP configuration (0: fp32->fp32, 1: fp16->fp32, 2: fp32->fp16,
@@ -24,7 +23,7 @@ void* rm_kernel(int fpconfig, bool descrambling);
 void* rm_noop_kernel();
 
 constexpr unsigned RM_BLOCK = 256;
-// Descrambling sequence words per CB held in LDS (48 KB): E up to
+// Descrambling sequence words per CB that fit in LDS (48 KB): E up to
 // 32 * (RM_SEQ_WORDS - 1) = 393,184 rate-matched bits per CB (a CB's bits
 // may start anywhere in a word).
 constexpr int RM_SEQ_WORDS = 12288;
@@ -32,8 +31,11 @@ constexpr int RM_MAX_DESCR_E = 32 * (RM_SEQ_WORDS - 1);
 
 // Dynamic LDS of a launch whose TBs have at most max_e[i] bits per CB: each
 // CB's descrambling words and, up to RM_LDS_LIMIT bytes in all (the size a
-// kernel gets without asking for more), its LLRs.
+// kernel gets without asking for more), its LLRs.  The kernel looks at the
+// size its launch really has; with less it makes the sequence in parts, at
+// least RM_SEQ_PART_WORDS words each.
 constexpr int RM_LDS_LIMIT = 64 * 1024;
+constexpr int RM_SEQ_PART_WORDS = 256;
 int rm_lds_bytes(int fpconfig, const uint32_t* max_e, int n, bool descrambling);
 
 // Whether a CB of E LLRs of `elem` bytes fits after seq_words words.

@@ -391,3 +391,153 @@ def test_derate_match_edges(case, fp, descr):
         assert np.array_equal(got[:, :n].view(np.uint32), exp[:, :n].view(np.uint32)), tx
         assert np.all(got[:, n:] == 55.0), "padding written"
     rm.close()
+
+
+# ---------------------------------------------------------------------------
+# de-rate-matching: the launch's LDS and the descriptor need not be of one setup
+# ---------------------------------------------------------------------------
+class _RmSetup:
+    """One descriptor (host and device) that setups are written to; setup()
+    gives the launch configuration, whose node is launched by the caller."""
+
+    def __init__(self, fp, descr):
+        import ctypes as C
+        from aerial_amd import _lib as L
+        from aerial_amd.pusch import DeRateMatch
+        self.C, self.L = C, L
+        self.rm = DeRateMatch(fp_config=fp, descrambling=descr)
+        n, al = C.c_size_t(), C.c_size_t()
+        L.check("info", L.lib().cuphyPuschRxRateMatchGetDescrInfo(C.byref(n), C.byref(al)))
+        self.host = (C.c_uint8 * n.value)()
+        self.dev = torch.zeros(n.value, dtype=torch.uint8, device="cuda")
+        self.prms = torch.zeros(64 * C.sizeof(L.PerTbParams), dtype=torch.uint8, device="cuda")
+        self.outs = torch.zeros(64, dtype=torch.int64, device="cuda")
+
+    def setup(self, params, xs, harqs):
+        from aerial_amd.decoder import _stream_handle
+        C, L, n = self.C, self.L, len(params)
+        arr = (L.PerTbParams * n)(*params)
+        raw = np.frombuffer(bytes(arr), np.uint8).copy()
+        self.prms[:raw.size].copy_(torch.from_numpy(raw))
+        self.outs[:n].copy_(torch.tensor([h.data_ptr() for h in harqs], dtype=torch.int64))
+        tin = (L.TensorPrm * n)()
+        for t, x in zip(tin, xs):
+            t.pAddr = x.data_ptr()
+        cfg = L.RateMatchLaunchCfg()
+        L.check("setup", L.lib().cuphySetupPuschRxRateMatch(
+            self.rm.h, n, (C.c_uint16 * n)(*range(n)), arr, C.c_void_p(self.prms.data_ptr()), tin, tin,
+            C.cast(C.c_void_p(self.outs.data_ptr()), C.POINTER(C.c_void_p)), C.cast(self.host, C.c_void_p),
+            C.c_void_p(self.dev.data_ptr()), 1, C.c_void_p(C.addressof(cfg)), _stream_handle(None)))
+        torch.cuda.synchronize()
+        return cfg
+
+    @staticmethod
+    def launch(cfg, shared=None):
+        from aerial_amd import _hip
+        from aerial_amd.decoder import _stream_handle
+        node = cfg.kernelNodeParamsDriver
+        if shared is not None:
+            node.sharedMemBytes = shared
+        _hip.launch_node(node, _stream_handle(None))
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("fp,descr", [(3, False), (3, True), (0, False), (0, True)])
+def test_derate_match_descriptor_set_up_again(fp, descr, graph):
+    """The node of a setup with short CBs launched (or captured and replayed)
+    after the descriptor was set up again for longer ones: the launch keeps
+    its own, smaller LDS."""
+    _need_gpu()
+    from aerial_amd.pusch import make_tb_params
+    print("[case] derate descriptor set up again fp=%d descr=%d graph=%d" % (fp, descr, graph), flush=True)
+    half = fp == 3
+    dt = torch.float16 if half else torch.float32
+    s = _RmSetup(fp, descr)
+    small = [make_tb_params(2, 20, 3, 160, 2, 1, 3 * 200, 0)[0]]
+    big, xs, harqs, refs = [], [], [], []
+    for u, (E, rv) in enumerate([(9088, 0), (24008, 2), (200, 1)]):
+        p, _ = make_tb_params(1, 384, 2, 8448, 8, 1, 2 * E, rv, user_group=u)
+        p.cinit = (0x5A3C7 * (u + 3)) if descr else 0
+        llr = tb_llrs(2 * E, 300 + u)
+        if half:
+            llr = llr.astype(np.float16).astype(np.float32)
+        ref = np.zeros(2 * p.Ncb_padded, np.float32)
+        O.derate_match(O.rm_cfg(bg=1, Zc=384, C=2, Qm=8, Nl=1, G=2 * E, K=p.K, F=p.F, Ncb=p.Ncb,
+                                Ncb_padded=p.Ncb_padded, k0=p.k0, ndi=1, descramble=int(descr), cinit=p.cinit),
+                       llr, ref, fp16=half)
+        big.append(p)
+        xs.append(torch.from_numpy(qam_stride_layout(llr, 8, 1, 1, [0])).cuda().to(dt))
+        harqs.append(torch.full((2 * p.Ncb_padded,), 9.0, dtype=dt, device="cuda"))
+        refs.append(ref)
+    x0 = torch.zeros(3 * 100 * 8, dtype=dt, device="cuda")
+    h0 = torch.zeros(3 * small[0].Ncb_padded, dtype=dt, device="cuda")
+    cfg = s.setup(small * 3, [x0] * 3, [h0] * 3)  # three TBs of three CBs: the grid covers what follows
+    assert cfg.kernelNodeParamsDriver.sharedMemBytes < 2000
+    if graph:
+        s.launch(cfg)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            s.launch(cfg)
+    s.setup(big, xs, harqs)
+    for _ in range(2):
+        for h in harqs:
+            h.fill_(9.0)
+        if graph:
+            g.replay()
+        else:
+            s.launch(cfg)
+        torch.cuda.synchronize()
+        for u, (p, h, ref) in enumerate(zip(big, harqs, refs)):
+            n = 2 * p.Zc + p.Ncb
+            got = h.float().cpu().numpy().reshape(2, -1)[:, :n]
+            assert np.array_equal(got.view(np.uint32), ref.reshape(2, -1)[:, :n].view(np.uint32)), u
+
+
+@pytest.mark.parametrize("fp,descr", [(3, False), (3, True), (0, True), (1, False), (2, True)])
+def test_derate_match_staged_equals_passes(fp, descr):
+    """Drawn geometries (limited buffers that end anywhere, start positions
+    anywhere in them, fillers of any length, repetition): the staged form
+    and, with no LDS for the LLRs, the passes over memory write the same."""
+    _need_gpu()
+    from aerial_amd.pusch import make_tb_params
+    print("[case] derate staged against passes fp=%d descr=%d" % (fp, descr), flush=True)
+    rng = np.random.RandomState(100 * fp + descr)
+    ti, to = (torch.float16 if fp in (1, 3) else torch.float32), (torch.float16 if fp in (2, 3) else torch.float32)
+    s = _RmSetup(fp, descr)
+    for i in range(60):
+        bg, Zc = int(rng.randint(1, 3)), int(rng.choice([2, 5, 13, 36, 104]))
+        ns, N = (22, 66 * Zc) if bg == 1 else (10, 50 * Zc)
+        Kp = int(rng.randint(2 * Zc + 1, ns * Zc + 1))
+        short = i % 6 == 0  # a short circle, and the start position past its end
+        if short:
+            Kp = (ns + 2) * Zc // 2
+        F = ns * Zc - Kp
+        Qm, Nl, C = int(rng.choice([1, 2, 4, 6, 8])), int(rng.choice([1, 2])), int(rng.randint(1, 4))
+        p, _ = make_tb_params(bg, Zc, C, Kp, Qm, Nl, C * Qm * Nl * int(rng.randint(1, 2 + 3 * N // (Qm * Nl))), 0,
+                              ndi=int(rng.randint(2)))
+        p.Ncb = int(rng.randint(F + 1, N + 1))
+        p.k0 = int(rng.randint(p.Ncb))
+        if short:
+            p.Ncb, p.k0 = F + max(1, Zc), Kp - 2 * Zc - 1
+        p.Ncb_padded = (2 * Zc + N + 7) // 8 * 8
+        p.cinit = int(rng.randint(1 << 31)) if descr else 0
+        x = (torch.from_numpy(tb_llrs(max(50, 8 * p.encodedSize // Qm), i)).cuda()).to(ti)
+        start = torch.from_numpy(rng.uniform(-50, 50, C * p.Ncb_padded).astype(np.float32)).cuda().to(to)
+        got = []
+        for shared in (None, 0):
+            h = start.clone()
+            s.launch(s.setup([p], [x], [h]), shared)
+            torch.cuda.synchronize()
+            got.append(h.cpu().numpy())
+        assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8)), (i, bg, Zc, Kp, Qm, Nl, C, p.Ncb, p.k0)
+
+
+@pytest.mark.parametrize("fp,descr", [(3, False), (3, True), (0, False), (0, True)])
+@pytest.mark.parametrize("past", [0, 1])
+def test_derate_match_lds_limit(fp, descr, past):
+    """The largest CB that is staged, and one symbol more."""
+    half, limit = fp == 3, 64 * 1024 // 4 - (256 if descr else 0)
+    E = max(e for e in range(8, 40000, 8)
+            if (((31 + e) // 32 + 5) // 4 * 4 if descr else 0) + (e * (2 if half else 4) + 3) // 4 <= limit)
+    test_derate_match_edges((1, 384, 1, 8448, 8, 1, E + 8 * past, 2, 0, 0), fp, descr)
