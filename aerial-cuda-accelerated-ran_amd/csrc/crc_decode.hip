@@ -20,16 +20,19 @@
 //
 // One wave per code block, four to a workgroup (they share the TB's step
 // table in LDS); the TB's bytes go out as aligned words, each assembled from
-// two decoded words, with single bytes only at a block's ends.  The TB kernel
-// gives each TB CRC_TB_PARTS workgroups, whose remainders meet in an XOR in the
-// descriptor (one workgroup reads 147 KB at 18 us, whatever its loads in flight).
-// The offsets of a TB are sums over the TBs before it, taken by the lanes of
-// the wave.  Both kernels are bound by their dependent loads (descriptor,
-// parameters, words), not by the 2 KB per code block.  Measured on 20 TBs of
-// 140 BG1 Zc = 384 code blocks, against contiguous chunks per thread with byte
-// tables in global memory, one loop over the TBs before and byte stores: CB
-// kernel 30 -> 9 us, TB kernel 73 -> 10 us (both with about 4 us that an empty
-// kernel measures the same way).
+// two decoded words, with single bytes only at a block's ends.  The offsets
+// of a TB are sums over the TBs before it, taken by the lanes of the wave.
+// The TB kernel gives each TB one workgroup, so that launches share no state
+// and a setup's nodes may run on several streams at once (16 workgroups per
+// TB, whose remainders met in the descriptor, took 10 us, but only one launch at
+// a time was right).  16 waves: 147 KB in L2 take 18 us with 4, 13.6 with 8, 8.3
+// with 16; bound by the four table reads per word (copies of the table against
+// bank conflicts, 8 to 32: 8.7 to 9.3) and, on bytes that the CB kernel just
+// wrote, by their way from other XCDs (more loads in flight: no change).
+// Measured on 20 TBs of 140 BG1 Zc = 384 code blocks, against contiguous chunks
+// per thread with byte tables in global memory, one loop over the TBs before and
+// byte stores: CB kernel 30 -> 9 us, TB kernel 73 -> 18 us (both with about 4 us
+// that an empty kernel measures the same way).
 #include "crc_core.hpp"
 #include "crc_decode.hpp"
 
@@ -117,7 +120,7 @@ __global__ __launch_bounds__(CRC_CB_BLOCK) void crc_cb_kernel(const crc_descript
     }
 }
 
-__global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(crc_descriptor* __restrict__ desc)
+__global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(const crc_descriptor* __restrict__ desc)
 {
     __shared__ uint32_t table[4][256];
     __shared__ uint32_t red[CRC_TB_BLOCK / 64];
@@ -132,38 +135,20 @@ __global__ __launch_bounds__(CRC_TB_BLOCK) void crc_tb_kernel(crc_descriptor* __
     const int Kp = (int)(p.K - p.F);
     const int data_bytes = (Kp - 24 + 7) / 8;
     const int nw = ((int)p.num_CBs * data_bytes + 3) / 4;
-    // this workgroup's words [w0, w1) of the TB
-    const int per = (nw + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int w0 = min(nw, per * (int)blockIdx.y), w1 = min(nw, w0 + per);
-    const uint32_t* tbw = reinterpret_cast<const uint32_t*>(d.tb_out + l.tb_byte_base) + w0;
+    const uint32_t* tbw = reinterpret_cast<const uint32_t*>(d.tb_out + l.tb_byte_base);
     __syncthreads();
     const uint32_t v = wave_sum_products<24>(
         (uint32_t)t & 63u,
         strided_crc<CRC_TB_BLOCK>(
-            w1 - w0, t, [&](int w) { return __builtin_bswap32(tbw[w]); },
+            nw, t, [&](int w) { return __builtin_bswap32(tbw[w]); },
             [&](int b, uint32_t x) { return table[b][x]; }),
         last, fold);
     if ((t & 63) == 0) red[t >> 6] = v;
     __syncthreads();
-    if (t >= 64) return;
+    if (t != 0) return;
     uint32_t crc = 0;
     for (int i = 0; i < (int)(CRC_TB_BLOCK / 64); ++i) crc ^= red[i];
-    // shifted by the words after the part
-    const uint32_t n = 4u * (uint32_t)(nw - w1);
-    crc = wave_mulmod24((uint32_t)t, crc,
-                        wave_mulmod24((uint32_t)t, g_crc_shift.lo[K_CRC24A][n & 1023u],
-                                      g_crc_shift.tb_hi[(n >> 10) & 255u], fold),
-                        fold);
-    if (t != 0) return;
-    // XORed into the TB's accumulator before the part is counted; the last
-    // part takes the sum and puts both words back to zero
-    uint32_t prev = __hip_atomic_fetch_xor(&desc->tb_acc[slot], crc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("" : "+v"(prev) : : "memory");
-    if (__hip_atomic_fetch_add(&desc->tb_parts[slot], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
-        gridDim.y - 1u)
-        return;
-    d.tb_crc_out[slot] = __hip_atomic_exchange(&desc->tb_acc[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(&desc->tb_parts[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    d.tb_crc_out[slot] = crc;
 }
 
 void* crc_cb_kernel_ptr() { return (void*)&crc_cb_kernel; }

@@ -19,10 +19,6 @@ struct crc_descriptor {
     uint32_t* tb_crc_out;        // one remainder per transport block
     const PerTbParams* tb_prms;  // device copy, indexed by UE index
     int reverse_bytes;
-    // TB kernel: XOR of the parts' remainders and count of finished parts of
-    // each slot; zero between launches (the last part puts them back)
-    uint32_t tb_acc[MAX_N_TBS_SUPPORTED];
-    uint32_t tb_parts[MAX_N_TBS_SUPPORTED];
 };
 
 void* crc_cb_kernel_ptr();
@@ -30,8 +26,6 @@ void* crc_tb_kernel_ptr();
 
 constexpr int CRC_CBS_PER_BLOCK = 4;  // code blocks (waves) per workgroup of the CB kernel
 constexpr unsigned CRC_CB_BLOCK = 64 * CRC_CBS_PER_BLOCK;
-constexpr unsigned CRC_TB_BLOCK = 256;
-// Workgroups per TB of the TB kernel (grid y), each a run of the TB's words.
-constexpr unsigned CRC_TB_PARTS = 16;
+constexpr unsigned CRC_TB_BLOCK = 1024;
 
 }  // namespace nrldpc

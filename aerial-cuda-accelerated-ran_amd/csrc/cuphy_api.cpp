@@ -649,8 +649,6 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxCrcDecode(cuphyPuschRxCrcDecodeHndl_t
     d.tb_crc_out = pOutputTBCRCs;
     d.tb_prms = pTbPrmsGpu;
     d.reverse_bytes = o.reverse_bytes;
-    std::memset(d.tb_acc, 0, sizeof(d.tb_acc));
-    std::memset(d.tb_parts, 0, sizeof(d.tb_parts));
     if (enableCpuToGpuDescrAsyncCpy &&
         hipMemcpyAsync(pGpuDesc, pCpuDesc, sizeof(nrldpc::crc_descriptor), hipMemcpyHostToDevice, strm) != hipSuccess)
         return CUPHY_STATUS_MEMCPY_ERROR;
@@ -663,8 +661,7 @@ cuphyStatus_t CUPHYWINAPI cuphySetupPuschRxCrcDecode(cuphyPuschRxCrcDecodeHndl_t
              pCbCrcLaunchCfg->kernelArgs);
     pTbCrcLaunchCfg->desc = pGpuDesc;
     pTbCrcLaunchCfg->kernelArgs[0] = &pTbCrcLaunchCfg->desc;
-    set_node(pTbCrcLaunchCfg->kernelNodeParamsDriver, nrldpc::crc_tb_kernel_ptr(),
-             dim3(std::max<unsigned>(1, nSchUes), nrldpc::CRC_TB_PARTS),
+    set_node(pTbCrcLaunchCfg->kernelNodeParamsDriver, nrldpc::crc_tb_kernel_ptr(), dim3(std::max<unsigned>(1, nSchUes)),
              dim3(nrldpc::CRC_TB_BLOCK), pTbCrcLaunchCfg->kernelArgs);
     return CUPHY_STATUS_SUCCESS;
 }

@@ -541,3 +541,44 @@ def test_derate_match_lds_limit(fp, descr, past):
     E = max(e for e in range(8, 40000, 8)
             if (((31 + e) // 32 + 5) // 4 * 4 if descr else 0) + (e * (2 if half else 4) + 3) // 4 <= limit)
     test_derate_match_edges((1, 384, 1, 8448, 8, 1, E + 8 * past, 2, 0, 0), fp, descr)
+
+
+def test_crc_decode_launches_overlap():
+    """The nodes of one setup launched many times on two streams at once:
+    launches share no state, so each gives the TBs' CRCs."""
+    _need_gpu()
+    from aerial_amd import _hip
+    from aerial_amd.decoder import _stream_handle
+    from aerial_amd.pusch import CrcDecode, make_tb_params
+    rng = np.random.RandomState(5)
+    shapes = [(152, 8448), (3, 8448), (2, 40), (1, 3000), (40, 8424)]
+    print("[case] crc overlapping launches, %d TBs" % len(shapes), flush=True)
+    params, words, refs = [], [], []
+    for C, Kp in shapes:
+        bg, Zc = (1, 384) if Kp > 3840 else (2, 384)
+        params.append(make_tb_params(bg, Zc, C, Kp, 2, 1, C * 4000, 0)[0])
+        w = rng.randint(0, 1 << 32, (C, O.WORDS_PER_CB), dtype=np.uint64).astype(np.uint32)
+        w[:, (Kp + 31) // 32:] = 0
+        if Kp % 32:
+            w[:, Kp // 32] &= np.uint32((1 << (Kp % 32)) - 1)
+        words.append(w)
+        refs.append(O.crc_desegment(w.reshape(-1), C, Kp))
+    want = np.array([r[2] for r in refs], np.uint32)
+    cb_crc = torch.zeros(sum(C for C, _ in shapes), dtype=torch.int32, device="cuda")
+    tb_crc = torch.zeros(len(shapes), dtype=torch.int32, device="cuda")
+    tb_bytes = torch.zeros(sum(len(r[1]) for r in refs) + 64, dtype=torch.uint8, device="cuda")
+    crc = CrcDecode()
+    crc.run(params, torch.from_numpy(np.concatenate(words).reshape(-1).view(np.int32).copy()).cuda(), cb_crc,
+            tb_bytes, tb_crc)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for _ in range(5):
+        tb_crc.fill_(-1)
+        torch.cuda.synchronize()
+        for _ in range(20):
+            for s in streams:
+                _hip.launch_node(crc.cb_cfg.kernelNodeParamsDriver, _stream_handle(s))
+                _hip.launch_node(crc.tb_cfg.kernelNodeParamsDriver, _stream_handle(s))
+        torch.cuda.synchronize()
+        assert np.array_equal(tb_crc.cpu().numpy().view(np.uint32), want)
+    crc.close()
