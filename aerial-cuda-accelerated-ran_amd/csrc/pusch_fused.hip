@@ -507,13 +507,14 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
 // when count > 1); descrambling words follow the last array.  Steps 1-3
 // run CB by CB with the whole workgroup; the decode runs the group side by
 // side (lanes [c * Zc, (c + 1) * Zc) of each lane group on CB c, each CB stopping
-// on its own syndrome: results as decoded alone); hard decisions and CRCs again CB by
-// CB.  Returns, in the completing thread, the XOR of the CBs' shares of the TB
-// CRC24A (each the remainder of the CB's payload bytes shifted to their
-// place in the TB; for a one-CB TB its CRC, which is the TB CRC), or
-// TB_ACC_ERROR when the group's parameters do not fit the launch (then only
-// the error marker is written, into the CBs' CRCs).  The TB CRC itself is
-// written by complete_cb.  GROUPED = false: the one-CB form (count = 1 at
+// on its own syndrome: results as decoded alone); hard decisions, CRCs and TB
+// bytes as tasks of the waves.  A CB's share of the TB CRC24A (the remainder of
+// its payload bytes shifted to their place in the TB) goes into the TB's
+// accumulator here; xor_prev holds the old values that thread 0's shares
+// found there.  Returns TB_ACC_ERROR when the group's parameters do not fit the
+// launch (then only the error marker is written, into the CBs' CRCs), else, in
+// the completing thread, a CB CRC: the TB CRC of a one-CB TB.  The TB CRC itself
+// is written by complete_cb.  GROUPED = false: the one-CB form (count = 1 at
 // compile time, no group state; an item of several CBs is rejected).
 template <typename TI, int MAXR, bool GROUPED, int PAIR>
 __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused_lds& sh,
@@ -626,9 +627,11 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
             const uint32_t share = tb_share_of(sh, words, tail, cb0 + c);
             // into the TB's accumulator now, so that the atomic's round trip
             // overlaps the other tasks (complete_cb raises the TB's count)
+            // (a wave of a group can have several shares: every old value is kept,
+            // so that the wait below covers each of them)
             if (lane0)
-                prev = __hip_atomic_fetch_xor(tbw + 2u * job.share_offset, share, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
+                prev |= __hip_atomic_fetch_xor(tbw + 2u * job.share_offset, share, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
         } else if (what == 1) {
             result = cb_crc_of(sh, words, tail);
             if (lane0) {
@@ -645,7 +648,7 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
         if (one) break;
     }
     // the other waves' shares are in the accumulator (their old values
-    // returned) before the caller's barrier; wave 0 hands its own on
+    // returned) before the caller's barrier; wave 0 hands its own ones on
     if (GROUPED && wave > 0) asm volatile("" : : "v"(prev) : "memory");
     xor_prev = prev;
     return result;
@@ -654,9 +657,9 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
 // Workspace words of a TB (after the queue words): TB-CRC accumulator at
 // 2 * share_offset, count of finished CBs at 2 * share_offset + 1.  Called
 // by one thread once the whole workgroup has finished a group of n CBs of
-// the TB (all of their outputs issued).  v: the XOR of the group's shares
-// (TB_ACC_ERROR: rejected group); for C > 1 and an accepted group, the
-// shares are already in the accumulator and xor_prev is its old value.
+// the TB (all of their outputs issued).  v: the TB CRC of a one-CB TB
+// (TB_ACC_ERROR: rejected group); for C > 1 and an accepted group, the shares
+// are in the accumulator once xor_prev, the old values found there, has returned.
 __device__ __forceinline__ void complete_cb(const cuphyHipPuschSlotTb_t& job, uint32_t C, uint32_t v, uint32_t n,
                                             uint32_t* __restrict__ tbw, uint32_t xor_prev)
 {

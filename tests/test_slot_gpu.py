@@ -342,3 +342,15 @@ def test_slot_rejects_cb_beyond_variant(dec):
     assert (tb.cb_crc.cpu().numpy().view(np.uint32) == L.SLOT_CB_ERROR).all()
     assert int(tb.tb_crc.cpu().numpy().view(np.uint32)[0]) == L.SLOT_CB_ERROR
     assert int(ln.workspace.abs().sum().item()) == 0
+
+
+# Work items of 16 code blocks of multi-CB TBs: more shares and CRCs than a
+# workgroup has waves, payloads of 23, 31 and 62 bytes (a block's last word filled
+# up past its place in the TB), and a last item with fewer blocks.
+GROUP_TAILS = [(2, 24, 37, 208, 2, 1, 1, 600, 0.5), (2, 24, 18, 240, 2, 1, 1, 400, 1.0),
+               (1, 24, 33, 520, 4, 1, 1, 1200, 0.5), (1, 16, 32, 272, 2, 1, 1, 360, 4.0)]
+
+
+@pytest.mark.parametrize("dtype", ["int8", "fp16"])
+def test_slot_large_groups_match_oracle(dec, dtype):
+    run_slot(dec, dtype, True, specs=GROUP_TAILS)
