@@ -37,6 +37,32 @@ class UploadBlock:
         self._dev.copy_(self._host, non_blocking=True)
 
 
+class _OnStream:
+    def __init__(self, stream):
+        self._stream = stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(stream.cuda_stream)
+        self._ctx = torch.cuda.stream(self._stream)
+
+    def __enter__(self):
+        capturing, before = torch.cuda.is_current_stream_capturing(), torch.cuda.current_stream()
+        self._ctx.__enter__()
+        if before != self._stream and not capturing and not torch.cuda.is_current_stream_capturing():
+            self._stream.wait_stream(before)
+        return self
+
+    def __exit__(self, *exc):
+        return self._ctx.__exit__(*exc)
+
+
 def on_stream(stream):
-    """Context in which blocks belong to the launching stream."""
-    return torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext()
+    """Context in which blocks belong to the launching stream.  What was queued
+    on the caller's current stream so far (the inputs' producers, the fill of an
+    output) comes before what is launched in it."""
+    return _OnStream(stream) if stream is not None else contextlib.nullcontext()
+
+
+def written_here(stream, tensor):
+    """Within on_stream(stream): `tensor`, allocated for the caller's current stream,
+    is written by the launching one; its memory is not handed out again before
+    that has run."""
+    if stream is not None and not torch.cuda.is_current_stream_capturing():
+        tensor.record_stream(torch.cuda.current_stream())

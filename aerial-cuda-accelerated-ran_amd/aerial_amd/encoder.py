@@ -16,7 +16,7 @@ import torch
 
 from . import _hip
 from . import _lib as L
-from ._upload import UploadBlock, on_stream
+from ._upload import UploadBlock, on_stream, written_here
 from .decoder import _stream_handle
 from .pusch import put_params, set_per_tb_params
 
@@ -85,7 +85,8 @@ class LdpcEncoder:
         nbits = (nsys + rows) * Z - (2 * Z if self.puncturing else 0)
         out_words = (nbits + 31) // 32
         # contiguous tensors of one allocation
-        outs = list(torch.empty((n, ncw, out_words), dtype=torch.int32, device="cuda").unbind(0))
+        whole = torch.empty((n, ncw, out_words), dtype=torch.int32, device="cuda")
+        outs = list(whole.unbind(0))
         tin = _BitTensor(in_words * 32, ncw, in_words * 32)
         tout = _BitTensor(out_words * 32, ncw, out_words * 32)
         in_ptrs = (C.c_void_p * n)(*[x.data_ptr() for x in info_words])
@@ -100,6 +101,7 @@ class LdpcEncoder:
             L.check("cuphySetupLDPCEncode", st)
             ws.send()
             _hip.launch_node(self.cfg.m_kernelNodeParams, sh)
+            written_here(stream, whole)
         self._ws = ws
         return outs
 
@@ -142,6 +144,7 @@ def dl_rate_match(params, coded_words, emax, scrambling=False, stream=None):
         blk.send()
         st = L.lib().cuphyHipDlRateMatch(blk.dev(0), n, blk.dev(1), max_cbs, emax, int(scrambling),
                                          C.c_void_p(out.data_ptr()), _stream_handle(stream))
+        written_here(stream, out)
     L.check("cuphyHipDlRateMatch", st)
     out._keep = blk  # the argument buffers live as long as the result
     return out

@@ -194,3 +194,52 @@ def test_dl_rate_match_edges(case):
         bits = words_to_bits(got[r], emax)
         assert np.array_equal(bits[:E], ref), (case, r)
         assert not bits[E:].any(), (case, r)
+
+
+def _busy():
+    """Keep the current stream busy for some milliseconds."""
+    a = torch.full((4096, 4096), 1e-4, device="cuda")
+    for _ in range(12):
+        a = a @ a
+    return a
+
+
+def test_calls_on_another_stream(enc):
+    """Inputs still being produced on the current stream, and outputs partly
+    filled there (TBs of different numbers of code blocks), when the calls are
+    launched on another stream."""
+    from aerial_amd.encoder import dl_rate_match
+    from aerial_amd.pusch import make_tb_params
+    print("[case] encoder and DL rate matching launched on another stream", flush=True)
+    rng = np.random.RandomState(3)
+    enc.puncturing = True
+    late, words, cws, params = [], [], [], []
+    for t, C in enumerate((3, 1, 2)):
+        p, _ = make_tb_params(2, 52, C, 480, 2, 1, C * 600, 0)
+        p.cinit = 77 + t
+        params.append(p)
+        info = rng.randint(0, 2, (C, 520)).astype(np.uint8)
+        info[:, 480:] = 0
+        late.append(torch.from_numpy(np.stack([O.pack_bits(x) for x in info]).view(np.int32)).cuda())
+        words.append(torch.zeros_like(late[-1]))
+        cws.append([O.encode(2, 52, x)[104:104 + p.N] for x in info])
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for w in words:
+            w.zero_()
+        keep = _busy()
+        for w, x in zip(words, late):
+            w.copy_(x)
+        coded = [enc.encode_words(2, 52, [w], stream=s)[0] for w in words]
+        s.synchronize()
+        keep = _busy()
+        coded = [c.clone() for c in coded]  # (on the current stream, after the work above)
+        out = dl_rate_match(params, coded, 640, scrambling=True, stream=s)
+        s.synchronize()
+        got = out.cpu().numpy()
+        for t, (p, cw) in enumerate(zip(params, cws)):
+            for r, ref in enumerate(dl_reference(p, cw, p.cinit, True)):
+                assert np.array_equal(words_to_bits(got[t, r], 640)[:ref.size], ref), (t, r)
+            assert (got[t, len(cw):] == -1).all()
+    del keep

@@ -582,3 +582,44 @@ def test_crc_decode_launches_overlap():
         torch.cuda.synchronize()
         assert np.array_equal(tb_crc.cpu().numpy().view(np.uint32), want)
     crc.close()
+
+
+def test_calls_on_another_stream():
+    """De-rate-matching and CRC launched on another stream while their inputs
+    are still being produced on the current one."""
+    _need_gpu()
+    from aerial_amd.pusch import CrcDecode, DeRateMatch, make_tb_params
+    print("[case] derate and crc launched on another stream", flush=True)
+    bg, Zc, C, Kp, Qm, Nl, E = 2, 104, 3, 1000, 4, 1, 1600
+    p, _ = make_tb_params(bg, Zc, C, Kp, Qm, Nl, C * E, 0, ndi=1)
+    llr = tb_llrs(C * E, 77)
+    ref = np.zeros(C * p.Ncb_padded, np.float32)
+    O.derate_match(O.rm_cfg(bg=bg, Zc=Zc, C=C, Qm=Qm, Nl=Nl, G=C * E, K=p.K, F=p.F, Ncb=p.Ncb,
+                            Ncb_padded=p.Ncb_padded, k0=p.k0, ndi=1), llr, ref)
+    w, kp = build_tb(3 * 976 - 24, 3, 78)  # K' = 1000
+    assert kp == Kp
+    cb_ref, bytes_ref, tb_ref = O.crc_desegment(w.reshape(-1), 3, kp)
+    late = (torch.from_numpy(qam_stride_layout(llr, Qm, Nl, Nl, [0])).cuda(),
+            torch.from_numpy(w.reshape(-1).view(np.int32).copy()).cuda())
+    x, words = torch.zeros_like(late[0]), torch.zeros_like(late[1])
+    harq = torch.zeros(C * p.Ncb_padded, device="cuda")
+    cb_crc, tb_crc = (torch.zeros(n, dtype=torch.int32, device="cuda") for n in (3, 1))
+    tb_bytes = torch.zeros(len(bytes_ref), dtype=torch.uint8, device="cuda")
+    rm, crc, s = DeRateMatch(fp_config=0), CrcDecode(), torch.cuda.Stream()
+    n = 2 * Zc + p.Ncb
+    for call in (lambda: rm.run([p], [x], [harq], stream=s),
+                 lambda: crc.run([p], words, cb_crc, tb_bytes, tb_crc, stream=s)):
+        torch.cuda.synchronize()
+        a = torch.full((4096, 4096), 1e-4, device="cuda")
+        for _ in range(12):
+            a = a @ a
+        x.copy_(late[0])
+        words.copy_(late[1])
+        call()
+        s.synchronize()
+    assert np.array_equal(harq.cpu().numpy().reshape(C, -1)[:, :n], ref.reshape(C, -1)[:, :n])
+    assert np.array_equal(cb_crc.cpu().numpy().view(np.uint32), cb_ref)
+    assert np.array_equal(tb_bytes.cpu().numpy(), bytes_ref)
+    assert int(tb_crc.cpu().numpy().view(np.uint32)[0]) == tb_ref
+    rm.close()
+    crc.close()
