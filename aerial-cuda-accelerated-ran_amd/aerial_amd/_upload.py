@@ -14,16 +14,21 @@ _ALIGN = 64
 
 
 class UploadBlock:
-    """Space for parts of the given sizes; part i at host(i) / dev(i)."""
+    """Space for parts of the given sizes; part i at host(i) / dev(i).
 
-    def __init__(self, sizes):
-        if torch.cuda.is_current_stream_capturing():
+    in_graph: may be used while the stream is being captured.  The graph's copy
+    then reads the host block at every replay, so the block is pageable memory of
+    its own, and whoever gets it keeps it (`captured`) as long as the graph may run."""
+
+    def __init__(self, sizes, in_graph=False):
+        self.captured = torch.cuda.is_current_stream_capturing()
+        if self.captured and not in_graph:
             raise RuntimeError("host parameters cannot be uploaded while the stream is being captured")
         self._off, n = [], 0
         for s in sizes:
             self._off.append(n)
             n += (s + _ALIGN - 1) // _ALIGN * _ALIGN
-        self._host = torch.empty(max(n, 1), dtype=torch.uint8, pin_memory=True)
+        self._host = torch.empty(max(n, 1), dtype=torch.uint8, pin_memory=not self.captured)
         self._dev = torch.empty(max(n, 1), dtype=torch.uint8, device="cuda")
         self._hptr, self._dptr = self._host.data_ptr(), self._dev.data_ptr()
 

@@ -71,6 +71,7 @@ class LdpcEncoder:
                 self._lib.cuphyLDPCEncodeGetDescrInfo(C.byref(dsz), C.byref(dal), max_tbs, C.byref(wsz)))
         self.cpu_desc = (C.c_uint8 * dsz.value)()  # (the kernel takes it by value)
         self._ws_bytes = wsz.value
+        self._graph_ws = []  # of captured calls: a graph's replays read them while the encoder lives
         self.cfg = L.LDPCEncodeLaunchConfig()
 
     def encode_words(self, bg, Z, info_words, num_rows=0, rv=0, stream=None):
@@ -92,7 +93,7 @@ class LdpcEncoder:
         in_ptrs = (C.c_void_p * n)(*[x.data_ptr() for x in info_words])
         out_ptrs = (C.c_void_p * n)(*[o.data_ptr() for o in outs])
         with on_stream(stream):
-            ws = UploadBlock((self._ws_bytes,))  # the TBs' addresses
+            ws = UploadBlock((self._ws_bytes,), in_graph=True)  # the TBs' addresses
             sh = _stream_handle(stream)
             st = self._lib.cuphySetupLDPCEncode(
                 C.byref(self.cfg), tin.h, None, tout.h, None, bg, Z, int(self.puncturing), num_rows, rv, 1, n,
@@ -102,7 +103,10 @@ class LdpcEncoder:
             ws.send()
             _hip.launch_node(self.cfg.m_kernelNodeParams, sh)
             written_here(stream, whole)
-        self._ws = ws
+        if ws.captured:
+            self._graph_ws.append(ws)
+        else:
+            self._ws = ws
         return outs
 
     def encode(self, code_blocks, tb_sizes, code_rates, redundancy_versions):

@@ -243,3 +243,34 @@ def test_calls_on_another_stream(enc):
                 assert np.array_equal(words_to_bits(got[t, r], 640)[:ref.size], ref), (t, r)
             assert (got[t, len(cw):] == -1).all()
     del keep
+
+
+def test_encode_words_captured():
+    """A captured call replays with the addresses it was captured with, also
+    after other calls of the same encoder."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from aerial_amd.encoder import LdpcEncoder
+    print("[case] encode_words under capture", flush=True)
+    enc = LdpcEncoder()
+    rng = np.random.RandomState(4)
+    x = [torch.from_numpy(rng.randint(0, 1 << 32, (3, 22 * 104 // 32 + 1), dtype=np.uint64).astype(np.uint32)
+                          .view(np.int32)).cuda() for _ in range(4)]
+    for t in x:
+        t[:, -1] &= (1 << (22 * 104 % 32)) - 1
+    want = [w.clone() for w in enc.encode_words(1, 104, x)]
+    graphs, outs = [], []
+    for k in (0, 2):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            o = enc.encode_words(1, 104, x[k:k + 2])
+        graphs.append(g)
+        outs.append(o)
+    for _ in range(3):
+        for k, g in zip((0, 2), graphs):
+            for o in outs[k // 2]:
+                o.zero_()
+            enc.encode_words(1, 104, x[3:])
+            g.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(o, w) for o, w in zip(outs[k // 2], want[k:k + 2]))
