@@ -274,3 +274,11 @@ def test_encode_words_captured():
             g.replay()
             torch.cuda.synchronize()
             assert all(torch.equal(o, w) for o, w in zip(outs[k // 2], want[k:k + 2]))
+
+
+def test_encode_words_results_are_aligned(enc):
+    """Each TB's words start on an address of their own, as separate tensors do
+    (9 words per TB here: viewed as bytes of any width)."""
+    print("[case] encode_words result alignment", flush=True)
+    outs = enc.encode_words(2, 5, [torch.zeros((1, 2), dtype=torch.int32, device="cuda")] * 5)
+    assert all(o.data_ptr() % 512 == 0 and o.is_contiguous() and o.storage_offset() % 4 == 0 for o in outs)
