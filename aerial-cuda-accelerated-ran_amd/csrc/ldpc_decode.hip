@@ -81,13 +81,11 @@ __global__ __launch_bounds__(768) void ldpc_layered_tb_pair(cuphyLDPCDecodeDesc_
 
 // The same with every edge's offset in a register (run_iterations PRE), for
 // workgroups whose waves have the registers for it: BG2 in binary16 holds 153,
-// three waves per SIMD; BG1 in binary16 254 and BG2 in binary32 207, two; BG1 in
-// binary32 278, one.  Used when every code block has a CU to itself; with more
-// code blocks the plain form's waves that share a CU hide each other's
-// latency.  Measured for 10 iterations, plain and this form: one code block BG2
-// Z = 64, 20 rows 53 and 48 us; eight BG1 Z = 128, 46 rows 119 and 107 us, in
-// binary32 151 (before explicit messages) and 135 us; eight BG2 Z = 384, 42 rows
-// 111 and 99 us; 256 BG1 Z = 128, 46 rows 122 and 110 us.
+// three waves per SIMD; BG1 in binary16 254 and BG2 in binary32 206, two; BG1 in
+// binary32 277, one.  Measured for 10 iterations, plain and this form: one code
+// block BG2 Z = 64, 20 rows 53 and 48 us; eight BG1 Z = 128, 46 rows 119 and 107
+// us, in binary32 151 (before explicit messages) and 135 us; eight BG2 Z = 384,
+// 42 rows 111 and 99 us; 256 BG1 Z = 128, 46 rows 122 and 110 us.
 template <int BG, typename T> constexpr int tb_pre_threads()
 {
     return sizeof(T) == 2 ? (BG == 2 ? 768 : 512) : (BG == 2 ? 512 : 256);
@@ -300,25 +298,22 @@ void* select_tb_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math)
     return nullptr;
 }
 
-// Row-pair kernel of a launch of `threads`-thread workgroups; own_cu: no more
-// workgroups than CUs.
-template <int BG, typename T, typename TIn> void* tb_pair_kernel(int threads, bool own_cu)
+// Row-pair kernels of a configuration; pre: nullptr where its launch bounds do
+// not take the workgroup.
+struct tb_pair_kernels {
+    void *full, *pre;
+};
+template <int BG, typename T, typename TIn> tb_pair_kernels tb_pair_kernels_of(int threads)
 {
-    return own_cu && threads <= tb_pre_threads<BG, T>() ? (void*)&ldpc_layered_tb_pair_pre<BG, T, TIn>
-                                                        : (void*)&ldpc_layered_tb_pair<BG, T, TIn>;
+    tb_pair_kernels k;
+    k.full = (void*)&ldpc_layered_tb_pair<BG, T, TIn>;
+    k.pre = threads <= tb_pre_threads<BG, T>() ? (void*)&ldpc_layered_tb_pair_pre<BG, T, TIn> : nullptr;
+    return k;
 }
-template <int BG> void* tb_pair_kernel_of(cuphyDataType_t llr_type, bool fp16_math, int threads, bool own_cu)
+template <int BG> tb_pair_kernels tb_pair_kernels_of(cuphyDataType_t llr_type, bool fp16_math, int threads)
 {
-    if (llr_type == CUPHY_R_32F)
-        return fp16_math ? tb_pair_kernel<BG, _Float16, float>(threads, own_cu)
-                         : tb_pair_kernel<BG, float, float>(threads, own_cu);
-    return llr_type == CUPHY_R_16F ? tb_pair_kernel<BG, _Float16, _Float16>(threads, own_cu) : nullptr;
-}
-void* select_tb_pair_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math, int threads, bool own_cu)
-{
-    return bg == 1   ? tb_pair_kernel_of<1>(llr_type, fp16_math, threads, own_cu)
-           : bg == 2 ? tb_pair_kernel_of<2>(llr_type, fp16_math, threads, own_cu)
-                     : nullptr;
+    if (llr_type == CUPHY_R_16F) return tb_pair_kernels_of<BG, _Float16, _Float16>(threads);
+    return fp16_math ? tb_pair_kernels_of<BG, _Float16, float>(threads) : tb_pair_kernels_of<BG, float, float>(threads);
 }
 
 void* select_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math, int mb)
@@ -366,7 +361,49 @@ static bool use_fp16_math(const cuphyLDPCDecodeConfigDesc_t& c)
     return c.llr_type == CUPHY_R_16F || c.algo == 2;
 }
 
-cuphyStatus_t check_lm_kernel(void* func);
+cuphyStatus_t check_lm_kernel(void* func, int& vgprs);
+
+// Workgroups of a kernel that a CU holds, by registers (512 per lane and SIMD, in
+// eights) and LDS.  The four SIMDs take a workgroup's waves in turn; of six
+// waves, two workgroups come to 4 on one SIMD (balanced_wave_place) and three to 5.
+int workgroups_per_cu(int vgprs, int threads, size_t lds_bytes)
+{
+    constexpr size_t CU_LDS = 160 * 1024;
+    const int per_simd = std::min(8, 512 / std::max(8, (vgprs + 7) & ~7)), waves = threads / 64;
+    const bool spread = waves < 4 || (waves == 6 && per_simd >= 4);
+    const int by_regs = spread ? 4 * per_simd / waves : per_simd / ((waves + 3) / 4);
+    return std::max(1, std::min(by_regs, (int)(CU_LDS / std::max<size_t>(lds_bytes, 1))));
+}
+
+// The form of the row-pair kernel for a launch: offsets in registers (with at
+// most one code block per CU) where that lets as many workgroups share a CU as
+// the plain form does, or as four such launches put on one (a process's launches
+// run from four hardware queues unless it asks for more).  So a launch gets the
+// registers when it leaves CUs idle anyway, and launches that fill the GPU
+// together keep their waves.  Four launches of 256 blocks on four streams, before
+// this form and with it: BG1 binary32 Z = 128, 46 rows 247 and 549 us, BG1
+// binary16 Z = 128 180 and 224; where both leave the same room it is faster there
+// too: BG1 binary16 Z = 256 527 and 464 us.
+// cu_count 0: a launch of any later size, the plain form.
+cuphyStatus_t select_tb_pair_kernel(const cuphyLDPCDecodeConfigDesc_t& c, bool fp16, int cu_count, launch_geometry& g)
+{
+    constexpr int QUEUES = 4;
+    const int threads = (int)g.block.x, groups = (int)g.grid.x;
+    const tb_pair_kernels k = c.BG == 1 ? tb_pair_kernels_of<1>(c.llr_type, fp16, threads)
+                                        : tb_pair_kernels_of<2>(c.llr_type, fp16, threads);
+    int vgprs = 0;
+    cuphyStatus_t s = check_lm_kernel(k.full, vgprs);
+    if (s != CUPHY_STATUS_SUCCESS) return s;
+    int need = workgroups_per_cu(vgprs, threads, g.lds_bytes);
+    if (cu_count > 0) need = (int)std::min<long long>(need, ((long long)QUEUES * groups + cu_count - 1) / cu_count);
+    for (void* func : {groups <= cu_count ? k.pre : nullptr, k.full}) {
+        if (!func) continue;
+        if ((s = check_lm_kernel(func, vgprs)) != CUPHY_STATUS_SUCCESS) return s;
+        g.func = func;
+        if (workgroups_per_cu(vgprs, threads, g.lds_bytes) >= need) break;
+    }
+    return CUPHY_STATUS_SUCCESS;
+}
 
 cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, int cu_count, launch_geometry& g)
 {
@@ -381,20 +418,15 @@ cuphyStatus_t fill_launch(const cuphyLDPCDecodeDesc_t& desc, int cu_count, launc
     const bool pair = P == 1 && c.num_parity_nodes > SMALL_MAXR;
     g.block = pair ? dim3((unsigned)(2 * ((c.Z + 63) / 64 * 64))) : dim3((unsigned)((P * c.Z + 63) / 64 * 64));
     g.grid = dim3((unsigned)((desc_codewords(desc) + P - 1) / P));
-    g.func = pair ? select_tb_pair_kernel(c.BG, c.llr_type, fp16, (int)g.block.x, (int)g.grid.x <= cu_count)
-                  : select_kernel(c.BG, c.llr_type, fp16, c.num_parity_nodes);
-    if (!g.func) return CUPHY_STATUS_UNSUPPORTED_CONFIG;
-    if (pair) {
-        const cuphyStatus_t s = check_lm_kernel(g.func);
-        if (s != CUPHY_STATUS_SUCCESS) return s;
-    }
     const int nsys = (c.BG == 1) ? 22 : 10;
     const size_t stride = (size_t)(((nsys + c.num_parity_nodes) * c.Z + 7) & ~7);
     // row-pair kernels keep the APP values lane-major (binary16: split layout)
     g.lds_bytes = pair ? (size_t)lm_app_bytes(c.BG, c.Z, nsys + c.num_parity_nodes, fp16 ? 2 : 4,
                                               lm_split_layout(fp16 ? 2 : 4, 46)) + 16u
                        : (size_t)P * stride * (fp16 ? 2u : 4u);
-    return CUPHY_STATUS_SUCCESS;
+    if (pair) return select_tb_pair_kernel(c, fp16, cu_count, g);
+    g.func = select_kernel(c.BG, c.llr_type, fp16, c.num_parity_nodes);
+    return g.func ? CUPHY_STATUS_SUCCESS : CUPHY_STATUS_UNSUPPORTED_CONFIG;
 }
 
 // Raise a kernel's dynamic-LDS limit above the 64 KB default, once per
@@ -420,16 +452,21 @@ cuphyStatus_t ensure_lds_attr(void* func, size_t bytes)
 
 // Lane-major kernels address their APP values from LDS address 0, so they
 // must hold no static LDS (which would come first); checked once per kernel.
-cuphyStatus_t check_lm_kernel(void* func)
+// vgprs: the kernel's registers per lane.
+cuphyStatus_t check_lm_kernel(void* func, int& vgprs)
 {
     static std::mutex mu;
-    static std::vector<void*> ok;
+    static std::vector<std::pair<void*, int>> ok;
     std::lock_guard<std::mutex> g(mu);
-    for (void* f : ok)
-        if (f == func) return CUPHY_STATUS_SUCCESS;
+    for (const auto& f : ok)
+        if (f.first == func) {
+            vgprs = f.second;
+            return CUPHY_STATUS_SUCCESS;
+        }
     hipFuncAttributes attr{};
     if (hipFuncGetAttributes(&attr, func) != hipSuccess || attr.sharedSizeBytes != 0) return CUPHY_STATUS_INTERNAL_ERROR;
-    ok.push_back(func);
+    vgprs = attr.numRegs;
+    ok.emplace_back(func, vgprs);
     return CUPHY_STATUS_SUCCESS;
 }
 
@@ -481,7 +518,8 @@ cuphyStatus_t decode_batch(cuphyHipLDPCWorkItem_t* d_items, const uint32_t* d_gr
     size_t lds = (size_t)max_values_per_group * elem + (lm ? 8u * 384u : 0u);
     if (lm && lm_split_layout((int)elem, (pair || max_mb > SMALL_MAXR) ? 46 : SMALL_MAXR))
         lds = std::max(lds, (size_t)lm_app_bytes_max((int)elem, true) + 16u);
-    cuphyStatus_t s = lm ? check_lm_kernel(func) : CUPHY_STATUS_SUCCESS;
+    int vgprs = 0;
+    cuphyStatus_t s = lm ? check_lm_kernel(func, vgprs) : CUPHY_STATUS_SUCCESS;
     if (s == CUPHY_STATUS_SUCCESS) s = ensure_lds_attr(func, lds);
     if (s != CUPHY_STATUS_SUCCESS) return s;
     int per_cu = 0;

@@ -386,3 +386,22 @@ def test_fp32_values_not_finite(dec, bg, Z, mb, kind):
             ref_h, ref_s = model_fp32(bg, Z, mb, llr[c], n_iter, alpha)
             assert np.array_equal(h[c], ref_h), (n_iter, c)
             assert np.array_equal(s[c], ref_s, equal_nan=True), (n_iter, c)
+
+
+# Launches at which the form of the row-pair kernel changes (offsets in
+# registers, full, lean): by how many code blocks share a CU.
+@pytest.mark.parametrize("bg,Z,mb,dtype,counts", [
+    (2, 192, 12, "fp16", (1, 64, 100, 300)), (2, 192, 12, "fp32in_fp16math", (65, 300)),
+    (2, 256, 9, "fp32", (64, 65, 300)), (2, 384, 9, "fp32", (256, 257)), (1, 128, 10, "fp32", (64, 65)),
+    (1, 128, 10, "fp16", (128, 129, 300)), (1, 208, 46, "fp16", (256, 257)), (2, 64, 42, "fp16", (256, 1100))])
+def test_row_pair_forms_bit_exact(dec, bg, Z, mb, dtype, counts):
+    _log("row-pair forms BG%d Z=%d mb=%d %s, %s code blocks, seed=23" % (bg, Z, mb, dtype, counts))
+    llr, _ = V.make_cbs(bg, Z, mb, 3, seed=23, snr_db=2.0)
+    if dtype != "fp32":
+        llr = V.to_half_rn(llr).astype(np.float32)
+    h_ref, s_ref, _ = run_oracle(bg, Z, mb, llr, n_iter=4, mode=O.FP32 if dtype == "fp32" else O.FP16)
+    for n in counts:
+        which = np.arange(n) % 3
+        h, s = run_gpu(dec, bg, Z, mb, llr[which], n_iter=4, dtype=dtype)
+        assert np.array_equal(h, h_ref[which]), n
+        assert_soft_equal(s, s_ref[which])
