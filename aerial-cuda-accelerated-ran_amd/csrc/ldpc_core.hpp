@@ -158,30 +158,41 @@ template <int BG, int NR> constexpr own_plan<BG, NR> kOwnPlan = make_own_plan<BG
 // instead of 3, so the degree is what the kernel's registers hold at its
 // occupancy: 168 per lane with two lane groups (three waves per SIMD), 256 with
 // one, 128 with at most SMALL_MAXR rows.  Measured, 8 code blocks Zc = 384,
-// all rows, two lane groups: BG1 213.6 -> 202.3 us, BG2 141.3 -> 120.2 us; 700
+// all rows, two lane groups: BG1 214.2 -> 204.3 us, BG2 141.3 -> 120.2 us; 700
 // blocks BG2 R = 0.5 219 -> 190 us; no change where the rows' latency bounds
 // (BG1 Zc = 128: 151.2 -> 150.2 us).
-template <int BG, int NR, int PAIR> struct f32_plan {
+// LEAN: for workgroups that share a CU, no more registers than leave the room
+// that compressed rows leave (BG2: 128 with two lane groups, 80 with at most
+// SMALL_MAXR rows).  2,048 blocks BG2 Zc = 256, 42 rows: every row compressed
+// 566 us, up to degree 10 explicit in 137 registers 871 us, up to degree 4 in
+// 126 534 us.
+template <int BG, int NR, int PAIR, bool LEAN> struct f32_plan {
     bool is_explicit[64];
     int slot[64];
     int messages, rows;  // registers' worth of the larger lane group
 };
-constexpr int f32_explicit_degree(int BG, int NR, int PAIR)
+constexpr int f32_explicit_degree(int BG, int NR, int PAIR, bool LEAN)
 {
-    if (NR <= SMALL_MAXR) return BG == 1 ? 5 : 6;
-    if (PAIR == 2) return BG == 1 ? 5 : 10;
+    if (NR <= SMALL_MAXR) return BG == 1 || LEAN ? 5 : 6;
+    if (PAIR == 2) return BG == 1 ? 5 : LEAN ? 4 : 10;
     return BG == 1 ? 4 : 6;
 }
-template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> make_f32_plan()
+// Registers per lane group that explicit messages may take beyond the compressed
+// rows': BG1 with two lane groups stays below 168 without spills, LEAN in the
+// batch kernel beside BG2's rows.
+constexpr int f32_explicit_extra(int BG, int PAIR, bool LEAN) { return BG == 1 && PAIR == 2 ? (LEAN ? 10 : 16) : 1000; }
+template <int BG, int NR, int PAIR, bool LEAN> constexpr f32_plan<BG, NR, PAIR, LEAN> make_f32_plan()
 {
     using BGT = bg_traits<BG>;
-    f32_plan<BG, NR, PAIR> p{};
-    int messages[2] = {0, 0}, rows[2] = {0, 0};
+    f32_plan<BG, NR, PAIR, LEAN> p{};
+    int messages[2] = {0, 0}, rows[2] = {0, 0}, extra[2] = {0, 0};
     const pair_plan<BG, NR> pp = make_pair_plan<BG, NR>();
     for (int r = 0; r < NR; ++r) {
         const int g = (PAIR == 2) ? pp.group[r] : 0;
         const int d = BGT::row_start(r + 1) - BGT::row_start(r);
-        p.is_explicit[r] = d <= f32_explicit_degree(BG, NR, PAIR);
+        p.is_explicit[r] = d <= f32_explicit_degree(BG, NR, PAIR, LEAN) &&
+                           extra[g] + d - 3 <= f32_explicit_extra(BG, PAIR, LEAN);
+        if (p.is_explicit[r]) extra[g] += d - 3;
         int& next = p.is_explicit[r] ? messages[g] : rows[g];
         p.slot[r] = next;
         next += p.is_explicit[r] ? d : 1;
@@ -190,7 +201,8 @@ template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> make_f32_pl
     p.rows = rows[0] > rows[1] ? rows[0] : rows[1];
     return p;
 }
-template <int BG, int NR, int PAIR> constexpr f32_plan<BG, NR, PAIR> kF32Plan = make_f32_plan<BG, NR, PAIR>();
+template <int BG, int NR, int PAIR, bool LEAN>
+constexpr f32_plan<BG, NR, PAIR, LEAN> kF32Plan = make_f32_plan<BG, NR, PAIR, LEAN>();
 
 // Slots of the offsets of run_iterations' PRE form: the edges that need a
 // rotation, counted per lane group.
@@ -766,7 +778,9 @@ template <> __device__ __forceinline__ _Float16 job_alpha<_Float16>(const cb_job
 // loads of its shifts, a multiplication and two vector operations per edge --
 // for launches of few small code blocks, whose time is the latency of one
 // row after another (a wave per SIMD has the registers).
-template <int BG, typename T, int MAXR, int PAIR = 1, bool LM = (PAIR == 2), bool PRE = false>
+// LEAN: no registers for what only speeds up a workgroup that has its CU to
+// itself (own parity columns; f32_plan).
+template <int BG, typename T, int MAXR, int PAIR = 1, bool LM = (PAIR == 2), bool PRE = false, bool LEAN = false>
 __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job& job, int count = 1, int stride = 0,
                                               uint32_t* cb_flags = nullptr, uint32_t* cb_iters = nullptr,
                                               uint32_t tid = threadIdx.x)
@@ -786,7 +800,7 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
                                       : padded_row_start<BG>(NR);
     constexpr int NW = NEDGE / 2;
     constexpr bool F32 = std::is_same<T, float>::value;
-    constexpr f32_plan<BG, NR, PAIR> FP = kF32Plan<BG, NR, PAIR>;
+    constexpr f32_plan<BG, NR, PAIR, LEAN> FP = kF32Plan<BG, NR, PAIR, LEAN>;
     constexpr int NRS = F32 && FP.rows > 0 ? FP.rows : 1, NM = F32 && FP.messages > 0 ? FP.messages : 1;
     float st_n1[NRS], st_n2[NRS], st_f[NM];
     uint32_t st_meta[NRS];
@@ -866,8 +880,9 @@ __device__ __forceinline__ int run_iterations(T* __restrict__ app, const cb_job&
     // rows), and these columns are 42 of BG1's 316 edges, 38 of BG2's 197.
     // Mixed slot of 16 UEs 153 -> 149 us, receive chain of 64 UEs 411 -> 396 us.
     // Not in the kernels whose registers are full (one lane group, offsets in
-    // registers, binary32).
-    constexpr bool OWNS = PAIR == 2 && !F32 && !PRE;
+    // registers, binary32) or whose workgroups share a CU (LEAN: 2,048 blocks BG2
+    // Zc = 192, 10 rows 182 us in 83 registers, 218 us with these in 102).
+    constexpr bool OWNS = PAIR == 2 && !F32 && !PRE && !LEAN;
     constexpr own_plan<BG, NR> own_slots = kOwnPlan<BG, NR>;
     constexpr int NOWN = OWNS && own_slots.count > 0 ? own_slots.count : 1;
     uint32_t own[NOWN];
@@ -1042,7 +1057,7 @@ struct cb_buffers {
 // workgroup (count * Z <= blockDim.x); LDS `app` holds count regions of
 // group_stride((NSYS + mb) * Z) values of type T.  buf(c) gives code block
 // c's buffers.  Every thread of the workgroup calls it.
-template <int BG, typename T, typename TIn, int MAXR, typename Buf>
+template <int BG, typename T, typename TIn, int MAXR, bool LEAN = false, typename Buf>
 __device__ __forceinline__ int decode_group(T* __restrict__ app, const cb_job& job, int count, const Buf& buf,
                                             uint32_t* cb_flags)
 {
@@ -1051,7 +1066,7 @@ __device__ __forceinline__ int decode_group(T* __restrict__ app, const cb_job& j
     for (int c = 0; c < count; ++c)
         load_llrs_nosync<T, TIn>(app + c * stride, static_cast<const TIn*>(buf(c).llr), nval, job.clamp);
     __syncthreads();
-    const int iters = run_iterations<BG, T, MAXR>(app, job, count, stride, cb_flags);
+    const int iters = run_iterations<BG, T, MAXR, 1, false, false, LEAN>(app, job, count, stride, cb_flags);
     const int nbits = job.Kb * job.Z;
     for (int c = 0; c < count; ++c) {
         const cb_buffers b = buf(c);
@@ -1070,7 +1085,7 @@ __device__ __forceinline__ int decode_group(T* __restrict__ app, const cb_job& j
 // at z * pitch + column * sizeof(T).  PAIR = 2: row-pair mode (blockDim.x >=
 // 2 * roundup64(Z)); PAIR = 1: one lane group (blockDim.x >= Z).  flag: one
 // LDS word outside the values (the early-termination vote).
-template <int BG, typename T, typename TIn, int MAXR, int PAIR, bool PRE = false>
+template <int BG, typename T, typename TIn, int MAXR, int PAIR, bool PRE = false, bool LEAN = false>
 __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job, const cb_buffers& b, uint32_t* flag,
                                          uint32_t tid = threadIdx.x, uint32_t nthr = blockDim.x)
 {
@@ -1110,7 +1125,7 @@ __device__ __forceinline__ int decode_lm(T* __restrict__ app, const cb_job& job,
         }
         __syncthreads();
     }
-    const int iters = run_iterations<BG, T, MAXR, PAIR, true, PRE>(app, job, 1, 0, flag, nullptr, tid);
+    const int iters = run_iterations<BG, T, MAXR, PAIR, true, PRE, LEAN>(app, job, 1, 0, flag, nullptr, tid);
     const int nbits = job.Kb * Z;
     // hard decisions, 64 per wave per step by ballot (as store_hard); each
     // lane walks its (column, z) position instead of dividing per bit

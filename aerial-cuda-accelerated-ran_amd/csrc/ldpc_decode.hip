@@ -53,7 +53,7 @@ __global__ __launch_bounds__(384) void ldpc_layered_tb(cuphyLDPCDecodeDesc_t des
     const int P = tb_group_size(desc.config.Z);
     const int first = (int)blockIdx.x * P;
     const int count = min(P, desc_codewords(desc) - first);
-    decode_group<BG, T, TIn, MAXR>(
+    decode_group<BG, T, TIn, MAXR, (MAXR <= SMALL_MAXR)>(
         reinterpret_cast<T*>(lds_raw), tb_job<TIn>(desc), count,
         [&](int c) { return tb_buffers<TIn>(desc, first + c); }, s_cb_flags);
 }
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(384) void ldpc_layered_tb(cuphyLDPCDecodeDesc_t des
 // workgroup, Z > 32, mb > 8): workgroup b decodes code word b with two lane
 // groups of roundup64(Z) lanes that take the column-disjoint block rows of
 // each barrier segment at the same time (run_iterations PAIR = 2).
-template <int BG, typename T, typename TIn, bool PRE>
+template <int BG, typename T, typename TIn, bool PRE, bool LEAN>
 __device__ __forceinline__ void tb_pair(const cuphyLDPCDecodeDesc_t& desc)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -71,12 +71,21 @@ __device__ __forceinline__ void tb_pair(const cuphyLDPCDecodeDesc_t& desc)
     uint32_t* flag = reinterpret_cast<uint32_t*>(
         lds_raw + lm_app_bytes(BG, job.Z, bg_traits<BG>::NSYS + job.mb, (int)sizeof(T),
                                lm_split_layout((int)sizeof(T), 46)));
-    decode_lm<BG, T, TIn, 46, 2, PRE>(reinterpret_cast<T*>(lds_raw), job, tb_buffers<TIn>(desc, (int)blockIdx.x), flag);
+    decode_lm<BG, T, TIn, 46, 2, PRE, LEAN>(reinterpret_cast<T*>(lds_raw), job, tb_buffers<TIn>(desc, (int)blockIdx.x),
+                                            flag);
 }
 template <int BG, typename T, typename TIn>
 __global__ __launch_bounds__(768) void ldpc_layered_tb_pair(cuphyLDPCDecodeDesc_t desc)
 {
-    tb_pair<BG, T, TIn, false>(desc);
+    tb_pair<BG, T, TIn, false, false>(desc);
+}
+
+// The same in fewer registers (run_iterations LEAN; BG2, whose rows leave room
+// for more workgroups per CU: binary16 83 against 102, binary32 126 against 137).
+template <int BG, typename T, typename TIn>
+__global__ __launch_bounds__(768) void ldpc_layered_tb_pair_lean(cuphyLDPCDecodeDesc_t desc)
+{
+    tb_pair<BG, T, TIn, false, true>(desc);
 }
 
 // The same with every edge's offset in a register (run_iterations PRE), for
@@ -93,7 +102,7 @@ template <int BG, typename T> constexpr int tb_pre_threads()
 template <int BG, typename T, typename TIn>
 __global__ __launch_bounds__((tb_pre_threads<BG, T>())) void ldpc_layered_tb_pair_pre(cuphyLDPCDecodeDesc_t desc)
 {
-    tb_pair<BG, T, TIn, true>(desc);
+    tb_pair<BG, T, TIn, true, false>(desc);
 }
 
 // Persistent heterogeneous decoder: each workgroup repeatedly takes the
@@ -218,7 +227,8 @@ __device__ __forceinline__ void persistent_lm(cuphyHipLDPCWorkItem_t* items, con
             if (st == 0) {
                 const cb_buffers b{w.llr, w.out, static_cast<_Float16*>(w.soft)};
                 if (w.BG == 1)
-                    decode_lm<1, T, TIn, MAXR, PAIR>(app, job, b, flag, tid, (uint32_t)rows_threads);
+                    decode_lm<1, T, TIn, MAXR, PAIR, false, PAIR == 2 && std::is_same<T, float>::value>(
+                        app, job, b, flag, tid, (uint32_t)rows_threads);
                 else
                     decode_lm<2, T, TIn, MAXR, PAIR>(app, job, b, flag, tid, (uint32_t)rows_threads);
             }
@@ -301,12 +311,16 @@ void* select_tb_kernel(int bg, cuphyDataType_t llr_type, bool fp16_math)
 // Row-pair kernels of a configuration; pre: nullptr where its launch bounds do
 // not take the workgroup.
 struct tb_pair_kernels {
-    void *full, *pre;
+    void *full, *lean, *pre;
 };
 template <int BG, typename T, typename TIn> tb_pair_kernels tb_pair_kernels_of(int threads)
 {
     tb_pair_kernels k;
     k.full = (void*)&ldpc_layered_tb_pair<BG, T, TIn>;
+    if constexpr (BG == 1)
+        k.lean = k.full;  // (three waves per SIMD either way)
+    else
+        k.lean = (void*)&ldpc_layered_tb_pair_lean<BG, T, TIn>;
     k.pre = threads <= tb_pre_threads<BG, T>() ? (void*)&ldpc_layered_tb_pair_pre<BG, T, TIn> : nullptr;
     return k;
 }
@@ -375,16 +389,19 @@ int workgroups_per_cu(int vgprs, int threads, size_t lds_bytes)
     return std::max(1, std::min(by_regs, (int)(CU_LDS / std::max<size_t>(lds_bytes, 1))));
 }
 
-// The form of the row-pair kernel for a launch: offsets in registers (with at
-// most one code block per CU) where that lets as many workgroups share a CU as
-// the plain form does, or as four such launches put on one (a process's launches
-// run from four hardware queues unless it asks for more).  So a launch gets the
-// registers when it leaves CUs idle anyway, and launches that fill the GPU
-// together keep their waves.  Four launches of 256 blocks on four streams, before
-// this form and with it: BG1 binary32 Z = 128, 46 rows 247 and 549 us, BG1
-// binary16 Z = 128 180 and 224; where both leave the same room it is faster there
-// too: BG1 binary16 Z = 256 527 and 464 us.
-// cu_count 0: a launch of any later size, the plain form.
+// The form of the row-pair kernel for a launch: the first of offsets in
+// registers (with at most one code block per CU), full and lean that lets as
+// many workgroups share a CU as the lean one does, or as four such launches put
+// on one (a process's launches run from four hardware queues unless it asks for
+// more).  So a launch gets the registers when it leaves CUs idle anyway, and
+// launches that fill the GPU together, or one that does alone, keep their
+// waves.  Four launches of 256 blocks on four streams, lean or full against the
+// form that is fastest alone: BG1 binary32 Z = 128, 46 rows 247 and 549 us, BG2
+// binary16 Z = 192, 42 rows 198 and 314, BG2 binary32 Z = 256, 42 rows 270 and
+// 375; where both leave the same room it is faster there too: BG1 binary16 Z =
+// 192, 46 rows 514 and 457 us.
+// cu_count 0: a launch of any later size (no offsets in registers, and the lean
+// form unless the full one leaves the same room).
 cuphyStatus_t select_tb_pair_kernel(const cuphyLDPCDecodeConfigDesc_t& c, bool fp16, int cu_count, launch_geometry& g)
 {
     constexpr int QUEUES = 4;
@@ -392,11 +409,11 @@ cuphyStatus_t select_tb_pair_kernel(const cuphyLDPCDecodeConfigDesc_t& c, bool f
     const tb_pair_kernels k = c.BG == 1 ? tb_pair_kernels_of<1>(c.llr_type, fp16, threads)
                                         : tb_pair_kernels_of<2>(c.llr_type, fp16, threads);
     int vgprs = 0;
-    cuphyStatus_t s = check_lm_kernel(k.full, vgprs);
+    cuphyStatus_t s = check_lm_kernel(k.lean, vgprs);
     if (s != CUPHY_STATUS_SUCCESS) return s;
     int need = workgroups_per_cu(vgprs, threads, g.lds_bytes);
     if (cu_count > 0) need = (int)std::min<long long>(need, ((long long)QUEUES * groups + cu_count - 1) / cu_count);
-    for (void* func : {groups <= cu_count ? k.pre : nullptr, k.full}) {
+    for (void* func : {groups <= cu_count ? k.pre : nullptr, k.full, k.lean}) {
         if (!func) continue;
         if ((s = check_lm_kernel(func, vgprs)) != CUPHY_STATUS_SUCCESS) return s;
         g.func = func;
