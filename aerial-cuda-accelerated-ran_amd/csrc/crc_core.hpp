@@ -169,14 +169,13 @@ template <int S, typename Word, typename Step>
 __device__ __forceinline__ uint32_t strided_crc(int nw, int t, Word word, Step step)
 {
     constexpr int U = 4;  // words in flight
-    uint32_t v = 0;
-    for (int i = (nw + S - 1) / S - 1; i >= 0; i -= U) {
+    int i = (nw + S - 1) / S - 1;
+    // (the first word needs no step; only it can be missing)
+    uint32_t v = (i >= 0 && i * S + t < nw) ? word(nw - 1 - i * S - t) : 0u;
+    for (--i; i >= 0; i -= U) {
         uint32_t w[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = (i - u) * S + t;  // words from the end
-            w[u] = (i >= u && e < nw) ? word(nw - 1 - e) : 0u;
-        }
+        for (int u = 0; u < U; ++u) w[u] = (i >= u) ? word(nw - 1 - (i - u) * S - t) : 0u;
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (i >= u) v = step(0, v & 255u) ^ step(1, (v >> 8) & 255u) ^ step(2, (v >> 16) & 255u) ^ step(3, v >> 24) ^ w[u];

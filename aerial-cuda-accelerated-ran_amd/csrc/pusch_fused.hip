@@ -311,102 +311,6 @@ __device__ __forceinline__ void combine_symbols(_Float16* __restrict__ cbuf, con
     __syncthreads();
 }
 
-// Combining as combine_symbols where, besides, none of the Qm runs of EQ
-// positions wraps around the circle or crosses the filler: bit k of symbol j
-// then goes to position at(k) + j with a uniform at(k).  A first transmission
-// (ndi) reads nothing, its sum is LLR + 0.  Per LLR one add for the address,
-// convert, scale, round and add, instead of about 25 operations with the wrap
-// and filler tests; int8 LLRs whose scale keeps them within the clamp are not
-// clamped on their own.
-template <int QM, typename TI, bool DESCR>
-__device__ __forceinline__ void combine_runs(_Float16* __restrict__ cbuf, const TI* __restrict__ in,
-                                             const rm_geometry& g, float scale, const uint32_t* __restrict__ seq,
-                                             int soff)
-{
-    typedef typename slot_vec<TI>::type vec_t;
-    constexpr int NB = 4;  // symbols per thread in flight
-    const bool clamp = !(std::is_same<TI, int8_t>::value && __builtin_fabsf(scale) <= LLR_MAX_ABS / 128.0f);
-    const int nthr = blockDim.x;
-    const vec_t* sym = reinterpret_cast<const vec_t*>(in + g.adj);
-    int at[QM];
-    int c0 = g.c0, EQ = g.EQ;  // (opaque: not hoisted out of the switch over the modulation orders)
-    asm volatile("" : "+s"(c0), "+s"(EQ));
-#pragma unroll
-    for (int k = 0; k < QM; ++k) {
-        int c = c0 + k * EQ;
-        if (c >= g.L) c -= g.L;
-        at[k] = (c >= g.Kd) ? c + g.F : c;
-    }
-    for (int j0 = opaque_tid(); j0 < EQ; j0 += NB * nthr) {
-        vec_t v[NB];
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int j = j0 + u * nthr;
-            if (j < EQ) v[u] = sym[j];
-        }
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            const int j = j0 + u * nthr;
-            if (j >= EQ) break;
-            _Float16 x[QM];
-#pragma unroll
-            for (int k = 0; k < QM; ++k) x[k] = (_Float16)(llr_as_float(v[u][k]) * scale);
-            if (clamp) {
-#pragma unroll
-                for (int k = 0; k < QM; ++k) x[k] = rm_num<_Float16>::clamp(x[k]);
-            }
-            if (DESCR) {  // bits n0 .. n0 + Qm - 1, n0 = soff + j * Qm (word n0/32 + 1 exists)
-                const int n0 = soff + j * QM;
-                const uint32_t bits = __builtin_amdgcn_alignbit(seq[(n0 >> 5) + 1], seq[n0 >> 5], (uint32_t)n0 & 31u);
-#pragma unroll
-                for (int k = 0; k < QM; ++k) x[k] = u2h((uint16_t)(h2u(x[k]) ^ ((bits << (15 - k)) & 0x8000u)));
-            }
-            if (g.ndi) {  // (0 + a clamped value is within the bounds)
-#pragma unroll
-                for (int k = 0; k < QM; ++k) cbuf[at[k] + j] = (_Float16)0.0f + x[k];
-            } else {
-                _Float16 prev[QM];
-#pragma unroll
-                for (int k = 0; k < QM; ++k) prev[k] = cbuf[at[k] + j];
-#pragma unroll
-                for (int k = 0; k < QM; ++k) cbuf[at[k] + j] = rm_num<_Float16>::clamp(prev[k] + x[k]);
-            }
-        }
-    }
-    __syncthreads();
-}
-
-// Whether none of the Qm runs wraps or crosses the filler (E <= L).
-__device__ __forceinline__ bool runs_whole(const rm_geometry& g)
-{
-    int c = g.c0;
-    bool whole = true;
-    for (int k = 0; k < g.Qm; ++k) {
-        if (c >= g.L) c -= g.L;
-        whole = whole && c + g.EQ <= g.L && (c >= g.Kd || c + g.EQ <= g.Kd || g.F == 0);
-        c += g.EQ;
-    }
-    return whole;
-}
-
-// RUNS: the one-CB kernels, whose per-CB operations bound them (64-cell int8
-// slot with the tasks of step 6: 600 -> 572 us); the kernels of groups, bound by
-// their slowest CB, ran 436 -> 445 us on 64 UEs with it (registers).
-template <typename TI, bool DESCR, bool RUNS>
-__device__ __forceinline__ void combine_once(_Float16* __restrict__ cbuf, const TI* __restrict__ in,
-                                             const rm_geometry& g, float scale, const uint32_t* __restrict__ seq,
-                                             int soff)
-{
-    if (!RUNS || !runs_whole(g)) return combine_symbols<TI, DESCR>(cbuf, in, g, scale, seq, soff);
-    switch (g.Qm) {  // (uniform) modulation order as a constant
-    case 8: return combine_runs<8, TI, DESCR>(cbuf, in, g, scale, seq, soff);
-    case 6: return combine_runs<6, TI, DESCR>(cbuf, in, g, scale, seq, soff);
-    case 4: return combine_runs<4, TI, DESCR>(cbuf, in, g, scale, seq, soff);
-    case 2: return combine_runs<2, TI, DESCR>(cbuf, in, g, scale, seq, soff);
-    default: return combine_symbols<TI, DESCR>(cbuf, in, g, scale, seq, soff);
-    }
-}
-
 // Words of the descrambling sequence covering a CB's rate-matched bits
 // [start, start + E): from word start / 32 to word (start + E - 1) / 32.
 __device__ __forceinline__ int rm_seq_words(const rm_geometry& g)
@@ -418,7 +322,7 @@ __device__ __forceinline__ int rm_seq_words(const rm_geometry& g)
 // transmission combined (descrambled with `seq` when descr), the buffer
 // written back to HBM and converted in place to the decoder's APP array of
 // nval values.  Ends with a barrier.
-template <typename TI, bool RUNS>
+template <typename TI>
 __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_t* __restrict__ seq,
                                               const cuphyHipPuschSlotTb_t& job, const PerTbParams& p,
                                               const rm_geometry& g, int r, int nh, int nval, bool descr)
@@ -471,9 +375,9 @@ __device__ __forceinline__ void fused_combine(_Float16* __restrict__ hb, uint32_
         else
             combine_tx<TI, false>(cbuf, in, g, p, scale, seq, soff);
     } else if (descr) {
-        combine_once<TI, true, RUNS>(cbuf, in, g, scale, seq, soff);
+        combine_symbols<TI, true>(cbuf, in, g, scale, seq, soff);
     } else {
-        combine_once<TI, false, RUNS>(cbuf, in, g, scale, seq, soff);
+        combine_symbols<TI, false>(cbuf, in, g, scale, seq, soff);
     }
 
     // ---- 3. write back the HARQ buffer; APP = clamp(HARQ), +0 for -0 ----
@@ -569,7 +473,7 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
             g = rm_geometry_of(p, cb0 + c);
             rm_make_uniform(g);
         }
-        fused_combine<TI, !GROUPED>(hb + c * S, seq, job, p, g, r0 + c, nh, nval, descr);
+        fused_combine<TI>(hb + c * S, seq, job, p, g, r0 + c, nh, nval, descr);
     }
 
     // ---- 4. decode -------------------------------------------------------
