@@ -624,13 +624,15 @@ void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,
     _Float16* hb = reinterpret_cast<_Float16*>(lds_raw);
     uint32_t* queue = ws;
     uint32_t* tbw = ws + FUSED_WS_QUEUE_WORDS;
+    uint32_t first = 0;  // (asked for now, needed after the tables)
+    if (threadIdx.x == 0) first = atomicAdd(&queue[0], 1u);
     load_crc_steps(sh);
     constexpr int PAIR = MAXR <= MID_MAXR ? 1 : 2;
     uint32_t row_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // one-CB form: bound by its instructions, 64-cell int8 slot 552 -> 546 us; groups
     // leave few waves without rows (64 UEs 411 -> 418 us with it: registers)
     if (PAIR == 1 && !GROUPED) row_wave = balanced_wave_place(sh.words);
-    if (threadIdx.x == 0) sh.item = (int)atomicAdd(&queue[0], 1u);
+    if (threadIdx.x == 0) sh.item = (int)first;
     __syncthreads();
     for (;;) {
         const int i = sh.item;
