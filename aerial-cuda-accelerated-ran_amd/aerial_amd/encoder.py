@@ -85,10 +85,13 @@ class LdpcEncoder:
         rows = num_rows if (rv == 0 and 0 < num_rows < (46 if bg == 1 else 42)) else (46 if bg == 1 else 42)
         nbits = (nsys + rows) * Z - (2 * Z if self.puncturing else 0)
         out_words = (nbits + 31) // 32
-        # contiguous tensors of one allocation, each at an address of its own 512 bytes
-        size = (ncw * out_words + 127) // 128 * 128
-        whole = torch.empty(n * size, dtype=torch.int32, device="cuda")
-        outs = list(whole.as_strided((n, ncw, out_words), (size, out_words, 1)).unbind(0))
+        if n == 1:
+            whole = torch.empty((ncw, out_words), dtype=torch.int32, device="cuda")
+            outs = [whole]
+        else:  # contiguous tensors of one allocation, each at an address of its own 512 bytes
+            size = (ncw * out_words + 127) // 128 * 128
+            whole = torch.empty(n * size, dtype=torch.int32, device="cuda")
+            outs = list(whole.as_strided((n, ncw, out_words), (size, out_words, 1)).unbind(0))
         tin = _BitTensor(in_words * 32, ncw, in_words * 32)
         tout = _BitTensor(out_words * 32, ncw, out_words * 32)
         in_ptrs = (C.c_void_p * n)(*[x.data_ptr() for x in info_words])
