@@ -8,7 +8,6 @@ pycuphy_ldpc_util.cpp:75-171; arrays are torch device tensors.
 """
 import ctypes as C
 
-import numpy as np
 import torch
 
 from . import _hip
@@ -90,12 +89,6 @@ def set_per_tb_params(tb_size, code_rate, qam_mod, rate_match_len, rv, ndi=1, ci
                                            user_group, nl, ng, lm, n_dmrs_cdm_grps_no_data,
                                            C.byref(lb) if lb is not None else None, C.byref(mb), C.byref(kb)))
     return p, mb.value, kb.value
-
-
-def params_to_device(params):
-    arr = (L.PerTbParams * len(params))(*params)
-    host = np.frombuffer(bytes(arr), dtype=np.uint8).copy()
-    return arr, torch.from_numpy(host).cuda()
 
 
 def put_params(address, params):

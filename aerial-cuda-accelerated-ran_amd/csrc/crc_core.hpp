@@ -1,9 +1,8 @@
 // Device core of the CRC checks (TS 38.212 5.1, zero initial value), shared
 // by the PUSCH CRC-decode kernels and the fused slot kernel.  Every thread
-// computes the remainder of some of the message's words, shifted by the bits
-// after them, and the shares are XOR-combined (CRC linearity): the CRC-decode
-// kernels give a thread every S-th word (strided_crc), the fused kernel one
-// word.  All tables are built at compile time.
+// computes the remainder of every S-th word of the message, shifted by the bits
+// after it (strided_crc), and the shares are XOR-combined (CRC linearity).  All
+// tables are built at compile time.
 #pragma once
 
 #include "nr_ldpc_common.hpp"
@@ -158,6 +157,10 @@ __device__ __forceinline__ uint32_t wave_mulmod24(uint32_t lane, uint32_t a, uin
     return wave_fold<24>(lane, (uint32_t)p, (uint32_t)(p >> 32), fold);
 }
 
+// Step tables of a wave (thread t of 64), by CRC kind.
+static __device__ const crc_stride_table<64> g_wave_stride[3] = {
+    make_crc_stride_table<64>(CRC24A_P), make_crc_stride_table<64>(CRC24B_P), make_crc_stride_table<64>(CRC16_P)};
+
 // Share of the remainder of nw message words (`word(i)` = message word i,
 // its first bit the most significant) that thread t of S holds: the words
 // nw - 1 - t - S * i, by Horner's rule from the first, step(b, x) =
@@ -183,40 +186,42 @@ __device__ __forceinline__ uint32_t strided_crc(int nw, int t, Word word, Step s
     return v;
 }
 
-// Byte-granular shift factors: x^(8m) mod g for m < CRC_SHIFT_LO (shifts
-// inside one code block, up to 1056 bytes), and for CRC24A x^(8 * 1024 * m)
-// mod g for m < 256 (shifts inside a TB of up to 256 KiB: x^(8n) =
-// x^(8 (n mod 1024)) * x^(8 * 1024 * (n / 1024))).  Built at compile time:
-// each entry is the previous one advanced by one byte-wise CRC step.
-constexpr int CRC_SHIFT_LO = 1088;
+// Byte-granular shift factors of CRC24A: x^(8m) and x^(8 * 1024 * m) mod g, for
+// shifts inside a TB of up to 256 KiB (x^(8n) = x^(8 (n mod 1024)) *
+// x^(8 * 1024 * (n / 1024))).  Built at compile time.
 struct crc_shift_tables {
-    uint32_t lo[3][CRC_SHIFT_LO];
-    uint32_t tb_hi[256];
+    uint32_t lo[1024];
+    uint32_t hi[256];
 };
 
 constexpr crc_shift_tables make_crc_shift_tables()
 {
     crc_shift_tables t{};
-    const crc_poly ps[3] = {CRC24A_P, CRC24B_P, CRC16_P};
-    for (int k = 0; k < 3; ++k) {
-        const uint32_t mask = (1u << ps[k].L) - 1u;
-        uint32_t v = 1;  // x^0
-        for (int m = 0; m < CRC_SHIFT_LO; ++m) {
-            t.lo[k][m] = v;
-            // v * x^8 mod g: one byte-wise step with a zero input byte
-            v = ((v << 8) & mask) ^ byte_entry((v >> (ps[k].L - 8)) & 0xFFu, ps[k]);
-        }
-    }
-    const uint32_t step = gf2_mulmod(t.lo[0][1023], t.lo[0][1], CRC24A_P);  // x^(8*1024)
-    uint32_t v = 1;
-    for (int m = 0; m < 256; ++m) {
-        t.tb_hi[m] = v;
-        v = gf2_mulmod(v, step, CRC24A_P);
-    }
+    uint32_t v = 1;  // x^0, advanced by x^8: one byte-wise step with a zero input byte
+    const auto step8 = [&] { v = ((v << 8) & 0xFFFFFFu) ^ byte_entry(v >> 16, CRC24A_P); };
+    for (int m = 0; m < 1024; ++m, step8()) t.lo[m] = v;
+    const uint32_t step = v;  // x^(8 * 1024)
+    v = 1;
+    for (int m = 0; m < 256; ++m, v = gf2_mulmod(v, step, CRC24A_P)) t.hi[m] = v;
     return t;
 }
 
 static __device__ const crc_shift_tables g_crc_shift = make_crc_shift_tables();
+
+// Bytes 0 .. nbytes - 1 of a message (bytes4(w): its word w, bytes in memory
+// order) to dst, by thread t of n: whole aligned words of the destination, each
+// from two message words, single bytes only at both ends.
+template <typename Bytes4> __device__ __forceinline__ void put_bytes(uint8_t* dst, int nbytes, Bytes4 bytes4, int t, int n)
+{
+    const int head = min(nbytes, (int)((0u - (uint32_t)(uintptr_t)dst) & 3u));
+    const int nfull = (nbytes - head) >> 2, tail = head + 4 * nfull;
+    for (int i = t; i < nfull; i += n) {
+        const uint32_t lo = bytes4(i), hi = (head != 0) ? bytes4(i + 1) : 0u;  // (byte 4 i + 3 + head < nbytes)
+        *reinterpret_cast<uint32_t*>(dst + head + 4 * i) = __builtin_amdgcn_alignbyte(hi, lo, (uint32_t)head);
+    }
+    const int b = t < head ? t : tail + t - head;
+    if (t < head + nbytes - tail) dst[b] = (uint8_t)(bytes4(b >> 2) >> (8 * (b & 3)));
+}
 
 // CRC bits attached to each CB: 24 (CRC24B) when the TB is segmented.
 __device__ __forceinline__ int cb_crc_bits(const PerTbParams& p)

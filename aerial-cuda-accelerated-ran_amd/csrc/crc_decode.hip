@@ -38,9 +38,7 @@
 
 namespace nrldpc {
 
-// Step tables: a wave per code block, by CRC kind; the TB kernel's threads.
-static __device__ const crc_stride_table<64> g_cb_stride[3] = {
-    make_crc_stride_table<64>(CRC24A_P), make_crc_stride_table<64>(CRC24B_P), make_crc_stride_table<64>(CRC16_P)};
+// Step tables of the TB kernel's threads.
 static __device__ const crc_stride_table<CRC_TB_BLOCK> g_tb_stride = make_crc_stride_table<CRC_TB_BLOCK>(CRC24A_P);
 
 struct tb_layout {
@@ -70,7 +68,7 @@ template <typename Word>
 __device__ __forceinline__ uint32_t wave_crc(int nw, int kind, Word word, const uint32_t (*table)[256])
 {
     const uint32_t t = threadIdx.x & 63u;
-    const uint32_t last = g_cb_stride[kind].last[t], fold = g_crc_fold.k[kind][t];
+    const uint32_t last = g_wave_stride[kind].last[t], fold = g_crc_fold.k[kind][t];
     const uint32_t v = strided_crc<64>(nw, (int)t, word, [&](int b, uint32_t x) { return table[b][x]; });
     return kind == K_CRC16 ? wave_sum_products<16>(t, v, last, fold) : wave_sum_products<24>(t, v, last, fold);
 }
@@ -84,7 +82,7 @@ __global__ __launch_bounds__(CRC_CB_BLOCK) void crc_cb_kernel(const crc_descript
     const int C = (int)p.num_CBs;
     if ((int)blockIdx.x * CRC_CBS_PER_BLOCK >= C) return;
     const int kind = cb_crc_kind(p);
-    for (int i = threadIdx.x; i < 4 * 256; i += blockDim.x) (&step[0][0])[i] = (&g_cb_stride[kind].step[0][0])[i];
+    for (int i = threadIdx.x; i < 4 * 256; i += blockDim.x) (&step[0][0])[i] = (&g_wave_stride[kind].step[0][0])[i];
     const tb_layout l = layout_of(d, slot);
     __syncthreads();
     const int cb_in_tb = (int)blockIdx.x * CRC_CBS_PER_BLOCK + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -98,18 +96,8 @@ __global__ __launch_bounds__(CRC_CB_BLOCK) void crc_cb_kernel(const crc_descript
     // message bytes in memory order; the message's first bit is the top bit of byte 0
     const auto bytes4 = [&](int w) { return rev ? rbit8x4(words[w]) : words[w]; };
     const uint32_t crc = wave_crc(nw, kind, [&](int w) { return __builtin_bswap32(bytes4(w)); }, step);
-    // the payload bytes: whole aligned words of the destination, single bytes at both ends
     uint8_t* const tb = d.tb_out + l.tb_byte_base;
-    uint8_t* const dst = tb + (size_t)cb * data_bytes;
-    const int head = min(data_bytes, (int)((0u - (uint32_t)(uintptr_t)dst) & 3u));
-    const int nfull = (data_bytes - head) >> 2;
-    for (int i = lane; i < nfull; i += 64) {
-        const uint32_t lo = bytes4(i), hi = (head != 0) ? bytes4(i + 1) : 0u;  // (byte 4 i + 3 + head < data_bytes)
-        *reinterpret_cast<uint32_t*>(dst + head + 4 * i) = __builtin_amdgcn_alignbyte(hi, lo, (uint32_t)head);
-    }
-    const int tail = head + 4 * nfull;
-    const int b = lane < head ? lane : tail + lane - head;
-    if (b < data_bytes && lane < head + (data_bytes - tail)) dst[b] = (uint8_t)(bytes4(b >> 2) >> (8 * (b & 3)));
+    put_bytes(tb + (size_t)cb * data_bytes, data_bytes, bytes4, lane, 64);
     if (lane == 0) {
         d.cb_crc_out[l.cb_count_base + cb] = crc;
         if (cb_in_tb == 0) {

@@ -39,8 +39,6 @@ struct dl_source {
     int words, L, Kd, F;
 };
 
-__device__ __forceinline__ uint32_t low_bits(int n) { return n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u; }
-
 // 32 selected bits from circle position c (< L) on, of which the first
 // `want` (1 .. 32) are used.
 __device__ __forceinline__ uint32_t circle_bits(const dl_source& s, int c, int want)

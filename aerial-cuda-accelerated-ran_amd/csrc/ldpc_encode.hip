@@ -122,7 +122,6 @@ __device__ __forceinline__ int wrap_any(int p, int Z)
     while (p >= Z) p -= Z;
     return p;
 }
-__device__ __forceinline__ uint32_t low_bits(int n) { return n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u; }
 
 // Encode one code block in LDS: l.raw holds its nsys * Z systematic bits on
 // entry (bits past them zero), l.x the columns on return, column c's Z bits

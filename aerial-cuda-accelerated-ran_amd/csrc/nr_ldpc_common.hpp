@@ -12,6 +12,9 @@
 
 namespace nrldpc {
 
+// The n lowest bits (n from 0 on).
+__device__ __forceinline__ uint32_t low_bits(int n) { return n >= 32 ? 0xFFFFFFFFu : (1u << n) - 1u; }
+
 // Compile-time view of a TS 38.212 base graph (tables in nr_bg_tables.h).
 template <int BG> struct bg_traits;
 // Rows are processed in order; a workgroup barrier is needed before row r

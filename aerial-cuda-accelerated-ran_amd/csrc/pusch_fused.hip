@@ -56,9 +56,6 @@ constexpr uint32_t FUSED_CB_ERROR = 0xFFFFFFFFu;  // CRC value of a CB/TB whose 
 constexpr uint32_t TB_ACC_ERROR = 0x80000000u;    // accumulator flag: a CB of the TB was rejected
 constexpr int SLOT_CB_WORDS = MAX_DECODED_CODE_BLOCK_BIT_SIZE / 32;  // 264: decoded-word stride per CB
 
-static __device__ const crc_stride_table<64> g_wave_stride[3] = {
-    make_crc_stride_table<64>(CRC24A_P), make_crc_stride_table<64>(CRC24B_P), make_crc_stride_table<64>(CRC16_P)};
-
 template <typename TI> __device__ __forceinline__ float llr_as_float(TI v) { return (float)v; }
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -149,25 +146,8 @@ __device__ __forceinline__ uint32_t tb_share_of(const fused_lds& sh, const uint3
         t.lane, t.tb);
     const int n = share_shift(t.C, t.data_bytes, cb_in_tb);
     const uint32_t f = n < 0 ? (n == -1 ? crc24a_unshift(1) : n == -2 ? crc24a_unshift(2) : crc24a_unshift(3))
-                             : wave_mulmod24(t.lane, g_crc_shift.lo[K_CRC24A][n & 1023],
-                                             g_crc_shift.tb_hi[(n >> 10) & 255], t.tb.fold);
+                             : wave_mulmod24(t.lane, g_crc_shift.lo[n & 1023], g_crc_shift.hi[(n >> 10) & 255], t.tb.fold);
     return wave_mulmod24(t.lane, part, f, t.tb.fold);
-}
-
-// The CB's payload bytes, by thread t of n: whole aligned words of the
-// destination, each from two decoded words, single bytes only at both ends.
-__device__ __forceinline__ void put_tb_bytes(const cuphyHipPuschSlotTb_t& job, int r, const uint32_t* words,
-                                             const cb_tail& tl, int t, int n)
-{
-    uint8_t* const dst = job.tb_bytes + (size_t)r * tl.data_bytes;
-    const int head = min(tl.data_bytes, (int)((0u - (uint32_t)(uintptr_t)dst) & 3u));
-    const int nfull = (tl.data_bytes - head) >> 2, tail = head + 4 * nfull;
-    for (int i = t; i < nfull; i += n) {
-        const uint32_t lo = rbit8x4(words[i]), hi = head ? rbit8x4(words[i + 1]) : 0u;
-        *reinterpret_cast<uint32_t*>(dst + head + 4 * i) = __builtin_amdgcn_alignbyte(hi, lo, (uint32_t)head);
-    }
-    const int b = t < head ? t : tail + t - head;
-    if (t < head + tl.data_bytes - tail) dst[b] = (uint8_t)(rbit8x4(words[b >> 2]) >> (8 * (b & 3)));
 }
 
 // Combine this transmission's E LLRs of the CB into the LDS circular buffer
@@ -547,7 +527,8 @@ __device__ __forceinline__ uint32_t fused_group(_Float16* __restrict__ hb, fused
             }
         } else {
             const int skip = one ? 64 * (2 - first_task) : tt & ~63;
-            put_tb_bytes(job, r0 + c, words, tail, tt - skip, one ? nthr - skip : 64);
+            put_bytes(job.tb_bytes + (size_t)(r0 + c) * tail.data_bytes, tail.data_bytes,
+                      [&](int w) { return rbit8x4(words[w]); }, tt - skip, one ? nthr - skip : 64);
         }
         if (one) break;
     }
