@@ -28,7 +28,7 @@ class UploadBlock:
         for s in sizes:
             self._off.append(n)
             n += (s + _ALIGN - 1) // _ALIGN * _ALIGN
-        self._host = torch.empty(max(n, 1), dtype=torch.uint8, pin_memory=not self.captured)
+        self._host = torch.empty(max(n, 1), dtype=torch.uint8, device="cpu", pin_memory=not self.captured)
         self._dev = torch.empty(max(n, 1), dtype=torch.uint8, device="cuda")
         self._hptr, self._dptr = self._host.data_ptr(), self._dev.data_ptr()
 

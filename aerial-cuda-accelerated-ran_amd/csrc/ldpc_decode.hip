@@ -521,10 +521,12 @@ cuphyStatus_t decode_batch(cuphyHipLDPCWorkItem_t* d_items, const uint32_t* d_gr
                                                                 : select_persistent_lm_kernel<46>(llr_type, f16))
                  : max_mb <= SMALL_MAXR ? select_persistent_kernel<SMALL_MAXR>(llr_type, f16)
                                         : select_persistent_kernel<46>(llr_type, f16);
-    // 5 or 6 waves of which two workgroups share a CU: balanced over its SIMDs
-    // (the 46-row kernels' registers leave one workgroup per CU).  2,800 BG1
-    // Zc = 384 blocks of 4 rows: 322 -> 311 us; with the two spare waves kept for
-    // the barriers 327 us
+    // 5 or 6 waves, several workgroups per CU: in workgroups of 8 waves, two per CU,
+    // balanced over its SIMDs (the 46-row kernels' registers leave one workgroup
+    // per CU).  2,800 BG1 blocks of 4 rows: 6 waves, Zc = 384 322 -> 312 us, with
+    // the two spare waves kept for the barriers 327 us; 5 waves, of which three
+    // workgroups had shared a CU, Zc = 320 301 -> 298, Zc = 288 306 -> 302 us, with 8
+    // rows 400 -> 397 and 399 -> 399 us, binary32 464 -> 452 and 463 -> 449 us
     const bool balance = lm && !pair && block_threads > 256 && max_mb <= SMALL_MAXR;
     const unsigned block = balance ? 64u * BALANCED_WAVES : (unsigned)block_threads;
     int rows_threads = block_threads;  // (of them, those that hold rows)

@@ -25,7 +25,7 @@
 // and an XOR per edge and 32 check rows.  The edges' bit offsets (column *
 // words + shift) are built in LDS once per code block.  The work is
 // 316 * 12 edge words per BG1 Zc = 384 code block, so the launch is bound by
-// its short dependent steps (seven barriers per code block), not by
+// its short dependent steps (eight barriers per code block), not by
 // arithmetic or HBM.  2,800 such code blocks: 345 -> 18.6 us against one byte
 // per bit and one check row per lane and step (12 MB in and out: 2.3 us).
 #include "nr_ldpc_common.hpp"

@@ -576,12 +576,15 @@ __device__ __forceinline__ void complete_cb(const cuphyHipPuschSlotTb_t& job, ui
 }
 
 // Threads of a workgroup.  With all rows, whose registers leave one workgroup
-// per CU, two lane groups of FUSED_BLOCK (run_iterations PAIR = 2; 168 VGPRs, no
-// spills): every phase has twice the waves and the rows of a barrier segment run
-// side by side.  One group against two: 64 descrambled UEs with a retransmission
-// 429 -> 411 us, a served burst of 384 TBs 1083 -> 1041 us.  Where two workgroups
-// share a CU, 8 waves, of which lanes past FUSED_BLOCK hold no rows in the decode:
-// 64-cell int8 slot 572 -> 546 us (6 waves -> 8, balanced_wave_place).
+// per CU, two lane groups of FUSED_BLOCK (run_iterations PAIR = 2; 168 VGPRs and 3
+// to 7 spilled, stored and loaded between the phases and once or twice per
+// iteration, not in the rows): every phase has twice the waves and the rows of a
+// barrier segment run side by side.  One group against two: 64 descrambled UEs with
+// a retransmission 429 -> 411 us, a served burst of 384 TBs 1083 -> 1041 us.  Where
+// two workgroups share a CU, 8 waves, of which lanes past FUSED_BLOCK hold no rows
+// in the decode: 64-cell int8 slot 572 -> 546 us (6 waves -> 8, balanced_wave_place);
+// 800 TBs of Zc = 20, one wave of rows each, pay for the wider barriers: 53.7 -> 54.4
+// us with early termination, 95 -> 98 us without.
 constexpr int fused_threads(int maxr) { return maxr <= MID_MAXR ? 64 * (int)BALANCED_WAVES : 2 * FUSED_BLOCK; }
 
 // Persistent fused slot kernel.  Workspace: queue state (2 words used of
@@ -592,8 +595,8 @@ constexpr int fused_threads(int maxr) { return maxr <= MID_MAXR ? 64 * (int)BALA
 // The high-rate variant (MAXR <= 8) and the middle one (MAXR <= 16) are
 // held to 4 waves per SIMD (at most 128 VGPRs): two workgroups of 8 waves fill
 // them.  At its natural 157 VGPRs (3 slots) the high-rate variant ran one
-// workgroup per CU.  (The middle variant's BG1 rows beyond 8 spill a few
-// registers; BG2 rows, half as long, do not.)
+// workgroup per CU.  (The middle variant's BG1 rows beyond 8 spill, 33 to 50
+// registers in all; the grouped high-rate variant spills 9.)
 template <typename TI, int MAXR, bool GROUPED>
 __global__ __launch_bounds__(fused_threads(MAXR)) __attribute__((amdgpu_waves_per_eu(MAXR <= MID_MAXR ? 4 : 1)))
 void pusch_slot_fused(const cuphyHipPuschSlotTb_t* __restrict__ tbs, int n_tbs,

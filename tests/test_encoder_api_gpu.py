@@ -282,3 +282,20 @@ def test_encode_words_results_are_aligned(enc):
     print("[case] encode_words result alignment", flush=True)
     outs = enc.encode_words(2, 5, [torch.zeros((1, 2), dtype=torch.int32, device="cuda")] * 5)
     assert all(o.data_ptr() % 512 == 0 and o.is_contiguous() and o.storage_offset() % 4 == 0 for o in outs)
+
+
+def test_calls_with_a_cuda_default_device(enc):
+    """The uploads' host blocks are host memory whatever torch's default device."""
+    from aerial_amd.encoder import dl_rate_match
+    from aerial_amd.pusch import make_tb_params
+    print("[case] encoder and DL rate matching, default device cuda", flush=True)
+    p, _ = make_tb_params(2, 52, 2, 520, 2, 1, 2 * 600, 0)
+    info = np.random.RandomState(6).randint(0, 2, (2, 520)).astype(np.uint8)
+    words = torch.from_numpy(np.stack([O.pack_bits(x) for x in info]).view(np.int32)).cuda()
+    enc.puncturing = True
+    with torch.device("cuda"):
+        out = dl_rate_match([p], enc.encode_words(2, 52, [words]), 640)
+    torch.cuda.synchronize()
+    cw = [O.encode(2, 52, x)[104:104 + p.N] for x in info]
+    for r, ref in enumerate(dl_reference(p, cw, 0, False)):
+        assert np.array_equal(words_to_bits(out.cpu().numpy()[0, r], 640)[:ref.size], ref), r
