@@ -144,9 +144,9 @@ def dl_rate_match(params, coded_words, emax, scrambling=False, stream=None):
     else:
         out = torch.full(shape, -1, dtype=torch.int32, device="cuda")
     with on_stream(stream):
-        blk = UploadBlock((n * C.sizeof(L.PerTbParams), 8 * n))
+        blk = UploadBlock((n * C.sizeof(L.PerTbParams), 8 * len(coded_words)))
         put_params(blk.host(0), params)
-        ptrs = (C.c_uint64 * n).from_address(blk.host(1))
+        ptrs = (C.c_uint64 * len(coded_words)).from_address(blk.host(1))
         for i, w in enumerate(coded_words):
             ptrs[i] = w.data_ptr()
         blk.send()
